@@ -253,12 +253,17 @@ struct DevBuf {
   T* as() const {
     return static_cast<T*>(p);
   }
-  Status alloc_zero(size_t n, hipStream_t s, const char* what) {
+  // Contents undefined: for arrays the next launch writes whole.
+  Status alloc(size_t n, const char* what) {
     release();
     if (n == 0) return Status{};
     HIP_TRY(hipMalloc(&p, n), what);
     bytes = n;
-    HIP_TRY(hipMemsetAsync(p, 0, n, s), what);
+    return Status{};
+  }
+  Status alloc_zero(size_t n, hipStream_t s, const char* what) {
+    KIVI_TRY(alloc(n, what));
+    if (n != 0) HIP_TRY(hipMemsetAsync(p, 0, n, s), what);
     return Status{};
   }
 };
@@ -1217,8 +1222,9 @@ Status quantize(const float* data, size_t data_len, size_t batch, size_t heads, 
   q->n_params = per_channel ? units * (tokens / group_size) * head_dim * 2
                             : units * tokens * (head_dim / group_size) * 2;
   hipStream_t s = device ? stream : nullptr;
-  KIVI_TRY(q->codes.alloc_zero(q->n_codes * 4, s, "quantized codes"));
-  KIVI_TRY(q->params.alloc_zero(q->n_params * 4, s, "quantized params"));
+  // the quantize launch writes every word and every (scale, zero) pair
+  KIVI_TRY(q->codes.alloc(q->n_codes * 4, "quantized codes"));
+  KIVI_TRY(q->params.alloc(q->n_params * 4, "quantized params"));
   const float* src = data;
   Scratch staging;
   if (!device) {

@@ -1153,6 +1153,36 @@ __global__ void __launch_bounds__(kThreads)
   }
 }
 
+// VW consecutive words (VW = 1, 2 or 4) at p, 4*VW-byte aligned, in one load.
+template <int VW>
+__device__ __forceinline__ void load_run(const uint32_t* p, uint32_t (&w)[VW]) {
+  if constexpr (VW == 4) {
+    const uint4 v = *reinterpret_cast<const uint4*>(p);
+    w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
+  } else if constexpr (VW == 2) {
+    const uint2 v = *reinterpret_cast<const uint2*>(p);
+    w[0] = v.x; w[1] = v.y;
+  } else {
+    w[0] = *p;
+  }
+}
+
+// Item `it` of a (q, b, a) index space with a < na fastest, then b < nb: one 32-bit division each
+// below 2^32 items (a 64-bit one costs several times as many instructions).
+__device__ __forceinline__ void split_item(uint64_t it, uint32_t na, uint32_t nb, uint64_t& q, uint32_t& b, uint32_t& a) {
+  if (it >> 32) {
+    a = static_cast<uint32_t>(it % na);
+    it /= na;
+    b = static_cast<uint32_t>(it % nb);
+    q = it / nb;
+  } else {
+    const uint32_t i = static_cast<uint32_t>(it), r = i / na;
+    a = i % na;
+    b = r % nb;
+    q = r / nb;
+  }
+}
+
 // The general forms (any head_dim and group): one workgroup per (unit, group) for keys, one
 // thread per (row, channel group) for values.
 
@@ -1219,7 +1249,8 @@ __global__ void __launch_bounds__(kThreads)
   }
 }
 
-// QuantizedTensor::dequantize (src/quant.rs:124-150 via dequant_keys/values :379-451).
+// QuantizedTensor::dequantize (src/quant.rs:124-150 via dequant_keys/values :379-451), any
+// head_dim, group and output alignment: one element per thread.
 __global__ void __launch_bounds__(kThreads)
     k_dequant_ref(const uint32_t* codes, const float* params, uint32_t units, uint64_t tokens,
                   uint32_t D, uint32_t bits, uint32_t G, int per_channel, float* out) {
@@ -1250,23 +1281,104 @@ __global__ void __launch_bounds__(kThreads)
   }
 }
 
-// QuantizedTensor::pytorch_codes for keys (src/quant.rs:81-94): out[tp][d] = word (g, d, w)
-// with tp = g*ipc + w. Values are already in that order (src/quant.rs:95-109).
+// The same for per-channel streams with head_dim % 4 == 0 and a 16-byte aligned output. Bound by
+// the HBM writes (4 bytes out per element against bits/8 in). A thread takes four channels of VW
+// words each (one vector load per channel), so that every store is a whole float4 and a wave's
+// store covers consecutive channels of a row; the four (scale, zero) pairs are loaded once for
+// VW * ppw tokens. One element per thread spent its time on 64-bit divisions and on a word and a
+// pair load per element: 32 units x 8192 x 128 at 4 bits 128 -> 25 us (5.4 TB/s written).
+template <int BITS, int VW>
 __global__ void __launch_bounds__(kThreads)
-    k_pytorch_keys(const uint32_t* codes, uint32_t units, uint64_t tokens, uint32_t D, uint32_t bits,
-                   uint32_t G, uint32_t* out) {
-  const uint32_t ppw = 32 / bits, ipc = G / ppw;
-  const uint64_t t_pack = tokens / ppw;
-  const uint64_t total = (uint64_t)units * t_pack * D;
-  for (uint64_t idx = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; idx < total;
-       idx += (uint64_t)gridDim.x * blockDim.x) {
-    const uint64_t ut = idx / D;
-    const uint32_t d = idx % D;
-    const uint32_t unit = ut / t_pack;
-    const uint64_t tp = ut % t_pack;
-    const uint64_t g = tp / ipc;
-    const uint32_t w = tp % ipc;
-    out[idx] = codes[unit * (t_pack * D) + (g * D + d) * ipc + w];
+    k_dequant_ref_keys(const uint32_t* codes, const float* params, uint64_t items, uint32_t D, uint32_t ipc,
+                       float* out) {
+  constexpr uint32_t PPW = 32 / BITS, MASK = (1u << BITS) - 1u;
+  const uint32_t q4 = D / 4, runs = ipc / VW;  // float4s per row, word runs per channel
+  for (uint64_t it = blockIdx.x * (uint64_t)kThreads + threadIdx.x; it < items; it += (uint64_t)gridDim.x * kThreads) {
+    // item = (group q over all units, word run w0, four channels d0); d0 fastest
+    uint64_t q;
+    uint32_t w0, d0;
+    split_item(it, q4, runs, q, w0, d0);
+    d0 *= 4;
+    w0 *= VW;
+    uint32_t w[4][VW];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) load_run<VW>(codes + (q * D + d0 + e) * ipc + w0, w[e]);
+    const float4* pp = reinterpret_cast<const float4*>(params) + (q * D + d0) / 2;
+    const float4 p01 = pp[0], p23 = pp[1];
+    float* row = out + (q * ipc + w0) * PPW * D + d0;
+#pragma unroll
+    for (int k = 0; k < VW; ++k)
+#pragma unroll
+      for (uint32_t i = 0; i < PPW; ++i) {
+        f4v x;
+        x.x = fmaf(static_cast<float>((w[0][k] >> (BITS * i)) & MASK), p01.x, p01.y);
+        x.y = fmaf(static_cast<float>((w[1][k] >> (BITS * i)) & MASK), p01.z, p01.w);
+        x.z = fmaf(static_cast<float>((w[2][k] >> (BITS * i)) & MASK), p23.x, p23.y);
+        x.w = fmaf(static_cast<float>((w[3][k] >> (BITS * i)) & MASK), p23.z, p23.w);
+        *reinterpret_cast<f4v*>(row + (k * PPW + i) * (uint64_t)D) = x;
+      }
+  }
+}
+
+// The same for per-token streams (16-byte aligned output): codes, pairs and elements run in one
+// order, so element e lies in word e / ppw and group e / G. A workgroup takes kRefSpan consecutive
+// elements, each thread float4s kThreads apart (whole-line stores; the lanes of a word and of a
+// group read the same line). Bound by the HBM writes; 32 units x 8192 x 128 at 4 bits
+// 102 -> 25 us against one element per thread.
+constexpr uint32_t kRefSpan = 8192;
+template <int BITS>
+__global__ void __launch_bounds__(kThreads)
+    k_dequant_ref_values(const uint32_t* codes, const float* params, uint64_t elems, uint32_t G, float* out) {
+  constexpr uint32_t PPW = 32 / BITS, MASK = (1u << BITS) - 1u;
+  for (uint64_t base = blockIdx.x * (uint64_t)kRefSpan; base < elems; base += (uint64_t)gridDim.x * kRefSpan) {
+    const uint32_t n = static_cast<uint32_t>(std::min<uint64_t>(kRefSpan, elems - base));
+    const uint64_t g0 = base / G;
+    const uint32_t r0 = static_cast<uint32_t>(base % G);
+    const uint32_t* wp = codes + base / PPW;  // kRefSpan is a multiple of every ppw
+    const float2* pp = reinterpret_cast<const float2*>(params) + g0;
+#pragma unroll
+    for (uint32_t j = 0; j < kRefSpan / (4 * kThreads); ++j) {
+      const uint32_t e = (j * kThreads + threadIdx.x) * 4;
+      if (e < n) {  // n is a multiple of G, which is one of 4
+        const uint32_t w = wp[e / PPW] >> (BITS * (e % PPW));
+        const float2 sz = pp[(r0 + e) / G];
+        f4v x;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = fmaf(static_cast<float>((w >> (BITS * i)) & MASK), sz.x, sz.y);
+        *reinterpret_cast<f4v*>(out + base + e) = x;
+      }
+    }
+  }
+}
+
+// QuantizedTensor::pytorch_codes for keys (src/quant.rs:81-94): out[tp][d] = word (g, d, w)
+// with tp = g*ipc + w, a transpose of each group's D x ipc words (units are contiguous on both
+// sides, so the groups of all units run in one index). Values are already in that order
+// (src/quant.rs:95-109). A thread takes CH channels of VW words each: VW-word loads and, with
+// four channels, 16-byte stores of consecutive channels (head_dim % 4 == 0 and an aligned output;
+// CH = 1 otherwise). HBM-bound; 32 units x 8192 x 128 at 4 bits 17.9 -> 6.8 us against one word
+// per thread with its divisions.
+template <int VW, int CH>
+__global__ void __launch_bounds__(kThreads)
+    k_pytorch_keys(const uint32_t* codes, uint64_t items, uint32_t D, uint32_t ipc, uint32_t* out) {
+  const uint32_t runs = ipc / VW;
+  for (uint64_t it = blockIdx.x * (uint64_t)kThreads + threadIdx.x; it < items; it += (uint64_t)gridDim.x * kThreads) {
+    uint64_t q;
+    uint32_t w0, d0;
+    split_item(it, D / CH, runs, q, w0, d0);
+    d0 *= CH;
+    w0 *= VW;
+    uint32_t w[CH][VW];
+#pragma unroll
+    for (int e = 0; e < CH; ++e) load_run<VW>(codes + (q * D + d0 + e) * ipc + w0, w[e]);
+    uint32_t* row = out + (q * ipc + w0) * D + d0;
+#pragma unroll
+    for (int k = 0; k < VW; ++k) {
+      if constexpr (CH == 4)
+        *reinterpret_cast<uint4*>(row + (uint64_t)k * D) = make_uint4(w[0][k], w[1][k], w[2][k], w[3][k]);
+      else
+        row[(uint64_t)k * D] = w[0][k];
+    }
   }
 }
 
@@ -1621,11 +1733,43 @@ hipError_t launch_quant_ref_values(const float* data, uint32_t units, uint64_t t
   return hipGetLastError();
 }
 
+// Words per load of a channel's ipc consecutive words: 4, 2 or 1, whichever divides ipc.
+uint32_t run_words(uint32_t ipc) { return ipc % 4 == 0 ? 4 : ipc % 2 == 0 ? 2 : 1; }
+
 hipError_t launch_dequant_ref(const uint32_t* codes, const float* params, uint32_t units,
                               uint64_t tokens, uint32_t D, uint32_t bits, uint32_t G,
                               int per_channel, float* out, hipStream_t stream) {
   const uint64_t work = (uint64_t)units * tokens * D;
   if (work == 0) return hipSuccess;
+  const bool aligned = reinterpret_cast<uintptr_t>(out) % 16 == 0;
+  // float4 outputs: whole rows of them for keys; for values G (a multiple of 4 at every width)
+  // keeps a float4 inside one group and one word
+  if (aligned && per_channel && D % 4 == 0) {
+    const uint32_t ipc = G * bits / 32, vw = run_words(ipc);
+    const uint64_t items = (uint64_t)units * (tokens / G) * (ipc / vw) * (D / 4);
+#define KIVI_DK(B, W)                                                                                        \
+  case B * 10 + W:                                                                                           \
+    k_dequant_ref_keys<B, W><<<grid_for(items), kThreads, 0, stream>>>(codes, params, items, D, ipc, out);   \
+    break;
+    switch (bits * 10 + vw) {
+      KIVI_DK(2, 1) KIVI_DK(2, 2) KIVI_DK(2, 4)
+      KIVI_DK(4, 1) KIVI_DK(4, 2) KIVI_DK(4, 4)
+      KIVI_DK(8, 1) KIVI_DK(8, 2) KIVI_DK(8, 4)
+      default: return hipErrorInvalidValue;
+    }
+#undef KIVI_DK
+    return hipGetLastError();
+  }
+  if (aligned && !per_channel) {
+    const unsigned grid = grid_for(work, kRefSpan);
+    switch (bits) {
+      case 2: k_dequant_ref_values<2><<<grid, kThreads, 0, stream>>>(codes, params, work, G, out); break;
+      case 4: k_dequant_ref_values<4><<<grid, kThreads, 0, stream>>>(codes, params, work, G, out); break;
+      case 8: k_dequant_ref_values<8><<<grid, kThreads, 0, stream>>>(codes, params, work, G, out); break;
+      default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+  }
   k_dequant_ref<<<grid_for(work), kThreads, 0, stream>>>(codes, params, units, tokens, D, bits, G,
                                                         per_channel, out);
   return hipGetLastError();
@@ -1638,7 +1782,19 @@ hipError_t launch_pytorch_order(const uint32_t* codes, uint32_t units, uint64_t 
   if (words == 0) return hipSuccess;
   if (!per_channel)
     return hipMemcpyAsync(out, codes, words * 4, hipMemcpyDeviceToDevice, stream);
-  k_pytorch_keys<<<grid_for(words), kThreads, 0, stream>>>(codes, units, tokens, D, bits, G, out);
+  const uint32_t ipc = G * bits / 32, vw = run_words(ipc);
+  const uint32_t ch = D % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 ? 4 : 1;
+  const uint64_t items = (uint64_t)units * (tokens / G) * (ipc / vw) * (D / ch);
+  const unsigned grid = grid_for(items);
+  switch (vw * 10 + ch) {
+    case 11: k_pytorch_keys<1, 1><<<grid, kThreads, 0, stream>>>(codes, items, D, ipc, out); break;
+    case 21: k_pytorch_keys<2, 1><<<grid, kThreads, 0, stream>>>(codes, items, D, ipc, out); break;
+    case 41: k_pytorch_keys<4, 1><<<grid, kThreads, 0, stream>>>(codes, items, D, ipc, out); break;
+    case 14: k_pytorch_keys<1, 4><<<grid, kThreads, 0, stream>>>(codes, items, D, ipc, out); break;
+    case 24: k_pytorch_keys<2, 4><<<grid, kThreads, 0, stream>>>(codes, items, D, ipc, out); break;
+    case 44: k_pytorch_keys<4, 4><<<grid, kThreads, 0, stream>>>(codes, items, D, ipc, out); break;
+    default: return hipErrorInvalidValue;
+  }
   return hipGetLastError();
 }
 

@@ -125,6 +125,39 @@ def test_quantized_device_exports_match_oracle(amd, oracle, case):
         dev.free()
 
 
+# The vector forms of the two reads: 1, 2 and 4 words per load (ipc = G*bits/32 odd, even, a
+# multiple of 4), rows that end inside a wave, spans of 8192 elements with a remainder, head_dims
+# that are no multiple of 4 and outputs 4 bytes off a 16-byte boundary (one element per thread).
+VECTOR_READS = [
+    (bits, group, tokens, dim)
+    for bits, group in ((2, 16), (2, 32), (2, 48), (4, 8), (4, 16), (4, 32), (8, 4), (8, 8), (8, 48))
+    for tokens, dim in ((group, group), (3 * group, 2 * group), (17 * group, 5 * group))
+] + [(8, 4, 12, 7), (2, 32, 64, 30), (4, 32, 96, 1)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("off", [0, 4])
+@pytest.mark.parametrize("case", VECTOR_READS)
+def test_vector_reads_match_oracle(amd, oracle, case, off):
+    bits, group, tokens, dim = case
+    data = fill(2 * tokens * dim, 91) * np.float32(2.5)
+    for q in (quantize_per_channel, quantize_per_token):
+        if q is quantize_per_token and dim % group:
+            continue
+        qa, qo = (q(b, data, 2, 1, tokens, dim, bits, group) for b in (amd, oracle))
+        dev = DeviceArrays()
+        try:
+            nc, n = qa.code_bytes() // 4, data.size
+            pc, dq = dev.empty(nc + 1), dev.empty(n + 1)
+            qa.pytorch_codes_device(pc + off, nc)
+            qa.dequantize_device(dq + off, n)
+            codes, dense = dev.download(pc, nc + 1)[off // 4:], dev.download(dq, n + 1)[off // 4:]
+            assert np.array_equal(codes[:nc].view(np.uint32), qo.pytorch_codes())
+            assert np.array_equal(dense[:n].view(np.uint32), qo.dequantize().view(np.uint32))
+        finally:
+            dev.free()
+
+
 # ------------------------------------------------------------------ HBM planning
 
 
