@@ -286,6 +286,9 @@ bool attention_fuses_decode(const AttnProblem& p);
 
 // Workspace floats the attention needs for `p` (split-K partials).
 size_t attention_workspace_floats(const AttnProblem& p);
+// Partials by which the allocation-free attention accepts a call (at most kStaticWorkspaceFloats);
+// attention_workspace_floats fits the static workspace whenever this does.
+size_t attention_counted_floats(const AttnProblem& p);
 hipError_t launch_attention(const AttnProblem& p, float* workspace, hipStream_t stream);
 
 // Static attention workspace (kernels_attn.hip): a file-scope device array of

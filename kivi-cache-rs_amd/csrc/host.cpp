@@ -879,7 +879,7 @@ Status cache_attention_noalloc(const kivi_cache* c, const float* query, size_t q
     HIP_TRY(launch_fill_zero(out, out_len, stream), "attention zero output");
     return Status{};
   }
-  const size_t floats = attention_workspace_floats(p);
+  const size_t floats = attention_counted_floats(p);
   if (floats > kStaticWorkspaceFloats)
     return Err(KIVI_ERR_CAPACITY, floats, kStaticWorkspaceFloats, "attention workspace floats");
   StaticWorkspaceSlot* slot = nullptr;

@@ -22,14 +22,17 @@
 //    a token (keys) or D/64 channels (values), and the native layout packs exactly that
 //    lane's codes into its words, so a word unpacks into 4-16 MFMA B operands. At head_dim
 //    128 the same launch takes the window / suffix chunks (fp32 rows, a quarter chunk per
-//    wave); at other head_dims the tokens after the packed chunks run as generic splits in
+//    wave); at other head_dims the tokens after the packed chunks run as row splits in
 //    its grid.
 //  * k_attn_shared / k_attn_sessions / k_attn_suffix — batched sessions over one shared
 //    prefix (the prefix read once for all sessions).
-//  * k_attn_generic — every shape the MFMA kernel does not cover, caches with no packed keys
-//    yet and the quality guard's fp32 attention: one wavefront per token in the reference's
-//    operation order (recon = fma(code, scale, zero); logit = fma(recon, q, logit), channels
-//    ascending, src/attention.rs:143-177, 289-300).
+//  * k_attn_lanes — packed chunks of the other head_dims and groups that are multiples of 16, in
+//    f32 on the vector ALU, with row splits for the tokens after them.
+//  * k_attn_rows — row splits alone: caches without a packed chunk, the quality guard's fp32
+//    attention, other groups (head_dim a multiple of 16).
+//  * k_attn_generic — any other head_dim: one wavefront per token in the reference's operation
+//    order (recon = fma(code, scale, zero); logit = fma(recon, q, logit), channels ascending,
+//    src/attention.rs:143-177, 289-300).
 #include "common.hpp"
 #include "kivi.h"
 
@@ -63,13 +66,13 @@ struct AttnArgs {
   const float* query;      // [batch][QH][D]
   uint32_t qh, heads, gq;
   float scale2;            // scale * log2(e)
-  // generic splits: tokens [t_begin, total) in splits of S
+  // row (or generic) splits: tokens [t_begin, total) in splits of S
   uint64_t t_begin;
   uint32_t S;
   uint32_t nsplit_gen;
   // MFMA splits: packed chunks [chunk_begin, chunk_end) in workgroups of 4 waves x kFastCpw
   // chunks (workspace splits 0 .. nsplit_fast-1), then window / suffix chunks
-  // [win_begin, win_end), one per workgroup (splits nsplit_fast .. +nsplit_win-1); generic
+  // [win_begin, win_end), one per workgroup (splits nsplit_fast .. +nsplit_win-1); row
   // splits, if any, follow.
   uint32_t chunk_begin;
   uint32_t chunk_end;
@@ -81,10 +84,16 @@ struct AttnArgs {
   // (unit, head group, split), each writing its group's partial rows. hgroups_fast: the head
   // groups of the packed splits (groups of 16 on the sixteen-head kernel, hgroups otherwise)
   uint32_t hgroups, hgroups_fast;
+  // head groups (of up to kRowHeads) of the row splits, which take the splits nsplit_gen counts;
+  // 0: generic splits, every head in one workgroup
+  uint32_t hgroups_rows;
   uint32_t gshift;         // log2(G) on the matrix-core path (G = 32, 64 or 128 there)
   // packed splits on the 16x16x32 kernels: 1 eight-head (k_attn_wide), 2 sixteen-head
   // (k_attn_wide16)
   uint32_t wide;
+  // lane splits (k_attn_lanes): chunks per split (0 on every other path) and log2 of the value
+  // phase's chunk slots
+  uint32_t lane_cps, lane_log;
   float* ws;               // [units][nsplit_total][gq][D+2]
   // batched sessions (0 otherwise): session count and the strides between consecutive
   // sessions' queries, partials and outputs
@@ -107,15 +116,13 @@ struct AttnArgs {
   uint32_t pend_evict;
 };
 
-// Key / value element (token t, channel d) of one unit, wherever it lives. BITS, DD, GG are
-// the compile-time shape (0 = read it from the geometry at run time). Branch free: the packed
+// Key / value element (token t, channel d) of one unit, wherever it lives. Branch free: the packed
 // and the fp32 candidate are both loaded from clamped, always-valid addresses and blended, so
 // unrolled callers keep many loads in flight. Both candidates are finite (arenas are zero
 // filled), so the blend returns exactly the selected one.
-template <int BITS, int DD, int GG>
 __device__ __forceinline__ float key_at(const AttnArgs& a, uint32_t unit, uint64_t t, uint32_t d) {
   const Geometry& g = a.c.geo;
-  const uint32_t bits = BITS ? BITS : g.bits, D = DD ? DD : g.D, G = GG ? GG : g.G;
+  const uint32_t bits = g.bits, D = g.D, G = g.G;
   const uint32_t ppw = 32 / bits, kw = D / ppw;
   const uint64_t kq = a.st.kq;
   // packed candidate
@@ -139,10 +146,9 @@ __device__ __forceinline__ float key_at(const AttnArgs& a, uint32_t unit, uint64
   return fmaf(fmaf(code, sz.x, sz.y), m, dense * (1.f - m));  // exact for m in {0, 1}
 }
 
-template <int BITS, int DD, int GG>
 __device__ __forceinline__ float value_at(const AttnArgs& a, uint32_t unit, uint64_t t, uint32_t d) {
   const Geometry& g = a.c.geo;
-  const uint32_t bits = BITS ? BITS : g.bits, D = DD ? DD : g.D, G = GG ? GG : g.G;
+  const uint32_t bits = g.bits, D = g.D, G = g.G;
   const uint32_t ppw = 32 / bits, vw = kValueBlock / ppw;
   const uint64_t vq = a.st.vq;
   const uint64_t tp = vq > 0 ? (t < vq ? t : vq - 1) : 0;
@@ -198,13 +204,11 @@ __device__ __forceinline__ float warp_sum(float v) {
 
 // ------------------------------------------------------------------ generic splits
 // One workgroup per (unit, split) over tokens [t_begin, total). LDS: q [gq][D], logits/weights
-// [gq][S]. Instantiated for every shape (BITS = DD = GG = 0) and, with the shape fixed, for the
-// tail of the MFMA path (the fp32 window, the session suffix and a partial last chunk).
-template <int BITS, int DD, int GG>
+// [gq][S]. For head_dims that are no multiple of 16; any bits and group.
 __device__ __forceinline__ void generic_split(const AttnArgs& a, uint32_t unit, uint32_t split,
                                               float* lds) {
   const Geometry& g = a.c.geo;
-  const uint32_t D = DD ? DD : g.D, gq = a.gq, S = a.S;
+  const uint32_t D = g.D, gq = a.gq, S = a.S;
   const uint32_t b = unit / a.heads, kvh = unit % a.heads;
   float* q_lds = lds;               // [gq][D], pre-scaled to base-2 logits
   float* w_lds = lds + gq * D;      // [gq][S]
@@ -233,7 +237,7 @@ __device__ __forceinline__ void generic_split(const AttnArgs& a, uint32_t unit, 
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const uint32_t k = std::min<uint32_t>(k0 + j, ntok - 1);
-          kv[j] = key_at<BITS, DD, GG>(a, unit, t0 + k, d) * live_d;
+          kv[j] = key_at(a, unit, t0 + k, d) * live_d;
         }
 #pragma unroll
         for (int h = 0; h < kHeadsPerPass; ++h) {
@@ -282,7 +286,7 @@ __device__ __forceinline__ void generic_split(const AttnArgs& a, uint32_t unit, 
     for (uint32_t k0 = 0; k0 < ntok; k0 += 8) {
       float v[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = value_at<BITS, DD, GG>(a, unit, t0 + std::min<uint32_t>(k0 + j, ntok - 1), d);
+      for (int j = 0; j < 8; ++j) v[j] = value_at(a, unit, t0 + std::min<uint32_t>(k0 + j, ntok - 1), d);
 #pragma unroll
       for (int j = 0; j < 8; ++j)
 #pragma unroll
@@ -297,11 +301,10 @@ __device__ __forceinline__ void generic_split(const AttnArgs& a, uint32_t unit, 
   }
 }
 
-template <int BITS, int DD, int GG>
 __global__ void __launch_bounds__(kThreads) k_attn_generic(AttnArgs a) {
   extern __shared__ float lds[];
   const uint32_t unit = blockIdx.x / a.nsplit_gen;
-  generic_split<BITS, DD, GG>(a, unit, blockIdx.x % a.nsplit_gen, lds);
+  generic_split(a, unit, blockIdx.x % a.nsplit_gen, lds);
 }
 
 // ------------------------------------------------------------------ MFMA splits
@@ -1221,6 +1224,560 @@ __device__ __forceinline__ void mfma_split(const AttnArgs& a, uint32_t unit, uin
   }
 }
 
+// ------------------------------------------------------------------ vector-ALU helpers
+// x = fma(code, sc, zr) of 16 elements from BITS / 2 native words (element order, see code_shift).
+// A mask leaves four codes one per byte and v_cvt_f32_ubyte0-3 takes them out, one instruction
+// each. The empty asm keeps the mask whole: the compiler would turn it into a bit-field extract
+// per element. (The packed fp4 / fp8 converters with v_fma_mix_f32 are fewer instructions, but
+// v_fma_mix takes twice the issue cycles of v_fmac: 24.2 -> 25.5 us at 16 units x 8192 tokens x 128
+// channels, 4 bits, G = 16, four heads.)
+template <int BITS>
+__device__ __forceinline__ void lane_recon(const uint32_t (&w)[BITS / 2], const float (&sc)[16],
+                                           const float (&zr)[16], float (&x)[16]) {
+  auto bytes = [&](uint32_t m, int a, int b, int c, int d) {
+    asm("" : "+v"(m));
+    x[a] = fmaf(static_cast<float>(m & 0xffu), sc[a], zr[a]);
+    x[b] = fmaf(static_cast<float>((m >> 8) & 0xffu), sc[b], zr[b]);
+    x[c] = fmaf(static_cast<float>((m >> 16) & 0xffu), sc[c], zr[c]);
+    x[d] = fmaf(static_cast<float>(m >> 24), sc[d], zr[d]);
+  };
+  if constexpr (BITS == 8) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) bytes(w[k], 4 * k, 4 * k + 1, 4 * k + 2, 4 * k + 3);
+  } else if constexpr (BITS == 4) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)  // byte i of word k / 2 holds elements i and i + 4
+      bytes((w[k / 2] >> (4 * (k % 2))) & 0x0f0f0f0fu, 4 * k, 4 * k + 1, 4 * k + 2, 4 * k + 3);
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {  // byte i holds elements 2i, 2i + 8, 2i + 1, 2i + 9
+      const int e = (k >> 1) + 8 * (k & 1);
+      bytes((w[0] >> (2 * k)) & 0x03030303u, e, e + 2, e + 4, e + 6);
+    }
+  }
+}
+
+template <int N>
+__device__ __forceinline__ void lane_words(const uint32_t* p, uint32_t (&w)[N]) {
+  if constexpr (N == 4) {
+    const uint4 v = *reinterpret_cast<const uint4*>(p);
+    w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
+  } else if constexpr (N == 2) {
+    const uint2 v = *reinterpret_cast<const uint2*>(p);
+    w[0] = v.x; w[1] = v.y;
+  } else {
+    w[0] = *p;
+  }
+}
+
+// 16 consecutive (scale, zero) pairs.
+__device__ __forceinline__ void lane_params(const float2* p, float (&s)[16], float (&z)[16]) {
+  const float4* q = reinterpret_cast<const float4*>(p);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float4 v = q[i];
+    s[2 * i] = v.x;
+    z[2 * i] = v.y;
+    s[2 * i + 1] = v.z;
+    z[2 * i + 1] = v.w;
+  }
+}
+
+// Orders a wave's own LDS writes before its later reads of them by other lanes (the hardware keeps a
+// wave's LDS operations in order; this holds the compiler to it).
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// ------------------------------------------------------------------ row splits
+// Tokens [t_begin, total) of any head_dim that is a multiple of 16, wherever each of them lives
+// (packed, key residual, value window, suffix): the tokens after the packed chunks at head_dims
+// other than 128, whole caches without packed chunks, the quality guard's fp32 tape, and packed
+// tokens of groups the other kernels do not take. A workgroup takes S tokens for up to four heads.
+//
+// These launches are short and bound by their chain of memory round trips, so every lane requests
+// both the packed and the fp32 form of what it needs from clamped addresses at once and selects
+// afterwards, a key lane reads 16 channels of a token in at most 13 loads, and the first values are
+// requested before the dot products. Measured against one wavefront per token with a load and a blend
+// per channel (k_attn_generic): 100 tokens, 8 units, four heads at head_dim 128: 67 -> 9.9 us; the
+// tokens behind the packed chunks of 40 units at head_dim 64, 12345 tokens: 20.9 -> 18.4 us for
+// the whole launch.
+constexpr uint32_t kRowHeads = 4;      // query heads per workgroup
+constexpr uint32_t kRowMaxTokens = 256;
+constexpr uint32_t kRowGroups = 1024;  // workgroups the row splits keep to, four per CU
+constexpr uint32_t kRowAhead = 4;      // value rows a thread requests at once
+
+// Tokens whose keys one pass of a workgroup covers (head_dim / 16 lanes each).
+__host__ __device__ inline uint32_t row_pass(uint32_t D) { return 4 * (64 / (D / 16)); }
+__host__ __device__ inline uint32_t row_lds_floats(uint32_t D, uint32_t S) {
+  return kRowHeads * (D + S) + 4 * kThreads * kRowHeads;
+}
+
+template <int BITS>
+__device__ __forceinline__ void row_split(const AttnArgs& a, uint32_t unit, uint32_t split, uint32_t hg,
+                                          float* lds) {
+  constexpr uint32_t NW = BITS / 2, PPW = 32 / BITS, VW = kValueBlock / PPW, MASK = (1u << BITS) - 1u;
+  const Geometry& g = a.c.geo;
+  const uint32_t D = g.D, G = g.G, R = g.R, gq = a.gq, S = a.S, h0 = hg * kRowHeads;
+  const uint32_t nh = std::min(kRowHeads, gq - h0);
+  const uint32_t b = unit / a.heads, kvh = unit % a.heads;
+  const uint32_t lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const uint64_t t0 = a.t_begin + (uint64_t)split * S;
+  const uint32_t ntok = static_cast<uint32_t>(std::min<uint64_t>(S, a.total - t0));
+  // the split's packed tokens [0, npk) / [0, npv), its tokens before the suffix [0, nseq), and the
+  // first token's offset into the residual, the window and the suffix
+  auto below = [&](uint64_t end) { return end > t0 ? static_cast<uint32_t>(std::min<uint64_t>(end - t0, ntok)) : 0u; };
+  const uint32_t npk = below(a.st.kq), npv = below(a.st.vq), nseq = below(a.seq);
+  const float* kres = a.c.kres + (uint64_t)unit * R * D;
+  const float* vring = a.c.vring + (uint64_t)unit * R * D;
+  float* q_lds = lds;                          // [4][D]
+  float* w_lds = lds + kRowHeads * D;          // [4][S]
+  float* xch = w_lds + kRowHeads * S;          // [256][4] dot products, then [rows][4][D] value sums
+
+  // fp32 row of token i of the split (any valid row for a packed one)
+  auto key_fp32_row = [&](uint32_t i) -> const float* {
+    if (i < nseq || a.suffix_k == nullptr) return kres + (i >= npk ? t0 + i - a.st.kq : 0) * D;
+    return a.suffix_k + unit * a.suffix_stride + (t0 + i - a.seq) * D;
+  };
+  auto value_fp32_row = [&](uint32_t i) -> const float* {
+    if (i < nseq || a.suffix_v == nullptr) {
+      uint32_t slot = a.st.vhead + (i >= npv ? static_cast<uint32_t>(t0 + i - a.st.vq) : 0u);  // < 2R
+      if (slot >= R) slot -= R;
+      return vring + (uint64_t)slot * D;
+    }
+    return a.suffix_v + unit * a.suffix_stride + (t0 + i - a.seq) * D;
+  };
+
+  // ---------------- values of up to kRowAhead rows per thread: four channels of every rows-th token
+  const uint32_t q4 = D / 4, rows = kThreads / q4, rs = threadIdx.x / q4, d0 = (threadIdx.x % q4) * 4;
+  // without packed values the packed candidates read the window instead (their arrays may not exist)
+  const uint32_t* vc = npv > 0 ? a.c.vcodes + unit * g.vcodes_unit() : reinterpret_cast<const uint32_t*>(vring);
+  const float2* vp = npv > 0 ? reinterpret_cast<const float2*>(a.c.vparams + unit * g.vparams_unit())
+                             : reinterpret_cast<const float2*>(vring);
+  uint32_t vwd[kRowAhead][4];
+  float2 vsz[kRowAhead];
+  float4 vf[kRowAhead];
+  auto load_values = [&](uint32_t k0) {
+#pragma unroll
+    for (uint32_t u = 0; u < kRowAhead; ++u) {
+      const uint32_t i = std::min(k0 + u * rows + rs, ntok - 1);
+      const uint64_t t = t0 + (npv > 0 ? std::min(i, npv - 1) : 0u);
+      const uint64_t tb = npv > 0 ? t / kValueBlock : 0;
+      const uint32_t tt = npv > 0 ? static_cast<uint32_t>(t % kValueBlock) : 0u;
+      const uint32_t* w = npv > 0 ? vc + (tb * D + d0) * VW + tt / PPW : vc;
+#pragma unroll
+      for (uint32_t e = 0; e < 4; ++e) vwd[u][e] = w[npv > 0 ? e * VW : 0];
+      vsz[u] = vp[npv > 0 ? (tb * g.ncg() + d0 / G) * kValueBlock + tt : 0];
+      vf[u] = *reinterpret_cast<const float4*>(value_fp32_row(i) + d0);
+    }
+  };
+
+  // ---------------- logits: lane (token, sixteenth of the channels)
+  const uint32_t NB = D / 16, TP = 64 / NB;
+  const uint32_t tp = std::min(lane / NB, TP - 1), j = lane % NB;
+  const uint32_t* kc = npk > 0 ? a.c.kcodes + unit * g.kcodes_unit() : reinterpret_cast<const uint32_t*>(kres);
+  const float2* kp = npk > 0 ? reinterpret_cast<const float2*>(a.c.kparams + unit * g.kparams_unit())
+                             : reinterpret_cast<const float2*>(kres);
+  uint32_t w[NW];
+  float sc[16], zr[16];
+  float4 f[4];
+  bool packed = false;
+  auto load_keys = [&](uint32_t k0) {
+    const uint32_t i = std::min(k0 + tp, ntok - 1);
+    const uint64_t t = t0 + (npk > 0 ? std::min(i, npk - 1) : 0u);
+    packed = i < npk;
+    lane_words<NW>(npk > 0 ? kc + t * g.kwords_per_token() + j * NW : kc, w);
+    lane_params(npk > 0 ? kp + t / G * D + j * 16 : kp, sc, zr);
+    const float4* fp = reinterpret_cast<const float4*>(key_fp32_row(i) + j * 16);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) f[k] = fp[k];
+  };
+  float x[16];
+  auto recon_keys = [&]() {
+    lane_recon<BITS>(w, sc, zr, x);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      x[4 * k] = packed ? x[4 * k] : f[k].x;
+      x[4 * k + 1] = packed ? x[4 * k + 1] : f[k].y;
+      x[4 * k + 2] = packed ? x[4 * k + 2] : f[k].z;
+      x[4 * k + 3] = packed ? x[4 * k + 3] : f[k].w;
+    }
+  };
+  load_keys(wave * TP);
+  for (uint32_t i = threadIdx.x; i < nh * D; i += kThreads)
+    q_lds[i] = a.query[((uint64_t)b * a.qh + kvh * gq + h0) * D + i];
+  __syncthreads();
+  recon_keys();
+  load_values(0);  // their round trip overlaps the dot products and the softmax
+  for (uint32_t k0 = wave * TP; k0 < ntok;) {
+    for (uint32_t h = 0; h < nh; ++h) {
+      const float4* qp = reinterpret_cast<const float4*>(q_lds + h * D + j * 16);
+      float v[2] = {0.f, 0.f};  // two chains: half the roundings after a large product
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float4 q = qp[k];
+        v[k / 2] = fmaf(x[4 * k], q.x, v[k / 2]);
+        v[k / 2] = fmaf(x[4 * k + 1], q.y, v[k / 2]);
+        v[k / 2] = fmaf(x[4 * k + 2], q.z, v[k / 2]);
+        v[k / 2] = fmaf(x[4 * k + 3], q.w, v[k / 2]);
+      }
+      xch[threadIdx.x * kRowHeads + h] = v[0] + v[1];
+    }
+    wave_lds_fence();
+    for (uint32_t o = lane; o < TP * kRowHeads; o += 64) {
+      const uint32_t r = o / kRowHeads, h = o % kRowHeads;
+      const float* src = xch + (wave * 64 + r * NB) * kRowHeads + h;
+      if (h < nh && k0 + r < ntok) {
+        float v = src[0];
+        for (uint32_t k = 1; k < NB; ++k) v += src[k * kRowHeads];
+        w_lds[h * S + k0 + r] = v * a.scale2;
+      }
+    }
+    wave_lds_fence();
+    k0 += 4 * TP;
+    if (k0 < ntok) {
+      load_keys(k0);
+      recon_keys();
+    }
+  }
+  __syncthreads();
+
+  // ---------------- softmax: wave h takes head h
+  float* part = a.ws + (((uint64_t)unit * a.nsplit_total + a.nsplit_fast + a.nsplit_win + split) * gq + h0) * (D + 2);
+  if (wave < nh) {
+    float* wl = w_lds + wave * S;
+    float m = -INFINITY;
+    for (uint32_t k = lane; k < ntok; k += 64) m = fmaxf(m, wl[k]);
+    m = warp_max(m);
+    float l = 0.f;
+    for (uint32_t k = lane; k < ntok; k += 64) {
+      const float e = exp2f(wl[k] - m);
+      wl[k] = e;
+      l += e;
+    }
+    l = warp_sum(l);
+    if (lane == 0) {
+      part[wave * (D + 2) + D] = m;
+      part[wave * (D + 2) + D + 1] = l;
+    }
+  }
+  __syncthreads();
+
+  // ---------------- value mix: thread (row slot rs, channels d0 .. d0 + 3)
+  float acc[kRowHeads][4] = {};
+  for (uint32_t k0 = 0; k0 < ntok;) {
+#pragma unroll
+    for (uint32_t u = 0; u < kRowAhead; ++u) {
+      const uint32_t i = k0 + u * rows + rs;
+      if (i >= ntok || rs >= rows) continue;
+      float x[4] = {vf[u].x, vf[u].y, vf[u].z, vf[u].w};
+      if (i < npv) {
+        const uint32_t sh = code_shift(BITS, static_cast<uint32_t>((t0 + i) % PPW));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = fmaf(static_cast<float>((vwd[u][e] >> sh) & MASK), vsz[u].x, vsz[u].y);
+      }
+#pragma unroll
+      for (uint32_t h = 0; h < kRowHeads; ++h) {
+        if (h >= nh) break;
+        const float wt = w_lds[h * S + i];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[h][e] = fmaf(x[e], wt, acc[h][e]);
+      }
+    }
+    k0 += rows * kRowAhead;
+    if (k0 < ntok) load_values(k0);
+  }
+  if (rs < rows) {
+#pragma unroll
+    for (uint32_t h = 0; h < kRowHeads; ++h)
+      if (h < nh)
+        *reinterpret_cast<float4*>(xch + (rs * kRowHeads + h) * D + d0) =
+            make_float4(acc[h][0], acc[h][1], acc[h][2], acc[h][3]);
+  }
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < nh * D; i += kThreads) {
+    const uint32_t h = i / D, d = i % D;
+    float v = xch[h * D + d];
+    for (uint32_t k = 1; k < rows; ++k) v += xch[(k * kRowHeads + h) * D + d];
+    part[h * (D + 2) + d] = v;
+  }
+}
+
+template <int BITS>
+__global__ void __launch_bounds__(kThreads) k_attn_rows(AttnArgs a) {
+  extern __shared__ float lds[];
+  const uint32_t vu = blockIdx.x / a.nsplit_gen;
+  row_split<BITS>(a, vu / a.hgroups_rows, blockIdx.x % a.nsplit_gen, vu % a.hgroups_rows, lds);
+}
+
+// ------------------------------------------------------------------ lane splits
+// Packed chunks of the shapes the matrix-core kernels do not take (head_dim a multiple of 16,
+// G a multiple of 16), on the vector ALU in f32 and in the reference's own arithmetic (each element
+// is reconstructed as fma(code, scale, zero) before it is used). A workgroup takes up to 16
+// consecutive 64-token chunks of a unit for HP query heads.
+//
+// What bounds it is vector issue (per element: unpacking, one fma of reconstruction, HP of use) and,
+// at one head, the cache lines its loads touch. So both contractions keep a (scale, zero) set in
+// registers over many elements instead of fetching pairs per element: a lane owns 16 channels of a
+// run of 16 tokens (keys; the run lies in one key group) or 16 tokens of a run of channels (values;
+// the run lies in one value group), and one to four code words hold its 16 codes. A (scale, zero)
+// pair in memory is then read by one lane of the workgroup.
+//  keys    lanes (run, channel sixteenth); the sixteenths of a token's dot product meet in LDS.
+//  values  lanes (chunk, token quarter); a channel's partial sums meet by a butterfly over the lanes.
+// 96 units x 5003 tokens x 96 channels at 4 bits, one head per unit: 26 us (k_attn_generic, which
+// blends a packed and an fp32 candidate per element: 460 us); 128 units x 32768 x 96 at 2 bits, four
+// heads: 227 us against 3411 us. Dot products run in two chains of eight channels: with one of
+// 16 the error against f64 attention was 10% above the generic splits', with two it is below.
+constexpr uint32_t kLaneChunks = 16;  // chunks per split, at most (64 lanes = 16 chunks x 4 quarters)
+constexpr uint32_t kLaneGroups = 256;  // workgroups a launch aims for, one per CU (measured: 1024 is 2-12% slower)
+
+// Sums of N values (N = 8 or 16) over each 16-lane row: lane r ends with value r * N / 16. Partners
+// r^15, r^7, r^2, r^1 each differ in the bit that decides which half of the remaining values a
+// lane keeps (with N = 8 the last step adds the lane's own value).
+template <int CTRL, int N>
+__device__ __forceinline__ void sum_step(const float* v, bool upper, float* o) {
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const float keep = upper ? v[N + j] : v[j], send = upper ? v[j] : v[N + j];
+    o[j] = keep + dpp_row<CTRL>(send);
+  }
+}
+template <int N>
+__device__ __forceinline__ float row_sums(const float (&v)[N], uint32_t lane) {
+  float a[N / 2], b[N / 4], c[N / 8];
+  sum_step<0x140, N / 2>(v, (lane & 8) != 0, a);
+  sum_step<0x141, N / 4>(a, (lane & 4) != 0, b);
+  sum_step<0x4E, N / 8>(b, (lane & 2) != 0, c);
+  if constexpr (N == 16) {
+    float d;
+    sum_step<0xB1, 1>(c, (lane & 1) != 0, &d);
+    return d;
+  } else {
+    return c[0] + dpp_row<0xB1>(c[0]);
+  }
+}
+
+constexpr uint32_t lane_rec(int hp) { return hp == 1 ? 4 : 4 * hp + 4; }  // floats a lane hands over
+// LDS floats of one workgroup: logits [HP][1024], key partials [256][lane_rec], reductions.
+constexpr uint32_t lane_lds_floats(int hp) {
+  return hp * kLaneChunks * 64 + kThreads * lane_rec(hp) + 2 * 4 * hp;
+}
+
+template <int BITS, int HP>
+__device__ __forceinline__ void lane_split(const AttnArgs& a, uint32_t unit, uint32_t split, uint32_t hg,
+                                           float* lds) {
+  constexpr uint32_t NW = BITS / 2;                // words of 16 codes
+  constexpr uint32_t REC = lane_rec(HP), ROW = kLaneChunks * 64;
+  constexpr uint32_t CB = HP == 4 ? 4 : 8;         // channels a lane takes per value batch
+  const Geometry& g = a.c.geo;
+  const uint32_t D = g.D, G = g.G, gq = a.gq, h0 = hg * HP;
+  const uint32_t b = unit / a.heads, kvh = unit % a.heads;
+  const uint32_t lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const uint32_t c0 = split * a.lane_cps;
+  const uint32_t nch = std::min(a.lane_cps, a.chunk_end - c0), ntok = nch * 64;
+  float* w_lds = lds;                       // [HP][ROW]
+  float* xch = lds + HP * ROW + wave * 64 * REC;
+  float* red = lds + HP * ROW + kThreads * REC;  // [2][4 waves][HP]
+
+  // ---------------- logits
+  float mx[HP];
+#pragma unroll
+  for (int h = 0; h < HP; ++h) mx[h] = -INFINITY;
+  {
+    const uint32_t NB = D / 16, TP = 64 / NB;  // lanes per token, runs per wave
+    const uint32_t tp = lane / NB, j = lane % NB;
+    const bool lives = tp < TP;
+    const uint32_t nsub = nch * 4, kw = g.kwords_per_token();
+    float q[HP][16];
+#pragma unroll
+    for (int h = 0; h < HP; ++h) {
+      const float* qp = a.query + ((uint64_t)b * a.qh + kvh * gq + std::min(h0 + h, gq - 1)) * D + j * 16;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) q[h][i] = qp[i];
+    }
+    const uint32_t* kc = a.c.kcodes + unit * g.kcodes_unit() + (uint64_t)c0 * 64 * kw + j * NW;
+    const float2* kp = reinterpret_cast<const float2*>(a.c.kparams + unit * g.kparams_unit()) + j * 16;
+    for (uint32_t s0 = wave * TP; s0 < nsub; s0 += 4 * TP) {
+      // run `sub` of 16 tokens; lanes past the last one take it again and write nothing
+      const uint32_t sub = std::min(s0 + (lives ? tp : TP - 1), nsub - 1);
+      float sc[16], zr[16];
+      lane_params(kp + (uint64_t)((c0 * 64 + sub * 16) / G) * D, sc, zr);
+      const uint32_t* wp = kc + (uint64_t)sub * 16 * kw;
+      uint32_t w[2][4][NW];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) lane_words<NW>(wp + i * kw, w[0][i]);
+#pragma unroll
+      for (int t4 = 0; t4 < 4; ++t4) {
+        if (t4 < 3) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) lane_words<NW>(wp + (4 * t4 + 4 + i) * kw, w[(t4 + 1) % 2][i]);
+        }
+        float acc[4][HP];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float x[16];
+          lane_recon<BITS>(w[t4 % 2][i], sc, zr, x);
+#pragma unroll
+          for (int h = 0; h < HP; ++h) {
+            // two chains: half the roundings after a large product
+            float v = x[0] * q[h][0], u = x[8] * q[h][8];
+#pragma unroll
+            for (int e = 1; e < 8; ++e) {
+              v = fmaf(x[e], q[h][e], v);
+              u = fmaf(x[8 + e], q[h][8 + e], u);
+            }
+            acc[i][h] = v + u;
+          }
+        }
+        // the NB sixteenths of each (run, token, head) meet in the wave's own LDS buffer
+        float* mine = xch + lane * REC;
+#pragma unroll
+        for (int k = 0; k < HP; ++k)
+          *reinterpret_cast<float4*>(mine + 4 * k) =
+              make_float4(acc[4 * k / HP][4 * k % HP], acc[(4 * k + 1) / HP][(4 * k + 1) % HP],
+                          acc[(4 * k + 2) / HP][(4 * k + 2) % HP], acc[(4 * k + 3) / HP][(4 * k + 3) % HP]);
+        wave_lds_fence();
+        for (uint32_t o = lane; o < TP * 4 * HP; o += 64) {
+          const uint32_t r = o / (4 * HP), ih = o % (4 * HP), run = s0 + r;
+          const float* src = xch + r * NB * REC + ih;
+          float v = src[0];
+          for (uint32_t k = 1; k < NB; ++k) v += src[k * REC];
+          v *= a.scale2;
+          if (run < nsub) w_lds[(ih % HP) * ROW + run * 16 + 4 * t4 + ih / HP] = v;
+        }
+        wave_lds_fence();
+      }
+    }
+  }
+  __syncthreads();
+
+  // ---------------- softmax over the split: thread t takes tokens 4t .. 4t + 3 of every head
+  {
+    const bool lives = threadIdx.x * 4 < ntok;
+#pragma unroll
+    for (int h = 0; h < HP; ++h) {
+      if (lives) {
+        const float4 v = *reinterpret_cast<const float4*>(w_lds + h * ROW + threadIdx.x * 4);
+        mx[h] = fmaxf(fmaxf(v.x, v.y), fmaxf(v.z, v.w));
+      }
+      mx[h] = warp_max(mx[h]);
+      if (lane == 0) red[wave * HP + h] = mx[h];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < HP; ++h) {
+      float m = red[h];
+#pragma unroll
+      for (int wv = 1; wv < 4; ++wv) m = fmaxf(m, red[wv * HP + h]);
+      float l = 0.f;
+      if (lives) {
+        float4* p = reinterpret_cast<float4*>(w_lds + h * ROW + threadIdx.x * 4);
+        float4 v = *p;
+        v.x = exp2f(v.x - m);
+        v.y = exp2f(v.y - m);
+        v.z = exp2f(v.z - m);
+        v.w = exp2f(v.w - m);
+        l = (v.x + v.y) + (v.z + v.w);
+        *p = v;
+      }
+      l = warp_sum(l);
+      if (lane == 0) red[4 * HP + wave * HP + h] = l;
+      mx[h] = m;
+    }
+    __syncthreads();
+  }
+  float* part = a.ws + (((uint64_t)unit * a.nsplit_total + split) * gq + h0) * (D + 2);
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int h = 0; h < HP; ++h) {
+      if (h0 + h >= gq) break;
+      float l = red[4 * HP + h];
+#pragma unroll
+      for (int wv = 1; wv < 4; ++wv) l += red[4 * HP + wv * HP + h];
+      part[h * (D + 2) + D] = mx[h];
+      part[h * (D + 2) + D + 1] = l;
+    }
+  }
+
+  // ---------------- value mix
+  {
+    const uint32_t lcs = a.lane_log, CS = 1u << lcs;  // chunk slots: 4, 8 or 16
+    const uint32_t quarter = lane & 3, cs = (lane >> 2) & (CS - 1), chs = lane >> (2 + lcs);
+    const uint32_t slots = 16u >> lcs;             // channel batches side by side in a wave
+    const bool lives = cs < nch;
+    const uint32_t ch = c0 + (lives ? cs : 0);     // idle slots read the first chunk, at weight 0
+    const uint32_t ncg = g.ncg(), vw = g.vwords_per_channel(), nbatch = D / CB;
+    float w[HP][16];
+#pragma unroll
+    for (int h = 0; h < HP; ++h) {
+      const float4* p = reinterpret_cast<const float4*>(w_lds + h * ROW + (lives ? cs : 0) * 64 + quarter * 16);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float4 v = p[k];
+        w[h][4 * k] = lives ? v.x : 0.f;
+        w[h][4 * k + 1] = lives ? v.y : 0.f;
+        w[h][4 * k + 2] = lives ? v.z : 0.f;
+        w[h][4 * k + 3] = lives ? v.w : 0.f;
+      }
+    }
+    const uint32_t* vc = a.c.vcodes + unit * g.vcodes_unit() + (uint64_t)ch * D * vw + quarter * NW;
+    const float2* vp = reinterpret_cast<const float2*>(a.c.vparams + unit * g.vparams_unit()) +
+                       (uint64_t)ch * ncg * kValueBlock + quarter * 16;
+    for (uint32_t b0 = wave * slots; b0 < nbatch; b0 += 4 * slots) {
+      const uint32_t bi = b0 + chs, d0 = std::min(bi, nbatch - 1) * CB;
+      float sc[16], zr[16];
+      lane_params(vp + (d0 / G) * kValueBlock, sc, zr);
+      float acc[CB * HP];
+      uint32_t wd[2][2][NW];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) lane_words<NW>(vc + (d0 + i) * vw, wd[0][i]);
+#pragma unroll
+      for (int c2 = 0; c2 < (int)CB / 2; ++c2) {
+        if (c2 + 1 < (int)CB / 2) {
+#pragma unroll
+          for (int i = 0; i < 2; ++i) lane_words<NW>(vc + (d0 + 2 * c2 + 2 + i) * vw, wd[(c2 + 1) % 2][i]);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          float x[16];
+          lane_recon<BITS>(wd[c2 % 2][i], sc, zr, x);
+#pragma unroll
+          for (int h = 0; h < HP; ++h) {
+            float v = x[0] * w[h][0];
+#pragma unroll
+            for (int e = 1; e < 16; ++e) v = fmaf(x[e], w[h][e], v);
+            acc[(2 * c2 + i) * HP + h] = v;
+          }
+        }
+      }
+      // over the batch's lanes: the row, then the rows of a 32- or 64-lane slot
+      float v = row_sums<CB * HP>(acc, lane);
+      if (lcs >= 3) v += __shfl_xor(v, 16);
+      if (lcs >= 4) v += __shfl_xor(v, 32);
+      const uint32_t idx = (lane % 16) * (CB * HP) / 16, h = idx % HP;
+      const bool writer = (lane & (4 * CS - 1)) < 16 && lane % (16 / (CB * HP)) == 0;
+      if (writer && bi < nbatch && h0 + h < gq) part[h * (D + 2) + d0 + idx / HP] = v;
+    }
+  }
+}
+
+// The row splits over the tokens after the packed chunks come first in the grid (their latency
+// overlaps the packed ones), then the lane splits of every (unit, head group).
+template <int BITS, int HP>
+__global__ void __launch_bounds__(kThreads, HP == 4 || (HP == 2 && BITS == 8) ? 3 : 4) k_attn_lanes(AttnArgs a) {
+  extern __shared__ float lds[];
+  const uint32_t ngen = a.units * a.hgroups_rows * a.nsplit_gen;
+  if (blockIdx.x < ngen) {
+    const uint32_t vr = blockIdx.x / a.nsplit_gen;
+    row_split<BITS>(a, vr / a.hgroups_rows, blockIdx.x % a.nsplit_gen, vr % a.hgroups_rows, lds);
+    return;
+  }
+  const uint32_t blk = blockIdx.x - ngen, vu = blk / a.nsplit_fast;
+  lane_split<BITS, HP>(a, vu / a.hgroups, blk % a.nsplit_fast, vu % a.hgroups, lds);
+}
+
+// ------------------------------------------------------------------ chunk launch
 // Chunk launch: workgroups [0, units*nsplit_win) take one window / suffix chunk each (MIXED
 // path, started first), the rest a split of 4*kFastCpw packed chunks. Every split writes its
 // partial with plain stores; the merge launch that follows on the stream reads them.
@@ -1240,10 +1797,10 @@ __global__ void __launch_bounds__(kThreads, SMALL ? 2 : fast_min_groups(BITS, NR
   extern __shared__ float lds[];
   // workgroups of (unit, head group) pairs: vu = unit * hgroups + hg. First in the grid, so
   // their latency-bound fp32 rows overlap the packed chunks: at head_dim 128 the window /
-  // suffix chunks, at other head_dims the generic splits over the tokens after the packed
+  // suffix chunks, at other head_dims the row splits over the tokens after the packed
   // chunks (one of the two counts is zero).
   const uint32_t nwin = a.units * a.hgroups * a.nsplit_win;
-  const uint32_t ngen = a.units * a.nsplit_gen;
+  const uint32_t ngen = a.units * a.hgroups_rows * a.nsplit_gen;
   if constexpr (D == 128) {
     if (blockIdx.x < nwin) {
       const uint32_t vu = blockIdx.x / a.nsplit_win;
@@ -1252,7 +1809,8 @@ __global__ void __launch_bounds__(kThreads, SMALL ? 2 : fast_min_groups(BITS, NR
     }
   } else {
     if (blockIdx.x < ngen) {
-      generic_split<BITS, D, 0>(a, blockIdx.x / a.nsplit_gen, blockIdx.x % a.nsplit_gen, lds);
+      const uint32_t vr = blockIdx.x / a.nsplit_gen;
+      row_split<BITS>(a, vr / a.hgroups_rows, blockIdx.x % a.nsplit_gen, vr % a.hgroups_rows, lds);
       return;
     }
   }
@@ -3076,9 +3634,24 @@ uint32_t head_groups(uint32_t D, uint32_t gq) {
   return (gq + per - 1) / per;
 }
 
+// Shapes whose packed chunks take the lane splits: the rest with whole runs of 16 channels and
+// tokens per group (a lane's 16 codes then share their scales). Other groups (4, 8, 12, 24 ...)
+// stay on the row splits, whose scales are read per token, or on the generic splits.
+bool lanes_eligible(const AttnProblem& p) {
+  const Geometry& g = p.cache.geo;
+  return !fast_eligible(p) && g.G % 16 == 0 && g.D % 16 == 0 && (g.bits == 2 || g.bits == 4 || g.bits == 8);
+}
+// query heads per lane-split workgroup
+uint32_t lane_heads(uint32_t gq) { return gq <= 2 ? gq : 4u; }
+
 // MFMA chunks: [0, floor(vq/64)) (keys and values packed; vq <= kq). Everything after
-// (value window, its band of packed keys, session suffix) goes to the generic kernel.
-AttnArgs make_args(const AttnProblem& p, float* ws) {
+// (value window, its band of packed keys, session suffix) goes to window chunks or row splits.
+// How many splits a plan takes: what pays, as few as its kernels go, or the plan by which the
+// allocation-free attention counts a call's partials (no lane splits, the rest in splits of 256
+// tokens, or of 16 to 64 behind matrix-core chunks).
+enum class SplitPlan { kUsual, kFewest, kCounted };
+
+AttnArgs make_args_as(const AttnProblem& p, float* ws, SplitPlan plan) {
   AttnArgs a{};
   a.c = p.cache;
   a.st = p.st;
@@ -3100,23 +3673,34 @@ AttnArgs make_args(const AttnProblem& p, float* ws) {
   // The MFMA path covers every 64-token chunk once some keys are packed: chunks
   // [0, floor(vq/64)) (keys and values all packed) in one launch, the rest (the fp32 value
   // window and key residual, the session suffix) in a second launch of the MIXED kernel.
-  // Without packed keys, or for other shapes, the generic splits cover everything.
-  // At head_dim 64 and 256 the MFMA launch takes only the fully packed chunks and the generic
-  // splits the rest.
-  const bool fast = fast_eligible(p) && p.st.kq > 0;
+  // At other head_dims the MFMA launch takes only the fully packed chunks and row splits the rest,
+  // as behind the lane splits of other shapes. Without packed chunks row splits cover everything.
+  const bool lanes = plan != SplitPlan::kCounted && lanes_eligible(p) && std::min(p.st.kq, p.st.vq) >= 64;
+  const bool fast = !lanes && fast_eligible(p) && p.st.kq > 0;
   const bool fast_win = fast && p.cache.geo.D == 128;
   a.S = split_tokens(a.gq);
   a.chunk_begin = 0;
-  a.chunk_end = fast ? static_cast<uint32_t>(std::min(p.st.kq, p.st.vq) / 64) : 0;
+  a.chunk_end = fast || lanes ? static_cast<uint32_t>(std::min(p.st.kq, p.st.vq) / 64) : 0;
   a.win_begin = a.chunk_end;
   a.win_end = fast_win ? static_cast<uint32_t>((a.total + 63) / 64) : a.chunk_end;
-  a.hgroups = fast ? head_groups(p.cache.geo.D, a.gq) : 1u;
+  a.hgroups = lanes ? (a.gq + lane_heads(a.gq) - 1) / lane_heads(a.gq) : fast ? head_groups(p.cache.geo.D, a.gq) : 1u;
   a.gshift = fast ? static_cast<uint32_t>(__builtin_ctz(p.cache.geo.G)) : 5u;
   a.wide = !(fast && wide_shape(p)) ? 0u : wide16_shape(p) ? 2u : 1u;
   a.hgroups_fast = a.wide == 2 ? a.gq / kWide16Heads : a.hgroups;
   // packed splits per unit: at most kFastCpw (wide_cpw) chunks per wave, at least one, and at
   // least kFastGroups workgroups (over units and head groups) when the chunks allow
-  {
+  a.lane_cps = a.lane_log = 0;
+  if (lanes) {
+    // up to 16 chunks per split, fewer (down to 4, which fill the value phase's 16-lane rows)
+    // while the launch would have fewer than kLaneGroups workgroups; then evened out
+    const uint32_t vu = p.cache.geo.units * a.hgroups;
+    uint32_t cps = kLaneChunks;
+    while (plan == SplitPlan::kUsual && cps > 4 && (uint64_t)vu * ((a.chunk_end + cps - 1) / cps) < kLaneGroups) cps /= 2;
+    a.nsplit_fast = (a.chunk_end + cps - 1) / cps;
+    a.lane_cps = (a.chunk_end + a.nsplit_fast - 1) / a.nsplit_fast;
+    a.nsplit_fast = (a.chunk_end + a.lane_cps - 1) / a.lane_cps;
+    a.lane_log = a.lane_cps > 8 ? 4 : a.lane_cps > 4 ? 3 : 2;
+  } else {
     const uint32_t units = p.cache.geo.units * a.hgroups_fast;
     const uint32_t cpw = a.wide == 2 ? static_cast<uint32_t>(kWide16Cpw)
                          : a.wide ? static_cast<uint32_t>(wide_cpw(static_cast<int>(p.cache.geo.bits)))
@@ -3126,13 +3710,22 @@ AttnArgs make_args(const AttnProblem& p, float* ws) {
     a.nsplit_fast = std::min(most, std::max(fewest, (kFastGroups + units - 1) / units));
   }
   a.nsplit_win = a.win_end - a.win_begin;  // one chunk per workgroup, a quarter per wave
-  a.t_begin = fast_win ? a.total : fast ? (uint64_t)a.chunk_end * 64 : 0;
-  if (fast && !fast_win) {
-    // the rest is short (the fp32 residual and window, a suffix): shorter splits, down to 16
-    // tokens while the rest would fill fewer than ~1024 workgroups
+  a.t_begin = fast_win ? a.total : fast || lanes ? (uint64_t)a.chunk_end * 64 : 0;
+  // Row splits: one pass of a workgroup (at least 16 tokens) while the launch has few workgroups,
+  // doubled while four per CU remain.
+  a.hgroups_rows = p.cache.geo.D % 16 == 0 ? (a.gq + kRowHeads - 1) / kRowHeads : 0u;
+  if (plan == SplitPlan::kFewest) a.S = kRowMaxTokens;
+  if (plan == SplitPlan::kCounted && fast && !fast_win) {
     a.S = std::max(32u, a.S / 4);
     const uint64_t rest = a.total - a.t_begin;
     while (a.S > 16 && (uint64_t)p.cache.geo.units * ((rest + a.S - 1) / a.S) < 1024) a.S >>= 1;
+  }
+  if (a.hgroups_rows != 0 && plan == SplitPlan::kUsual) {
+    const uint64_t rest = a.total - a.t_begin, vu = (uint64_t)p.cache.geo.units * a.hgroups_rows;
+    const uint32_t pass = std::min(64u, std::max(16u, row_pass(p.cache.geo.D)));
+    auto splits = [&](uint32_t S) { return (rest + S - 1) / S; };
+    a.S = pass;
+    while (2 * a.S <= kRowMaxTokens && vu * splits(2 * a.S) >= kRowGroups) a.S *= 2;
   }
   a.nsplit_gen = static_cast<uint32_t>((a.total - a.t_begin + a.S - 1) / a.S);
   a.nsplit_total = a.nsplit_fast + a.nsplit_win + a.nsplit_gen;
@@ -3142,6 +3735,23 @@ AttnArgs make_args(const AttnProblem& p, float* ws) {
   a.nsess = 0;
   a.gemm_end = 0;
   a.q_sess_stride = a.ws_sess_stride = 0;
+  return a;
+}
+
+uint64_t workspace_floats(const AttnArgs& a) {
+  return (uint64_t)a.units * a.nsplit_total * a.gq * (a.c.geo.D + 2);
+}
+
+// The lane and row splits can take more partials than the counted plan; a call whose counted
+// partials fit the static workspace keeps to a plan that does too, so that the allocation-free
+// attention takes (and refuses) the same calls whatever splits pay.
+AttnArgs make_args(const AttnProblem& p, float* ws) {
+  const AttnArgs a = make_args_as(p, ws, SplitPlan::kUsual);
+  if (workspace_floats(a) <= kStaticWorkspaceFloats) return a;
+  for (SplitPlan plan : {SplitPlan::kFewest, SplitPlan::kCounted}) {
+    const AttnArgs f = make_args_as(p, ws, plan);
+    if (workspace_floats(f) <= kStaticWorkspaceFloats) return f;
+  }
   return a;
 }
 
@@ -3157,10 +3767,11 @@ hipError_t launch_fast(const AttnArgs& a, double bytes, hipStream_t stream) {
   const bool small = D == 128 && NRS == 1 && small_launch(a);
   const size_t logits = (size_t)4 * NH * ((a.nsplit_fast > 0 && !small ? fast_cpw(BITS, NRS) : 1) * 64 + kRowPad);
   const size_t combine = (size_t)4 * NH * (D + 2);
-  const size_t gen = a.nsplit_gen > 0 ? (size_t)a.gq * (D + a.S) : 0;  // generic splits' q and weights
+  const size_t gen = a.nsplit_gen > 0 ? row_lds_floats(D, a.S) : 0;
   const size_t lds = std::max(std::max(logits, combine), gen) * sizeof(float);
   TimedLaunch timed(KIVI_KERNEL_ATTN_PACKED, stream, bytes);
-  const uint32_t grid = a.units * (a.hgroups * a.nsplit_win + a.hgroups_fast * a.nsplit_fast + a.nsplit_gen);
+  const uint32_t grid =
+      a.units * (a.hgroups * a.nsplit_win + a.hgroups_fast * a.nsplit_fast + a.hgroups_rows * a.nsplit_gen);
   if constexpr (D == 128 && NRS == 2) {
     if (a.wide == 2) {
       const size_t wide = (size_t)4 * kWide16Heads * (kWide16Cpw * 64 + kRowPad);
@@ -3191,7 +3802,35 @@ hipError_t launch_fast(const AttnArgs& a, double bytes, hipStream_t stream) {
   return hipGetLastError();
 }
 
+template <int BITS, int HP>
+hipError_t launch_lanes(const AttnArgs& a, double bytes, hipStream_t stream) {
+  const size_t gen = a.nsplit_gen > 0 ? row_lds_floats(a.c.geo.D, a.S) : 0;
+  const size_t lds = std::max<size_t>(lane_lds_floats(HP), gen) * sizeof(float);
+  const hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(&k_attn_lanes<BITS, HP>), lds);
+  if (e != hipSuccess) return e;
+  TimedLaunch timed(KIVI_KERNEL_ATTN_PACKED, stream, bytes);
+  const uint32_t grid = a.units * (a.hgroups * a.nsplit_fast + a.hgroups_rows * a.nsplit_gen);
+  k_attn_lanes<BITS, HP><<<grid, kThreads, lds, stream>>>(a);
+  return hipGetLastError();
+}
+
+hipError_t dispatch_lanes(const AttnArgs& a, double bytes, hipStream_t stream) {
+  switch (a.c.geo.bits * 10 + lane_heads(a.gq)) {
+    case 21: return launch_lanes<2, 1>(a, bytes, stream);
+    case 22: return launch_lanes<2, 2>(a, bytes, stream);
+    case 24: return launch_lanes<2, 4>(a, bytes, stream);
+    case 41: return launch_lanes<4, 1>(a, bytes, stream);
+    case 42: return launch_lanes<4, 2>(a, bytes, stream);
+    case 44: return launch_lanes<4, 4>(a, bytes, stream);
+    case 81: return launch_lanes<8, 1>(a, bytes, stream);
+    case 82: return launch_lanes<8, 2>(a, bytes, stream);
+    case 84: return launch_lanes<8, 4>(a, bytes, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
 hipError_t dispatch_fast(const AttnArgs& a, double bytes, hipStream_t stream) {
+  if (a.lane_cps != 0) return dispatch_lanes(a, bytes, stream);
   const uint32_t D = a.c.geo.D;
   const int nrs = fast_nrs(D, a.gq);
   switch (D * 100 + a.c.geo.bits * 10 + nrs) {
@@ -3218,8 +3857,19 @@ hipError_t dispatch_fast(const AttnArgs& a, double bytes, hipStream_t stream) {
 }
 
 hipError_t dispatch_generic(const AttnArgs& a, hipStream_t stream) {
+  if (a.hgroups_rows != 0) {
+    const size_t lds = row_lds_floats(a.c.geo.D, a.S) * sizeof(float);
+    const uint32_t grid = a.units * a.hgroups_rows * a.nsplit_gen;
+    switch (a.c.geo.bits) {
+      case 2: k_attn_rows<2><<<grid, kThreads, lds, stream>>>(a); break;
+      case 4: k_attn_rows<4><<<grid, kThreads, lds, stream>>>(a); break;
+      case 8: k_attn_rows<8><<<grid, kThreads, lds, stream>>>(a); break;
+      default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+  }
   const size_t lds = ((size_t)a.gq * a.c.geo.D + (size_t)a.gq * a.S) * sizeof(float);
-  k_attn_generic<0, 0, 0><<<a.units * a.nsplit_gen, kThreads, lds, stream>>>(a);
+  k_attn_generic<<<a.units * a.nsplit_gen, kThreads, lds, stream>>>(a);
   return hipGetLastError();
 }
 
@@ -3276,8 +3926,11 @@ bool attention_fuses_decode(const AttnProblem& p) {
 }
 
 size_t attention_workspace_floats(const AttnProblem& p) {
-  const AttnArgs a = make_args(p, nullptr);
-  return (size_t)p.cache.geo.units * a.nsplit_total * a.gq * (p.cache.geo.D + 2);
+  return workspace_floats(make_args(p, nullptr));
+}
+
+size_t attention_counted_floats(const AttnProblem& p) {
+  return workspace_floats(make_args_as(p, nullptr, SplitPlan::kCounted));
 }
 
 hipError_t launch_attention(const AttnProblem& p, float* workspace, hipStream_t stream) {
@@ -3296,7 +3949,7 @@ hipError_t launch_attention(const AttnProblem& p, float* workspace, hipStream_t 
   const double tail_bytes = units * (kp * key_tok + vp * val_tok + (kd + vd + 2.0 * p.suffix_len) * row);
   if (a.nsplit_fast > 0 || a.nsplit_win > 0) {
     // one launch over every chunk (the tokens after the packed chunks as window chunks at
-    // head_dim 128, as generic splits in the same grid otherwise): packed tokens at packed
+    // head_dim 128, as row splits in the same grid otherwise): packed tokens at packed
     // cost, the rest as fp32 rows
     const double kpt = (double)std::min<uint64_t>(kq, p.seq), vpt = (double)vq;
     const double fp32_rows = (double)(p.seq - kq) + (double)(p.seq - vq) + 2.0 * p.suffix_len;
