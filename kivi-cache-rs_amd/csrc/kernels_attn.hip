@@ -3646,6 +3646,25 @@ uint32_t lane_heads(uint32_t gq) { return gq <= 2 ? gq : 4u; }
 
 // MFMA chunks: [0, floor(vq/64)) (keys and values packed; vq <= kq). Everything after
 // (value window, its band of packed keys, session suffix) goes to window chunks or row splits.
+// Packed splits per unit near `base` (at most four times as many, at most `most`) that leave the
+// busiest CU the fewest chunk steps: workgroups per CU, rounded up, times chunks per wave, rounded
+// up. base itself unless another count saves a fifth: below that, more workgroups measured slower as
+// often as faster. What it mends is a grid just above a multiple of the CUs, or waves just above
+// a whole chunk. 56 units x 91 chunks at head_dim 256, 4 bits: 5 splits leave some CUs two
+// workgroups of 5 chunks per wave, 9 splits two of 3: 51.7 -> 43.1 us; 24 units x 310 chunks at
+// head_dim 192, 8 bits: 58.8 -> 44.3 us; 160 units x 53 chunks at head_dim 128, 2 bits: 28.9 ->
+// 24.3 us. Even grids (2048 workgroups of 8 chunks, 256 of 5) keep their counts.
+uint32_t level_splits(uint32_t base, uint32_t most, uint32_t units, uint32_t chunks) {
+  auto steps = [&](uint32_t ns) {
+    return (uint64_t)(((uint64_t)units * ns + kFastGroups - 1) / kFastGroups) * ((chunks + 4 * ns - 1) / (4 * ns));
+  };
+  if (base == 0) return base;
+  uint32_t best = base;
+  for (uint32_t ns = base + 1; ns <= std::min(most, 4 * base); ++ns)
+    if (steps(ns) < steps(best)) best = ns;
+  return steps(best) * 5 <= steps(base) * 4 ? best : base;
+}
+
 // How many splits a plan takes: what pays, as few as its kernels go, or the plan by which the
 // allocation-free attention counts a call's partials (no lane splits, the rest in splits of 256
 // tokens, or of 16 to 64 behind matrix-core chunks).
@@ -3708,6 +3727,7 @@ AttnArgs make_args_as(const AttnProblem& p, float* ws, SplitPlan plan) {
     const uint32_t fewest = (a.chunk_end + 4 * cpw - 1) / (4 * cpw);
     const uint32_t most = (a.chunk_end + 3) / 4;
     a.nsplit_fast = std::min(most, std::max(fewest, (kFastGroups + units - 1) / units));
+    if (plan == SplitPlan::kUsual) a.nsplit_fast = level_splits(a.nsplit_fast, most, units, a.chunk_end);
   }
   a.nsplit_win = a.win_end - a.win_begin;  // one chunk per workgroup, a quarter per wave
   a.t_begin = fast_win ? a.total : fast || lanes ? (uint64_t)a.chunk_end * 64 : 0;

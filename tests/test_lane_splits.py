@@ -20,6 +20,39 @@ from test_parity import assert_close
 
 pytestmark = pytest.mark.gpu
 
+def dense_attention(cache, q, heads, scale):
+    """f64 attention of q [batch, heads, gq, dim] over the cache's dequantized rows."""
+    batch, _, _, dim = q.shape
+    kd, vd = (x.reshape(batch, heads, -1, dim).astype(np.float64) for x in cache.dequantize())
+    logits = q.astype(np.float64) @ kd.swapaxes(-1, -2) * float(scale)
+    w = np.exp(logits - logits.max(-1, keepdims=True))
+    return (w / w.sum(-1, keepdims=True)) @ vd
+
+
+# Grids the split planner evens out (matrix-core kernels): a few workgroups above 256, waves just
+# above a whole chunk. Bar of the matrix-core path against f64 (22-bit products): 1e-4.
+UNEVEN = [
+    # bits, group, dim, batch, kv heads, query heads per KV head, tokens
+    (2, 32, 64, 5, 8, 4, 2000),    # 40 units x 29 chunks: 7 splits of 2 chunks per wave -> 8 of 1
+    (4, 64, 256, 7, 8, 1, 700),    # 56 units x 9 chunks
+    (8, 32, 128, 5, 8, 3, 2500),
+    (4, 32, 128, 3, 8, 7, 3000),   # eight-head kernel
+]
+
+
+@pytest.mark.parametrize("case", UNEVEN)
+def test_evened_grids_against_dense(amd, case):
+    bits, group, dim, batch, heads, gq, n = case
+    rng = np.random.default_rng(4700 + n)
+    a = KiviCache(amd, KiviConfig(bits, group, 128), batch, heads, dim)
+    k, v = (rng.standard_normal((batch, heads, n, dim)).astype(np.float32) for _ in range(2))
+    q = rng.standard_normal((batch, heads, gq, dim)).astype(np.float32)
+    a.append(k, v, n)
+    scale = np.float32(1 / np.sqrt(dim))
+    got = a.attention(q, heads * gq, scale).reshape(q.shape)
+    assert np.abs(got - dense_attention(a, q, heads, scale)).max() < 1e-4
+
+
 CASES = [
     # bits, group, residual, dim, batch, kv heads, query heads per KV head, tokens
     (2, 32, 32, 32, 1, 1, 1, 96),          # one packed chunk
@@ -48,11 +81,7 @@ def test_lane_splits_against_oracle_and_dense(amd, oracle, case):
     a = KiviCache(amd, cfg, batch, heads, dim)
     a.append(k, v, n)
     got = a.attention(q, qh, scale).reshape(batch, heads, gq, dim)
-    kd, vd = (x.reshape(batch, heads, n, dim).astype(np.float64) for x in a.dequantize())
-    logits = q.reshape(batch, heads, gq, dim).astype(np.float64) @ kd.swapaxes(-1, -2) * float(scale)
-    w = np.exp(logits - logits.max(-1, keepdims=True))
-    dense = (w / w.sum(-1, keepdims=True)) @ vd
-    assert np.abs(got - dense).max() < 2e-5
+    assert np.abs(got - dense_attention(a, q.reshape(got.shape), heads, scale)).max() < 2e-5
     if batch * heads < 10:
         o = KiviCache(oracle, cfg, batch, heads, dim)
         o.append(k, v, n)
