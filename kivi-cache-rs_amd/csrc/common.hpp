@@ -319,10 +319,11 @@ struct SessionTable {
   SessionDesc d[kMaxLaunchSessions];
 };
 
-// n sessions sharing one prefix: each workgroup of the prefix's packed chunks serves every
-// session in turn (the chunk data stays in L2 between sessions, so HBM sees the prefix once);
-// the prefix window and each session's suffix run per session. Returns hipErrorNotSupported
-// for shapes without the packed-chunk path (the caller then runs the sessions one by one).
+// n sessions sharing one prefix: the prefix's packed chunks serve all sessions' rows (session, head)
+// at once, 16 rows per pass over them or, from kSharedMinRows rows on, as a GEMM operand (which takes
+// the prefix window too); each session's suffix (and window) runs per session. Returns
+// hipErrorNotSupported for shapes without the packed-chunk path (the caller then runs the sessions
+// one by one).
 struct SessionsProblem {
   CacheView cache;
   SeqState st;

@@ -2345,7 +2345,28 @@ constexpr int kWide16Heads = 16;
 constexpr int kWide16Cpw = 4;     // chunks per wave: four chunks of 16 heads' logits, 16.6 KB
 constexpr int kWide16Blocks = 2;  // workgroups per CU (66.6 KB of LDS each)
 
+//
+// SESS: the columns are rows (session, head) of a batched call, hg the group of 16 rows: each row
+// has its own query pointer, its own operand range (sessions' queries may differ in magnitude) and
+// its session's partials. Its codes are taken about the middle of their range (exact in f16) and
+// its zeros moved there, x = (code - mid) scale + (zero + mid scale): a group's zero is its minimum,
+// so uncentred code and zero terms largely cancel in the sums: 13 sessions of four heads over 30007
+// tokens at 4 bits are 1.9e-6 off f64 attention uncentred, 7e-7 centred (1.4e-6 in the GEMM form),
+// for 3-5% of the time.
+// The middle of the code range (a value f16 holds, whole at 8 bits).
+constexpr float code_mid(int bits) { return bits == 8 ? 128.f : bits == 4 ? 7.5f : 1.5f; }
 template <int BITS>
+__device__ __forceinline__ h8 centred(h8 codes) {  // codes times 2^kExp as the code operands are
+  constexpr int kExp = CodeUnit<BITS>::kExp;
+  const _Float16 m = (_Float16)(code_mid(BITS) * (kExp == 0 ? 1.0f : kExp == -1 ? 0.5f : 0.001953125f));
+  return codes - h8{m, m, m, m, m, m, m, m};
+}
+__device__ __forceinline__ void centre_pairs(float4& p, float mid) {
+  p.y = fmaf(mid, p.x, p.y);
+  p.w = fmaf(mid, p.z, p.w);
+}
+
+template <int BITS, bool SESS>
 __device__ __forceinline__ void wide16_split(const AttnArgs& a, uint32_t unit, uint32_t split, uint32_t hg,
                                              float* lds) {
   constexpr int CPW = kWide16Cpw, NH = kWide16Heads, D = 128;
@@ -2375,13 +2396,16 @@ __device__ __forceinline__ void wide16_split(const AttnArgs& a, uint32_t unit, u
     wide_load_key_params(a, unit, chunk_of(0), lane, kp0, kp1);
     wide_load_keys<BITS>(a, unit, chunk_of(0), g, n, kw0);
   }
-  // q in base-2 logit units: head hg*16 + n, channels 32g .. 32g+31 (0 for padded heads)
+  // q in base-2 logit units: head (row) hg*16 + n, channels 32g .. 32g+31 (0 for padded columns)
+  const uint32_t nrows = SESS ? a.nsess * gq : gq;
   float qv[32];
   float qmax = 0.f;
   {
     const uint32_t h = hg * NH + n;
-    const float s = h < gq ? a.scale2 : 0.f;
-    const float* qp = a.query + ((uint64_t)b * a.qh + kvh * gq + min(h, gq - 1)) * D + 32 * g;
+    const float s = h < nrows ? a.scale2 : 0.f;
+    const uint32_t r = min(h, nrows - 1), head = SESS ? r % gq : r;
+    const float* qp = a.query + ((uint64_t)b * a.qh + kvh * gq + head) * D + 32 * g +
+                      (SESS ? r / gq * a.q_sess_stride : 0);
 #pragma unroll
     for (int r = 0; r < 32; r += 4) {
       const float4 v = *reinterpret_cast<const float4*>(qp + r);
@@ -2393,7 +2417,12 @@ __device__ __forceinline__ void wide16_split(const AttnArgs& a, uint32_t unit, u
 #pragma unroll
     for (int r = 0; r < 32; ++r) qmax = fmaxf(qmax, fabsf(qv[r]));
   }
-  qmax = warp_max(qmax);
+  if constexpr (SESS) {  // the row's four lanes
+    qmax = fmaxf(qmax, __shfl_xor(qmax, 16));
+    qmax = fmaxf(qmax, __shfl_xor(qmax, 32));
+  } else {
+    qmax = warp_max(qmax);
+  }
   float kmax, vmax_all;  // the unit's largest key and value scales
   unit_scale_max(a.c, unit, kmax, vmax_all);
   const int ek = std::min(60, std::max(-100, 15 - __builtin_amdgcn_frexp_expf(qmax * kmax)));
@@ -2407,6 +2436,10 @@ __device__ __forceinline__ void wide16_split(const AttnArgs& a, uint32_t unit, u
   {
     auto step = [&](int k, const WideKeyWords<BITS>& cur, WideKeyWords<BITS>& next) {
       if constexpr (kRaise) __builtin_amdgcn_s_setprio(1);
+      if constexpr (SESS) {
+        centre_pairs(kp0, code_mid(BITS));
+        centre_pairs(kp1, code_mid(BITS));
+      }
       wide_stage(wl, ROW, k, lane, kp0, kp1);
       const int32_t kn = chunk_of(std::min(k + 1, nch - 1));
       wide_load_key_params(a, unit, kn, lane, kp0, kp1);
@@ -2436,7 +2469,8 @@ __device__ __forceinline__ void wide16_split(const AttnArgs& a, uint32_t unit, u
         }
 #pragma unroll
         for (int m2 = 0; m2 < 4; m2 += 2) {
-          const h8 A0 = wide_key_codes<BITS>(cur, m2, kt), A1 = wide_key_codes<BITS>(cur, m2 + 1, kt);
+          h8 A0 = wide_key_codes<BITS>(cur, m2, kt), A1 = wide_key_codes<BITS>(cur, m2 + 1, kt);
+          if constexpr (SESS) A0 = centred<BITS>(A0), A1 = centred<BITS>(A1);
           acc[m2] = mfma_wide(A0, bhi[m2 / 2], acc[m2]);
           acc[m2 + 1] = mfma_wide(A1, bhi[m2 / 2], acc[m2 + 1]);
           acc[m2] = mfma_wide(A0, blo[m2 / 2], acc[m2]);
@@ -2499,6 +2533,10 @@ __device__ __forceinline__ void wide16_split(const AttnArgs& a, uint32_t unit, u
 #pragma unroll
         for (int r = 0; r < 4; ++r) lg[r] = lp[r];
       }
+      if constexpr (SESS) {
+        centre_pairs(vp0, code_mid(BITS));
+        centre_pairs(vp1, code_mid(BITS));
+      }
       wide_stage(wl, ROW, k, lane, vp0, vp1);
       const int32_t kn = chunk_of(std::min(k + 1, nch - 1));
       wide_load_value_params(a, unit, kn, lane, vp0, vp1);
@@ -2532,7 +2570,8 @@ __device__ __forceinline__ void wide16_split(const AttnArgs& a, uint32_t unit, u
           }
           h8 bhi, blo;
           wide_split8(p, bhi, blo);
-          const h8 A0 = wide_value_codes<BITS>(cur, 2 * cg, kt), A1 = wide_value_codes<BITS>(cur, 2 * cg + 1, kt);
+          h8 A0 = wide_value_codes<BITS>(cur, 2 * cg, kt), A1 = wide_value_codes<BITS>(cur, 2 * cg + 1, kt);
+          if constexpr (SESS) A0 = centred<BITS>(A0), A1 = centred<BITS>(A1);
           vacc[2 * cg] = mfma_wide(A0, bhi, vacc[2 * cg]);
           vacc[2 * cg + 1] = mfma_wide(A1, bhi, vacc[2 * cg + 1]);
           vacc[2 * cg] = mfma_wide(A0, blo, vacc[2 * cg]);
@@ -2570,8 +2609,8 @@ __device__ __forceinline__ void wide16_split(const AttnArgs& a, uint32_t unit, u
     cw[n * (D + 2) + D + 1] = nch > 0 ? lsum * vinv : 0.f;
   }
   __syncthreads();
-  const uint32_t hrows = std::min<uint32_t>(NH, gq - hg * NH);
-  float* part = a.ws + (((uint64_t)unit * a.nsplit_total + split) * gq + hg * NH) * (D + 2);
+  const uint32_t hrows = std::min<uint32_t>(NH, nrows - hg * NH);
+  float* part = a.ws + (((uint64_t)unit * a.nsplit_total + split) * gq + (SESS ? 0 : hg * NH)) * (D + 2);
   for (uint32_t idx = threadIdx.x; idx < hrows * (D + 2); idx += blockDim.x) {
     const uint32_t h = idx / (D + 2), d = idx % (D + 2);
     float M = -INFINITY;
@@ -2588,7 +2627,12 @@ __device__ __forceinline__ void wide16_split(const AttnArgs& a, uint32_t unit, u
         v += (d == D + 1 ? c[D + 1] : c[d]) * f;
       }
     }
-    part[h * (D + 2) + d] = v;
+    if constexpr (SESS) {
+      const uint32_t row = hg * NH + h;
+      part[row / gq * a.ws_sess_stride + row % gq * (D + 2) + d] = v;
+    } else {
+      part[h * (D + 2) + d] = v;
+    }
   }
 }
 
@@ -2605,7 +2649,7 @@ __global__ void __launch_bounds__(kThreads, kWide16Blocks) k_attn_wide16(AttnArg
     return;
   }
   const uint32_t blk = blockIdx.x - nwin, vu = blk / a.nsplit_fast;
-  wide16_split<BITS>(a, vu / a.hgroups_fast, blk % a.nsplit_fast, vu % a.hgroups_fast, lds);
+  wide16_split<BITS, false>(a, vu / a.hgroups_fast, blk % a.nsplit_fast, vu % a.hgroups_fast, lds);
 }
 
 // Arguments of session s of a batched call: its queries, partials and suffix.
@@ -2624,15 +2668,16 @@ __device__ __forceinline__ AttnArgs session_args(const AttnArgs& a, const Sessio
   return as;
 }
 
-// Packed chunks per wave in a batched-sessions launch: a workgroup's chunks (4*kSessCpw*8 KB at
-// 2-bit) are re-read for every session, so they are kept few enough to stay cache resident.
-constexpr int kSessCpw = 4;
-
-// Batched sessions over one prefix: workgroups [0, nsess*units*nsplit_win) take one window /
-// suffix chunk of one session; the rest one packed-chunk split of a unit, for every session
-// in turn (the split's chunks are re-read from L2, not HBM, after the first session).
+// Batched sessions over one prefix, fewer than kSharedMinRows rows (session, head): the window / suffix
+// chunks of every session first (one workgroup each, the 4x4x4 MIXED path), then the prefix's packed
+// chunks for groups of 16 rows on the sixteen-head 16x16x32 path, a chunk's codes exact and its
+// scales folded into the rows, so that no chunk is dequantized. Each group of 16 reads the chunks
+// again (from L2 or the Infinity Cache) and costs the same; the GEMM form dequantizes a chunk once
+// for up to 256 rows but costs nearly as much for 16. 8 units x 10007 tokens, 10 rows at 8 bits:
+// 67 -> 20 us (one pass of the 4x4x4 path per session before); 65536 tokens, 16 rows at 2 bits:
+// 165 -> 34 us (GEMM form before).
 template <int BITS, int NRS>
-__global__ void __launch_bounds__(kThreads, BITS == 2 && NRS == 1 ? 3 : 2) k_attn_sessions(AttnArgs a, SessionTable t) {
+__global__ void __launch_bounds__(kThreads, kWide16Blocks) k_attn_sessions(AttnArgs a, SessionTable t) {
   extern __shared__ float lds[];
   const uint32_t per_sess = a.units * a.nsplit_win;
   const uint32_t nwin = a.nsess * per_sess;
@@ -2640,17 +2685,10 @@ __global__ void __launch_bounds__(kThreads, BITS == 2 && NRS == 1 ? 3 : 2) k_att
     const uint32_t s = blockIdx.x / per_sess, r = blockIdx.x % per_sess;
     const AttnArgs as = session_args(a, t, s);
     mfma_split<BITS, NRS, 1, true, 128>(as, r / a.nsplit_win, r % a.nsplit_win, 0, lds);
-  } else {
-    const uint32_t blk = blockIdx.x - nwin;
-    const uint32_t unit = blk / a.nsplit_fast, split = blk % a.nsplit_fast;
-    for (uint32_t s = 0; s < a.nsess; ++s) {
-      AttnArgs as = a;
-      as.query = a.query + s * a.q_sess_stride;
-      as.ws = a.ws + s * a.ws_sess_stride;
-      mfma_split<BITS, NRS, kSessCpw, false, 128>(as, unit, split, 0, lds);
-      __syncthreads();  // the next session reuses the LDS
-    }
+    return;
   }
+  const uint32_t blk = blockIdx.x - nwin, vu = blk / a.nsplit_fast;
+  wide16_split<BITS, true>(a, vu / a.hgroups_fast, blk % a.nsplit_fast, vu % a.hgroups_fast, lds);
 }
 
 // Session suffixes of the shared-prefix form (fp32 rows, head_dim 128, GQA <= 8): one
@@ -4007,7 +4045,11 @@ AttnArgs make_session_args(const SessionsProblem& sp, uint32_t nsess, uint64_t m
   p.batch = sp.batch;
   p.scale = sp.scale;
   AttnArgs a = make_args(p, ws);
-  a.nsplit_fast = (a.chunk_end + 4 * kSessCpw - 1) / (4 * kSessCpw);
+  // packed splits: 16 rows each, at most kWide16Cpw chunks per wave, at least kFastGroups workgroups
+  a.hgroups_fast = (nsess * a.gq + kWide16Heads - 1) / kWide16Heads;
+  const uint32_t vu = a.units * a.hgroups_fast, most = (a.chunk_end + 3) / 4;
+  const uint32_t fewest = (a.chunk_end + 4 * kWide16Cpw - 1) / (4 * kWide16Cpw);
+  a.nsplit_fast = level_splits(std::min(most, std::max(fewest, (kFastGroups + vu - 1) / vu)), most, vu, a.chunk_end);
   a.nsplit_total = a.nsplit_fast + a.nsplit_win + a.nsplit_gen;
   a.nsess = nsess;
   a.q_sess_stride = (uint64_t)sp.batch * sp.qh * sp.cache.geo.D;
@@ -4032,9 +4074,12 @@ uint64_t longest_suffix(const SessionsProblem& sp, uint32_t first, uint32_t coun
   return m;
 }
 
-// Rows (sessions x GQA heads) from which one launch group takes the GEMM form: below it a
-// 32-row MFMA tile would be mostly padding and the per-session form does less work.
-constexpr uint32_t kSharedMinRows = 16;
+// Rows (sessions x GQA heads) from which one launch group takes the GEMM form. Below, groups of 16
+// rows on the 16x16x32 path: each costs a pass over the chunks, where the GEMM form dequantizes
+// them once but then costs nearly the same for 16 rows as for 128. Step times at 8 units, 2 bits:
+// 16 rows x 65536 tokens 35.3 us (GEMM form 165), 80 rows x 10007 40.7 (53.6), 128 rows x 30000
+// 102 (98), 256 rows x 65536 380 (221).
+constexpr uint32_t kSharedMinRows = 97;
 // Workgroups the GEMM form aims for (one per CU: 148 KB of LDS each).
 constexpr uint32_t kSharedTargetGroups = 256;
 
@@ -4072,11 +4117,12 @@ struct GroupBytes {
 template <int BITS, int NRS>
 hipError_t launch_sessions(const AttnArgs& a, const SessionTable& t, const GroupBytes& by,
                            hipStream_t stream) {
-  constexpr int NH = 4 * NRS;
-  const size_t logits = (size_t)4 * NH * ((a.nsplit_fast > 0 ? kSessCpw : 1) * 64 + kRowPad);
-  const size_t combine = (size_t)4 * NH * (128 + 2);
+  const size_t logits = (size_t)4 * kWide16Heads * ((a.nsplit_fast > 0 ? kWide16Cpw : 1) * 64 + kRowPad);
+  const size_t combine = (size_t)4 * kWide16Heads * (128 + 2);
   const size_t lds = std::max(logits, combine) * sizeof(float);
-  const uint32_t grid = a.nsess * a.units * a.nsplit_win + a.units * a.nsplit_fast;
+  const hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(&k_attn_sessions<BITS, NRS>), lds);
+  if (e != hipSuccess) return e;
+  const uint32_t grid = a.nsess * a.units * a.nsplit_win + a.units * a.hgroups_fast * a.nsplit_fast;
   TimedLaunch timed(KIVI_KERNEL_ATTN_SESSIONS, stream, by.prefix + by.suffixes + by.queries);
   k_attn_sessions<BITS, NRS><<<grid, kThreads, lds, stream>>>(a, t);
   return hipGetLastError();
