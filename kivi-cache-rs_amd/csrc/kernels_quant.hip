@@ -74,18 +74,20 @@ __device__ __forceinline__ uint32_t dpp_u(uint32_t v) {
 
 // min and max over aligned groups of L lanes (L a power of two, 1 <= L <= 64; wave-uniform),
 // as compare-and-select (src/quant.rs:356 f32::min / max on finite values).
+// SKIP: a NaN operand is passed over (minNum / maxNum), as the general kernels pass it over.
+template <bool SKIP = false>
 __device__ __forceinline__ void minmax_with(float& mn, float& mx, float omn, float omx) {
-  mn = omn < mn ? omn : mn;
-  mx = omx > mx ? omx : mx;
+  mn = SKIP ? fminf(mn, omn) : omn < mn ? omn : mn;
+  mx = SKIP ? fmaxf(mx, omx) : omx > mx ? omx : mx;
 }
-template <uint32_t L>
+template <uint32_t L, bool SKIP = false>
 __device__ __forceinline__ void group_minmax(float& mn, float& mx) {
-  if constexpr (L >= 2) minmax_with(mn, mx, dpp_f<kDppXor1>(mn), dpp_f<kDppXor1>(mx));
-  if constexpr (L >= 4) minmax_with(mn, mx, dpp_f<kDppXor2>(mn), dpp_f<kDppXor2>(mx));
-  if constexpr (L >= 8) minmax_with(mn, mx, dpp_f<kDppHalfMirror>(mn), dpp_f<kDppHalfMirror>(mx));
-  if constexpr (L >= 16) minmax_with(mn, mx, dpp_f<kDppMirror>(mn), dpp_f<kDppMirror>(mx));
-  if constexpr (L >= 32) minmax_with(mn, mx, __shfl_xor(mn, 16), __shfl_xor(mx, 16));
-  if constexpr (L >= 64) minmax_with(mn, mx, __shfl_xor(mn, 32), __shfl_xor(mx, 32));
+  if constexpr (L >= 2) minmax_with<SKIP>(mn, mx, dpp_f<kDppXor1>(mn), dpp_f<kDppXor1>(mx));
+  if constexpr (L >= 4) minmax_with<SKIP>(mn, mx, dpp_f<kDppXor2>(mn), dpp_f<kDppXor2>(mx));
+  if constexpr (L >= 8) minmax_with<SKIP>(mn, mx, dpp_f<kDppHalfMirror>(mn), dpp_f<kDppHalfMirror>(mx));
+  if constexpr (L >= 16) minmax_with<SKIP>(mn, mx, dpp_f<kDppMirror>(mn), dpp_f<kDppMirror>(mx));
+  if constexpr (L >= 32) minmax_with<SKIP>(mn, mx, __shfl_xor(mn, 16), __shfl_xor(mx, 16));
+  if constexpr (L >= 64) minmax_with<SKIP>(mn, mx, __shfl_xor(mn, 32), __shfl_xor(mx, 32));
 }
 
 // v as held by lane p of the lane's 16-lane row (DPP row_newbcast).
@@ -104,7 +106,7 @@ __device__ __forceinline__ float row_bcast(float v, int p) {
 // One exchange step of row_minmax16: of its n token pairs (lo[j], hi[j]) a lane keeps the lo
 // half when `upper` is false and the hi half otherwise, sends the other half to its DPP partner
 // (whose `upper` is the opposite) and combines what it keeps with what it receives.
-template <int CTRL, int N>
+template <int CTRL, int N, bool SKIP>
 __device__ __forceinline__ void minmax_step(const float* mn, const float* mx, bool upper, float* omn,
                                             float* omx) {
 #pragma unroll
@@ -112,8 +114,9 @@ __device__ __forceinline__ void minmax_step(const float* mn, const float* mx, bo
     const float kmn = upper ? mn[N + j] : mn[j], smn = upper ? mn[j] : mn[N + j];
     const float kmx = upper ? mx[N + j] : mx[j], smx = upper ? mx[j] : mx[N + j];
     const float rmn = dpp_f<CTRL>(smn), rmx = dpp_f<CTRL>(smx);
-    omn[j] = rmn < kmn ? rmn : kmn;
-    omx[j] = rmx > kmx ? rmx : kmx;
+    omn[j] = kmn;
+    omx[j] = kmx;
+    minmax_with<SKIP>(omn[j], omx[j], rmn, rmx);
   }
 }
 
@@ -122,14 +125,15 @@ __device__ __forceinline__ void minmax_step(const float* mn, const float* mx, bo
 // (mirror), r^7 (half mirror), r^2 and r^1 each differ in the bit that decides which half of
 // the remaining tokens a lane keeps, and the four steps together reach all 16 lanes. 15 lane
 // exchanges per quantity instead of 64 for a reduction of every token.
+template <bool SKIP = false>
 __device__ __forceinline__ void row_minmax16(const float (&mn)[16], const float (&mx)[16], float& mn_r,
                                              float& mx_r) {
   const uint32_t r = threadIdx.x % 16;
   float a[8], b[8], c[4], d[4], e[2], f[2];
-  minmax_step<kDppMirror, 8>(mn, mx, (r & 8) != 0, a, b);
-  minmax_step<kDppHalfMirror, 4>(a, b, (r & 4) != 0, c, d);
-  minmax_step<kDppXor2, 2>(c, d, (r & 2) != 0, e, f);
-  minmax_step<kDppXor1, 1>(e, f, (r & 1) != 0, &mn_r, &mx_r);
+  minmax_step<kDppMirror, 8, SKIP>(mn, mx, (r & 8) != 0, a, b);
+  minmax_step<kDppHalfMirror, 4, SKIP>(a, b, (r & 4) != 0, c, d);
+  minmax_step<kDppXor2, 2, SKIP>(c, d, (r & 2) != 0, e, f);
+  minmax_step<kDppXor1, 1, SKIP>(e, f, (r & 1) != 0, &mn_r, &mx_r);
 }
 
 // OR over aligned groups of L lanes (L a power of two <= 16).
@@ -686,6 +690,237 @@ __global__ void __launch_bounds__(kThreads)
   raise_max(max_slot(c, unit, blockIdx.x) + kMaxValueScale, smax, amax);
 }
 
+// ------------------------------------------------------------------ pair forms (native layout)
+// The same for any even head_dim whose groups are 16, 32, 64 or 128 wide: a lane holds two adjacent
+// channels (a float2 per row) and the workgroup's lanes run over (run of tokens, channel pair) items,
+// pairs fastest. head_dim is a multiple of G and of the ppw channels of a word, so the lanes of a
+// word and of a channel group stay together, aligned, inside a wave, and the lane exchanges of
+// the wave forms carry over. HBM-bound like them; what they replace (k_quant_keys, k_quant_values)
+// stages rows in LDS and runs a thread per channel or per (token, group), with a byte per code:
+// 96 units x 5003 tokens x 96 channels at 4 bits, keys 136 -> 39 us, values 143 -> 68 us.
+
+// Item i of `half` channel pairs per run: i = base + thread, with the division kept to 32 bits.
+struct PairItem {
+  uint64_t run;
+  uint32_t d;  // first channel
+};
+__device__ __forceinline__ PairItem pair_item(uint64_t base, uint32_t thread, uint32_t half) {
+  const uint32_t r = static_cast<uint32_t>(base % half) + thread;  // uniform 64-bit division
+  return PairItem{base / half + r / half, 2 * (r % half)};
+}
+
+// Per-channel min and max of a lane's two channels over GG rows of D floats at `rows`, kept in x
+// when they fit (GG <= 64; 128 rows are read again for their codes). A zero minimum takes its
+// first zero's sign.
+template <int GG>
+struct PairRows {
+  static constexpr int KEEP = GG <= 64 ? GG : 32;
+  float x[KEEP][2];
+  float2 mn, mx;
+  __device__ __forceinline__ void load(const float* rows, uint32_t D, int t0) {
+#pragma unroll
+    for (int t = 0; t < KEEP; ++t) {
+      const f2v v = __builtin_nontemporal_load(reinterpret_cast<const f2v*>(rows + (uint64_t)(t0 + t) * D));
+      x[t][0] = v.x;
+      x[t][1] = v.y;
+    }
+  }
+  __device__ __forceinline__ void minmax(const float* rows, uint32_t D) {
+    mn = make_float2(INFINITY, INFINITY);
+    mx = make_float2(-INFINITY, -INFINITY);
+#pragma unroll 1
+    for (int t0 = 0; t0 < GG; t0 += KEEP) {
+      load(rows, D, t0);
+#pragma unroll
+      for (int t = 0; t < KEEP; ++t) {
+        mn.x = fminf(mn.x, x[t][0]);
+        mn.y = fminf(mn.y, x[t][1]);
+        mx.x = fmaxf(mx.x, x[t][0]);
+        mx.y = fmaxf(mx.y, x[t][1]);
+      }
+    }
+    if (__ballot(mn.x == 0.f || mn.y == 0.f)) {  // rare, and wave-uniform
+      if (mn.x == 0.f) mn.x = first_zero(rows, D, GG);
+      if (mn.y == 0.f) mn.y = first_zero(rows + 1, D, GG);
+    }
+  }
+};
+
+// Keys: workgroup (unit, span) takes items span*256 .. +255 of the unit's (group, channel pair)s.
+template <int BITS, int GG>
+__global__ void __launch_bounds__(kThreads)
+    k_quant_keys_pairs(CacheView c, RowSource src, uint64_t g0, uint32_t ngroups, uint32_t spans) {
+  constexpr uint32_t PPW = 32 / BITS, LPW = PPW / 2;  // lanes per code word
+  constexpr uint32_t kLevels = (1u << BITS) - 1u;
+  constexpr float levels = static_cast<float>(kLevels);
+  constexpr int KEEP = PairRows<GG>::KEEP;
+  const Geometry& geo = c.geo;
+  const uint32_t D = geo.D, half = D / 2, KW = D / PPW;
+  const uint32_t unit = blockIdx.x / spans;
+  const uint64_t base = (uint64_t)(blockIdx.x % spans) * kThreads, items = (uint64_t)ngroups * half;
+  // lanes past the last item (whole words of them) repeat the last word's lanes and write nothing
+  const bool live = base + threadIdx.x < items;
+  const uint32_t last = static_cast<uint32_t>(std::min<uint64_t>(items - base, kThreads)) - LPW;
+  const PairItem it = pair_item(base, live ? threadIdx.x : last + threadIdx.x % LPW, half);
+  const float* rows = src.base + unit * src.stride_unit + (src.offset + it.run * GG) * D + it.d;
+  PairRows<GG> r;
+  r.minmax(rows, D);
+  const float2 sc = make_float2(scale_of(r.mx.x - r.mn.x, levels), scale_of(r.mx.y - r.mn.y, levels));
+  const float2 inv = make_float2(quant_inv(sc.x), quant_inv(sc.y));
+  const uint32_t sh0 = code_shift(BITS, it.d % PPW), sh1 = code_shift(BITS, (it.d + 1) % PPW);
+  const uint32_t m = (it.d / 2) % LPW, j = it.d / PPW;
+  if (live)
+    *reinterpret_cast<float4*>(c.kparams + unit * geo.kparams_unit() + ((g0 + it.run) * D + it.d) * 2) =
+        make_float4(sc.x, r.mn.x, sc.y, r.mn.y);
+  uint32_t* words = c.kcodes + unit * geo.kcodes_unit() + (g0 + it.run) * GG * KW + j;
+#pragma unroll 1
+  for (int t0 = 0; t0 < GG; t0 += KEEP) {
+    if constexpr (GG > KEEP) r.load(rows, D, t0);
+    uint32_t keep[KEEP / LPW];
+#pragma unroll
+    for (int t = 0; t < KEEP; ++t) {
+      uint32_t part = quant_code_fast(r.x[t][0], r.mn.x, sc.x, inv.x, kLevels) << sh0 |
+                      quant_code_fast(r.x[t][1], r.mn.y, sc.y, inv.y, kLevels) << sh1;
+      part = group_or<LPW>(part);
+      if (t % LPW == 0 || m == t % LPW) keep[t / LPW] = part;
+    }
+    if (live) {
+#pragma unroll
+      for (int k = 0; k < KEEP / (int)LPW; ++k) words[(uint64_t)(t0 + k * LPW + m) * KW] = keep[k];
+    }
+  }
+  raise_max(max_slot(c, unit, blockIdx.x) + kMaxKeyScale, fmaxf(0.f, fmaxf(sc.x, sc.y)),
+            fmaxf(fmaxf(fabsf(r.mn.x), fabsf(r.mx.x)), fmaxf(fabsf(r.mn.y), fabsf(r.mx.y))));
+}
+
+// (scale, zero) of 16 tokens of a channel group held as pairs by the group's GG / 2 lanes:
+// sz[p] in every lane of the group, and the lane's share of them to store. Zero minima take the
+// group's first zero, scanned by `first(p)`.
+template <int GG, class First>
+__device__ __forceinline__ void pair_groups(const float (&x)[16][2], float levels, float (&scale)[16],
+                                            float (&zero)[16], float (&top)[16], First&& first) {
+  constexpr uint32_t L = GG / 2;
+  if constexpr (L == 16) {
+    // a channel group is a DPP row: row p's min and max end in lane p of the row
+    float pmn[16], pmx[16], mn, mx;
+#pragma unroll
+    for (int p = 0; p < 16; ++p) {
+      pmn[p] = fminf(fminf(INFINITY, x[p][0]), x[p][1]);
+      pmx[p] = fmaxf(fmaxf(-INFINITY, x[p][0]), x[p][1]);
+    }
+    row_minmax16<true>(pmn, pmx, mn, mx);
+    if (__ballot(mn == 0.f)) {  // rare, and wave-uniform
+      if (mn == 0.f) mn = first(threadIdx.x % 16);
+    }
+    const float sc = scale_of(mx - mn, levels);
+#pragma unroll
+    for (int p = 0; p < 16; ++p) {
+      scale[p] = row_bcast(sc, p);
+      zero[p] = row_bcast(mn, p);
+      top[p] = row_bcast(mx, p);
+    }
+  } else {
+#pragma unroll
+    for (int p = 0; p < 16; ++p) {
+      float mn = fminf(fminf(INFINITY, x[p][0]), x[p][1]), mx = fmaxf(fmaxf(-INFINITY, x[p][0]), x[p][1]);
+      group_minmax<L, true>(mn, mx);
+      if (__ballot(mn == 0.f)) {
+        if (mn == 0.f) mn = first(p);
+      }
+      scale[p] = scale_of(mx - mn, levels);
+      zero[p] = mn;
+      top[p] = mx;
+    }
+  }
+}
+
+// Values: workgroup (unit, 64-token block of this call); its items are the block's four runs of 16
+// tokens times the channel pairs, 256 at a time. The words meet in LDS for contiguous stores, as in
+// the wave form; words that already hold earlier tokens of the block are read and OR-ed.
+template <int BITS, int GG>
+__global__ void __launch_bounds__(kThreads)
+    k_quant_values_pairs(CacheView c, RowSource ring, uint32_t n_ring, RowSource in, uint64_t vq0,
+                         uint64_t n, uint64_t blk0, uint32_t nblk) {
+  constexpr uint32_t PPW = 32 / BITS, WPW = 16 / PPW, VW = kValueBlock / PPW, VWP = VW + 1;
+  constexpr uint32_t kLevels = (1u << BITS) - 1u;
+  constexpr float levels = static_cast<float>(kLevels);
+  extern __shared__ uint32_t words_lds[];  // [D][VWP]
+  const Geometry& geo = c.geo;
+  const uint32_t D = geo.D, R = geo.R, ncg = geo.ncg(), half = D / 2;
+  const uint32_t unit = blockIdx.x / nblk;
+  const uint64_t tb = blk0 + blockIdx.x % nblk, blk = tb * kValueBlock;
+  // the call's tokens in this block: [lo, hi) of the block's 64
+  const uint32_t lo = vq0 > blk ? static_cast<uint32_t>(vq0 - blk) : 0u;
+  const uint32_t hi = static_cast<uint32_t>(std::min<uint64_t>(vq0 + n - blk, kValueBlock));
+  const bool linear = blk + lo - vq0 >= n_ring && !in.ring;  // every row from the (linear) input
+  auto row_of = [&](uint32_t tt) -> const float* {           // tt in [lo, hi)
+    const uint64_t i = blk + tt - vq0;
+    if (linear) return in.base + unit * in.stride_unit + (in.offset + (i - n_ring)) * D;
+    return i < n_ring ? source_row(ring, unit, i, R, D) : source_row(in, unit, i - n_ring, R, D);
+  };
+  float2* params = reinterpret_cast<float2*>(c.vparams + unit * geo.vparams_unit()) + tb * ncg * kValueBlock;
+  float smax = 0.f, amax = 0.f;
+  for (uint32_t i0 = 0; i0 < 4 * half; i0 += kThreads) {
+    const bool live = i0 + threadIdx.x < 4 * half;
+    // lanes past the last item (whole channel groups of them) repeat the last group's lanes
+    const uint32_t i = live ? i0 + threadIdx.x : 4 * half - GG / 2 + threadIdx.x % (GG / 2);
+    const uint32_t run = i / half, d = 2 * (i % half), cg = d / GG;
+    auto clamped = [&](uint32_t p) { return std::min(std::max(16 * run + p, lo), hi - 1); };
+    float x[16][2];
+    if (linear) {
+      const float* row0 = row_of(lo);
+#pragma unroll
+      for (uint32_t p = 0; p < 16; ++p) {
+        const f2v v = __builtin_nontemporal_load(reinterpret_cast<const f2v*>(row0 + (clamped(p) - lo) * D + d));
+        x[p][0] = v.x;
+        x[p][1] = v.y;
+      }
+    } else {
+#pragma unroll
+      for (uint32_t p = 0; p < 16; ++p) {
+        const f2v v = __builtin_nontemporal_load(reinterpret_cast<const f2v*>(row_of(clamped(p)) + d));
+        x[p][0] = v.x;
+        x[p][1] = v.y;
+      }
+    }
+    float scale[16], zero[16], top[16];
+    pair_groups<GG>(x, levels, scale, zero, top,
+                    [&](uint32_t p) { return first_zero(row_of(clamped(p)) + cg * GG, 1, GG); });
+    uint32_t word[2][WPW];
+#pragma unroll
+    for (int k = 0; k < (int)WPW; ++k) word[0][k] = word[1][k] = 0;
+#pragma unroll
+    for (int p = 0; p < 16; ++p) {
+      const uint32_t tt = 16 * run + p;
+      const bool valid = live && tt >= lo && tt < hi;
+      const float inv = quant_inv(scale[p]);
+      if (valid) {
+        smax = fmaxf(smax, scale[p]);
+        amax = fmaxf(amax, fmaxf(fabsf(zero[p]), fabsf(top[p])));
+        if (d % GG == 0) params[cg * kValueBlock + tt] = make_float2(scale[p], zero[p]);
+      }
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        word[j][p / PPW] |= (valid ? quant_code_fast(x[p][j], zero[p], scale[p], inv, kLevels) : 0u) << code_shift(BITS, p % PPW);
+    }
+    if (live) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int k = 0; k < (int)WPW; ++k) words_lds[(d + j) * VWP + run * WPW + k] = word[j][k];
+    }
+  }
+  __syncthreads();
+  uint32_t* base = c.vcodes + unit * geo.vcodes_unit() + tb * D * VW;
+  for (uint32_t idx = threadIdx.x; idx < D * VW; idx += kThreads) {
+    const uint32_t d = idx / VW, w = idx % VW;
+    if ((w + 1) * PPW <= lo || w * PPW >= hi) continue;
+    const uint32_t v = words_lds[d * VWP + w];
+    base[idx] = w * PPW < lo ? (v | base[idx]) : v;
+  }
+  raise_max(max_slot(c, unit, blockIdx.x) + kMaxValueScale, smax, amax);
+}
+
 // ------------------------------------------------------------------ export to reference order
 
 // Swap mask of a block-transpose round: the low s-element half of every 2s-element run of a
@@ -1153,6 +1388,95 @@ __global__ void __launch_bounds__(kThreads)
   }
 }
 
+// The pair forms of the codec (see k_quant_keys_pairs): items over all units' groups (keys) or runs of
+// 16 rows (values). Keys: a lane's two channels are 2*ipc consecutive words. Values: the LPW lanes of
+// a word OR their parts, lane m keeps rows p = m (mod LPW).
+template <int BITS, int GG>
+__global__ void __launch_bounds__(kThreads)
+    k_codec_keys_pairs(const float* data, uint64_t groups, uint32_t D, uint32_t* codes, float* params) {
+  constexpr uint32_t PPW = 32 / BITS, IPC = GG / PPW, KEEP = PairRows<GG>::KEEP;
+  constexpr uint32_t kLevels = (1u << BITS) - 1u;
+  constexpr float levels = static_cast<float>(kLevels);
+  const uint32_t half = D / 2;
+  const uint64_t items = groups * half;
+  for (uint64_t base = blockIdx.x * (uint64_t)kThreads; base < items; base += (uint64_t)gridDim.x * kThreads) {
+    if (base + threadIdx.x >= items) break;
+    const PairItem it = pair_item(base, threadIdx.x, half);
+    const float* rows = data + it.run * GG * D + it.d;
+    PairRows<GG> r;
+    r.minmax(rows, D);
+    const float sc[2] = {scale_of(r.mx.x - r.mn.x, levels), scale_of(r.mx.y - r.mn.y, levels)};
+    const float zr[2] = {r.mn.x, r.mn.y}, inv[2] = {quant_inv(sc[0]), quant_inv(sc[1])};
+    *reinterpret_cast<float4*>(params + (it.run * D + it.d) * 2) = make_float4(sc[0], zr[0], sc[1], zr[1]);
+#pragma unroll 1
+    for (uint32_t t0 = 0; t0 < GG; t0 += KEEP) {
+      if constexpr (GG > KEEP) r.load(rows, D, t0);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        uint32_t w[KEEP / PPW];
+#pragma unroll
+        for (int k = 0; k < (int)(KEEP / PPW); ++k) {
+          w[k] = 0;
+#pragma unroll
+          for (int i = 0; i < (int)PPW; ++i)
+            w[k] |= quant_code_fast(r.x[k * PPW + i][j], zr[j], sc[j], inv[j], kLevels) << (BITS * i);
+        }
+        store_words<KEEP / PPW>(codes + (it.run * D + it.d + j) * IPC + t0 / PPW, w);
+      }
+    }
+  }
+}
+
+template <int BITS, int GG>
+__global__ void __launch_bounds__(kThreads)
+    k_codec_values_pairs(const float* data, uint64_t rows, uint32_t D, uint32_t* codes, float* params) {
+  constexpr uint32_t PPW = 32 / BITS, LPW = PPW / 2, NS = 16 / LPW;
+  constexpr uint32_t kLevels = (1u << BITS) - 1u;
+  constexpr float levels = static_cast<float>(kLevels);
+  const uint32_t half = D / 2, ncg = D / GG, KW = D / PPW;
+  const uint64_t items = (rows + 15) / 16 * half;
+  for (uint64_t base = blockIdx.x * (uint64_t)kThreads; base < items; base += (uint64_t)gridDim.x * kThreads) {
+    // lanes past the last item (whole channel groups of them) repeat the last group's lanes
+    const bool live = base + threadIdx.x < items;
+    const uint32_t last = static_cast<uint32_t>(std::min<uint64_t>(items - base, kThreads)) - GG / 2;
+    const PairItem it = pair_item(base, live ? threadIdx.x : last + threadIdx.x % (GG / 2), half);
+    const uint64_t r0 = it.run * 16;
+    const uint32_t nvalid = live ? static_cast<uint32_t>(std::min<uint64_t>(rows - r0, 16)) : 1u;
+    const float* src = data + r0 * D;
+    float x[16][2];
+#pragma unroll
+    for (uint32_t p = 0; p < 16; ++p) {
+      const f2v v = __builtin_nontemporal_load(reinterpret_cast<const f2v*>(src + (uint64_t)std::min(p, nvalid - 1) * D + it.d));
+      x[p][0] = v.x;
+      x[p][1] = v.y;
+    }
+    const uint32_t cg = it.d / GG;
+    float scale[16], zero[16], top[16];
+    pair_groups<GG>(x, levels, scale, zero, top, [&](uint32_t p) {
+      return first_zero(src + (uint64_t)std::min(p, nvalid - 1) * D + cg * GG, 1, GG);
+    });
+    const uint32_t m = (it.d / 2) % LPW, sh0 = BITS * (it.d % PPW);
+    float2* pp = reinterpret_cast<float2*>(params) + r0 * ncg + cg;
+    uint32_t keep[NS];
+#pragma unroll
+    for (int p = 0; p < 16; ++p) {
+      const float inv = quant_inv(scale[p]);
+      if (live && it.d % GG == 0 && (uint32_t)p < nvalid) pp[(uint64_t)p * ncg] = make_float2(scale[p], zero[p]);
+      uint32_t part = quant_code_fast(x[p][0], zero[p], scale[p], inv, kLevels) << sh0 |
+                      quant_code_fast(x[p][1], zero[p], scale[p], inv, kLevels) << (sh0 + BITS);
+      part = group_or<LPW>(part);
+      if (p % LPW == 0 || m == p % LPW) keep[p / LPW] = part;
+    }
+    if (live) {
+#pragma unroll
+      for (int k = 0; k < (int)NS; ++k) {
+        const uint32_t p = k * LPW + m;
+        if (p < nvalid) codes[(r0 + p) * KW + it.d / PPW] = keep[k];
+      }
+    }
+  }
+}
+
 // VW consecutive words (VW = 1, 2 or 4) at p, 4*VW-byte aligned, in one load.
 template <int VW>
 __device__ __forceinline__ void load_run(const uint32_t* p, uint32_t (&w)[VW]) {
@@ -1467,6 +1791,13 @@ bool values_wave_bits(uint32_t cpl, uint32_t G, unsigned grid, uint32_t spans, h
 #undef KIVI_VW
 }
 
+// Groups of the pair forms, and the rows they load as float2s.
+#define KIVI_PAIR_CASES(X)                                                                              \
+  X(2, 16) X(2, 32) X(2, 64) X(2, 128) X(4, 16) X(4, 32) X(4, 64) X(4, 128) X(8, 16) X(8, 32) X(8, 64) X(8, 128)
+bool pairs_aligned(const RowSource& r, uint32_t D) {
+  return D % 16 == 0 && reinterpret_cast<uintptr_t>(r.base) % 8 == 0 && r.stride_unit % 2 == 0;
+}
+
 hipError_t launch_quant_keys(const CacheView& c, RowSource src, uint64_t g0, uint32_t ngroups,
                              hipStream_t stream) {
   if (ngroups == 0) return hipSuccess;
@@ -1485,6 +1816,24 @@ hipError_t launch_quant_keys(const CacheView& c, RowSource src, uint64_t g0, uin
     const unsigned grid = c.geo.units * spans;
     if (keys_wave_dispatch(c.geo.bits, cpl, c.geo.G, grid, stream, c, src, g0, ngroups, spans))
       return hipGetLastError();
+  }
+  if (pairs_aligned(src, c.geo.D)) {
+    const uint64_t items = (uint64_t)ngroups * (c.geo.D / 2), spans = (items + kThreads - 1) / kThreads;
+    const uint64_t grid = spans * c.geo.units;
+    bool done = grid < (1ull << 31);
+    if (done) {
+#define KIVI_KP(B, GG)                                                                                        \
+  case B * 1000 + GG:                                                                                         \
+    k_quant_keys_pairs<B, GG><<<static_cast<unsigned>(grid), kThreads, 0, stream>>>(c, src, g0, ngroups,      \
+                                                                                   static_cast<uint32_t>(spans)); \
+    break;
+      switch (c.geo.bits * 1000 + c.geo.G) {
+        KIVI_PAIR_CASES(KIVI_KP)
+        default: done = false;
+      }
+#undef KIVI_KP
+    }
+    if (done) return hipGetLastError();
   }
   k_quant_keys<<<static_cast<unsigned>(blocks), kThreads, lds, stream>>>(c, src, g0, ngroups, staged ? 1u : 0u,
                                                                         rows_vec4(src, c.geo.D) ? 1u : 0u);
@@ -1527,6 +1876,21 @@ hipError_t launch_quant_values(const CacheView& c, RowSource ring, uint32_t n_ri
       case 8: done = values_wave_bits<8>(cpl, G, nb, spans, stream, c, ring, n_ring, in, vq0, n, blk0, nblk); break;
       default: break;
     }
+    if (done) return hipGetLastError();
+  }
+  const size_t pair_lds = (size_t)D * (c.geo.vwords_per_channel() + 1) * sizeof(uint32_t);
+  if (pairs_aligned(ring, D) && (n_in == 0 || pairs_aligned(in, D)) && pair_lds <= 65536 && blocks < (1ull << 31)) {
+    bool done = true;
+#define KIVI_VP(B, GG)                                                                                    \
+  case B * 1000 + GG:                                                                                     \
+    k_quant_values_pairs<B, GG><<<static_cast<unsigned>(blocks), kThreads, pair_lds, stream>>>(           \
+        c, ring, n_ring, in, vq0, n, blk0, nblk);                                                         \
+    break;
+    switch (c.geo.bits * 1000 + c.geo.G) {
+      KIVI_PAIR_CASES(KIVI_VP)
+      default: done = false;
+    }
+#undef KIVI_VP
     if (done) return hipGetLastError();
   }
   k_quant_values<<<static_cast<unsigned>(blocks), kThreads, lds, stream>>>(c, ring, n_ring, in, vq0, n,
@@ -1704,6 +2068,22 @@ hipError_t launch_quant_ref_keys(const float* data, uint32_t units, uint64_t tok
     }
     if (done) return hipGetLastError();
   }
+  // whole words of channels per lane group are not needed here (a lane packs its own words), but
+  // its float2s and float4 pairs want an even, aligned row
+  if (D % 2 == 0 && reinterpret_cast<uintptr_t>(data) % 8 == 0) {
+    const unsigned grid = grid_for(blocks * (D / 2));
+    bool done = true;
+#define KIVI_CP(B, GG)                                                                             \
+  case B * 1000 + GG:                                                                              \
+    k_codec_keys_pairs<B, GG><<<grid, kThreads, 0, stream>>>(data, blocks, D, codes, params);      \
+    break;
+    switch (bits * 1000 + G) {
+      KIVI_PAIR_CASES(KIVI_CP)
+      default: done = false;
+    }
+#undef KIVI_CP
+    if (done) return hipGetLastError();
+  }
   k_quant_ref_keys<<<static_cast<unsigned>(blocks), kThreads, (size_t)G * D, stream>>>(
       data, tokens, D, bits, G, codes, params);
   return hipGetLastError();
@@ -1727,6 +2107,20 @@ hipError_t launch_quant_ref_values(const float* data, uint32_t units, uint64_t t
       case 8: done = codec_values_bits<8>(cpl, G, grid, stream, data, rows, codes, params); break;
       default: break;
     }
+    if (done) return hipGetLastError();
+  }
+  if (D % 16 == 0 && reinterpret_cast<uintptr_t>(data) % 8 == 0) {
+    const unsigned grid = grid_for((rows + 15) / 16 * (D / 2));
+    bool done = true;
+#define KIVI_CP(B, GG)                                                                             \
+  case B * 1000 + GG:                                                                              \
+    k_codec_values_pairs<B, GG><<<grid, kThreads, 0, stream>>>(data, rows, D, codes, params);      \
+    break;
+    switch (bits * 1000 + G) {
+      KIVI_PAIR_CASES(KIVI_CP)
+      default: done = false;
+    }
+#undef KIVI_CP
     if (done) return hipGetLastError();
   }
   k_quant_ref_values<<<grid_for(work), kThreads, 0, stream>>>(data, units, tokens, D, bits, G, codes, params);
