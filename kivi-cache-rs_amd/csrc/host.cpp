@@ -237,32 +237,159 @@ struct DeviceScope {
   }
 };
 
+// Device memory the library's objects gave back, kept for the next ones: a request that makes and
+// frees a cache spent more on hipMalloc and hipFree (page mapping, 20-300 us each) than on its
+// kernels (16 x 8 units x 32768 tokens prefilled and exported: 1100 of 2370 us). Per device, at most
+// kPoolBytes in kPoolBlocks blocks; past that the oldest are freed at once, and all of a device's
+// are when an allocation there fails. A block is only given back while the device is idle (see
+// QuietDevice), as hipFree would have waited for, so whoever takes it next may use it on any
+// stream. Any thread may take and give.
+class DevicePool {
+ public:
+  static constexpr size_t kPoolBytes = (size_t)1 << 30;
+  static constexpr size_t kPoolBlocks = 256;
+  static DevicePool& get() {
+    static DevicePool* pool = new DevicePool;  // never destroyed: HIP may be gone by then
+    return *pool;
+  }
+  // A block of at least n bytes (*got: its size) on the current device; with `fresh` a new one.
+  hipError_t take(void** p, size_t n, bool fresh, int* device, size_t* got) {
+    hipError_t e = hipGetDevice(device);
+    if (e != hipSuccess) return e;
+    if (!fresh) {
+      std::lock_guard<std::mutex> lock(mu_);
+      size_t best = blocks_.size();
+      // the smallest that fits with at most an eighth (and a page) to spare
+      for (size_t i = 0; i < blocks_.size(); ++i) {
+        const Block& b = blocks_[i];
+        if (b.device == *device && b.bytes >= n && b.bytes - n <= n / 8 + 4096 &&
+            (best == blocks_.size() || b.bytes < blocks_[best].bytes))
+          best = i;
+      }
+      if (best != blocks_.size()) {
+        *p = blocks_[best].p;
+        *got = blocks_[best].bytes;
+        blocks_.erase(blocks_.begin() + best);
+        return hipSuccess;
+      }
+    }
+    *got = n;
+    e = hipMalloc(p, n);
+    if (e == hipErrorOutOfMemory && !fresh && trim(*device, 0, 0)) {
+      (void)hipGetLastError();
+      e = hipMalloc(p, n);
+    }
+    return e;
+  }
+  void give(void* p, size_t n, int device) {
+    try {
+      std::lock_guard<std::mutex> lock(mu_);
+      blocks_.push_back(Block{p, n, device});
+    } catch (...) {
+      (void)hipFree(p);
+      return;
+    }
+    (void)trim(device, kPoolBytes, kPoolBlocks);
+  }
+
+ private:
+  struct Block {
+    void* p;
+    size_t bytes;
+    int device;
+  };
+  std::mutex mu_;
+  std::vector<Block> blocks_;  // oldest first
+  // Frees a device's oldest blocks down to the limits; true when any was freed.
+  bool trim(int device, size_t bytes, size_t count) {
+    bool any = false;
+    for (;;) {
+      void* p = nullptr;
+      {
+        std::lock_guard<std::mutex> lock(mu_);
+        size_t held = 0, n = 0, oldest = blocks_.size();
+        for (size_t i = blocks_.size(); i-- > 0;) {
+          if (blocks_[i].device != device) continue;
+          held += blocks_[i].bytes;
+          ++n;
+          oldest = i;
+        }
+        if (oldest == blocks_.size() || (held <= bytes && n <= count)) return any;
+        p = blocks_[oldest].p;
+        blocks_.erase(blocks_.begin() + oldest);
+      }
+      (void)hipFree(p);
+      any = true;
+    }
+  }
+};
+
+// Waits for all work on the current device once and lets the buffers released in its scope (on
+// this thread) go back to the pool without waiting again.
+struct QuietDevice {
+  static thread_local int depth;
+  const int quiet = hipDeviceSynchronize() == hipSuccess ? 1 : 0;  // 0: refused, as under capture
+  QuietDevice() { depth += quiet; }
+  ~QuietDevice() { depth -= quiet; }
+  QuietDevice(const QuietDevice&) = delete;
+  QuietDevice& operator=(const QuietDevice&) = delete;
+};
+thread_local int QuietDevice::depth = 0;
+
 struct DevBuf {
   void* p = nullptr;
-  size_t bytes = 0;
+  size_t bytes = 0;   // asked for
+  size_t block = 0;   // held
+  int device = 0;
   DevBuf() = default;
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
   ~DevBuf() { release(); }
+  void swap(DevBuf& o) {
+    std::swap(p, o.p);
+    std::swap(bytes, o.bytes);
+    std::swap(block, o.block);
+    std::swap(device, o.device);
+  }
   void release() {
-    if (p != nullptr) (void)hipFree(p);
+    if (p != nullptr) {
+      bool idle = QuietDevice::depth > 0;
+      if (!idle) {
+        DeviceScope scope(device);
+        idle = hipDeviceSynchronize() == hipSuccess;  // as hipFree would
+      }
+      if (idle)
+        DevicePool::get().give(p, block, device);
+      else
+        (void)hipFree(p);
+    }
     p = nullptr;
-    bytes = 0;
+    bytes = block = 0;
   }
   template <class T>
   T* as() const {
     return static_cast<T*>(p);
   }
-  // Contents undefined: for arrays the next launch writes whole.
-  Status alloc(size_t n, const char* what) {
+  // Contents undefined: for arrays the next launch writes whole. While `s`, the stream of the call, is
+  // captured the pool is passed by, so hipMalloc takes or refuses the call by the capture's mode and
+  // never by what the pool holds.
+  Status alloc(size_t n, hipStream_t s, const char* what) {
     release();
     if (n == 0) return Status{};
-    HIP_TRY(hipMalloc(&p, n), what);
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    const bool captured = hipStreamIsCapturing(s, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone;
+    if (captured) (void)hipGetLastError();
+    const hipError_t e = DevicePool::get().take(&p, n, captured, &device, &block);
+    if (e != hipSuccess) {
+      p = nullptr;
+      block = 0;
+      return DevErr(e, what);
+    }
     bytes = n;
     return Status{};
   }
   Status alloc_zero(size_t n, hipStream_t s, const char* what) {
-    KIVI_TRY(alloc(n, what));
+    KIVI_TRY(alloc(n, s, what));
     if (n != 0) HIP_TRY(hipMemsetAsync(p, 0, n, s), what);
     return Status{};
   }
@@ -384,14 +511,17 @@ struct CacheCore {
                          geo.vparams_unit() * 4, geo.units, s), "grow value params");
       HIP_TRY(hipStreamSynchronize(s), "grow");
     }
-    std::swap(kcodes.p, nkc.p);
-    std::swap(kcodes.bytes, nkc.bytes);
-    std::swap(kparams.p, nkp.p);
-    std::swap(kparams.bytes, nkp.bytes);
-    std::swap(vcodes.p, nvc.p);
-    std::swap(vcodes.bytes, nvc.bytes);
-    std::swap(vparams.p, nvp.p);
-    std::swap(vparams.bytes, nvp.bytes);
+    kcodes.swap(nkc);
+    kparams.swap(nkp);
+    vcodes.swap(nvc);
+    vparams.swap(nvp);
+    if (geo.cap > 0) {
+      QuietDevice quiet;
+      nkc.release();
+      nkp.release();
+      nvc.release();
+      nvp.release();
+    }
     geo.cap = want;
     return Status{};
   }
@@ -605,13 +735,10 @@ struct AttnSync {
     return Status{};
   }
   // Workspace of at least `bytes`; growing waits for the previous call to finish with it.
-  Status reserve(size_t bytes) {
+  Status reserve(size_t bytes, hipStream_t s) {
     if (bytes <= workspace.bytes) return Status{};
     KIVI_TRY(drain());
-    workspace.release();
-    HIP_TRY(hipMalloc(&workspace.p, bytes), "attention workspace");
-    workspace.bytes = bytes;
-    return Status{};
+    return workspace.alloc(bytes, s, "attention workspace");
   }
 };
 
@@ -655,7 +782,7 @@ Status attend(const CacheCore& core, AttnSync& sync, const float* suffix_k, cons
     return Status{};
   }
   std::lock_guard<std::mutex> lock(sync.mu);
-  KIVI_TRY(sync.reserve(attention_workspace_floats(p) * sizeof(float)));
+  KIVI_TRY(sync.reserve(attention_workspace_floats(p) * sizeof(float), s));
   KIVI_TRY(sync.before(s));
   HIP_TRY(launch_attention(p, sync.workspace.as<float>(), s), "attention");
   KIVI_TRY(sync.after(s));
@@ -1018,7 +1145,7 @@ Status decode_fused(kivi_cache* c, const float* key, size_t key_len, const float
   KIVI_TRY(core.ensure_capacity(p.st.vq, s));
   p.cache = core.view();  // capacity growth moves the arrays
   std::lock_guard<std::mutex> alock(c->attn.mu);
-  KIVI_TRY(c->attn.reserve(attention_workspace_floats(p) * sizeof(float)));
+  KIVI_TRY(c->attn.reserve(attention_workspace_floats(p) * sizeof(float), s));
   KIVI_TRY(c->attn.before(s));
   HIP_TRY(launch_attention(p, c->attn.workspace.as<float>(), s), "decode attention");
   KIVI_TRY(c->attn.after(s));
@@ -1085,10 +1212,8 @@ Status session_append(kivi_session* se, const float* keys, size_t keys_len, cons
       HIP_TRY(copy_units(nv.p, cap * D * 4, se->values.p, se->cap * D * 4, se->len * D * 4, units, s), "suffix grow");
     }
     HIP_TRY(hipStreamSynchronize(s), "suffix grow");
-    std::swap(se->keys.p, nk.p);
-    std::swap(se->keys.bytes, nk.bytes);
-    std::swap(se->values.p, nv.p);
-    std::swap(se->values.bytes, nv.bytes);
+    se->keys.swap(nk);
+    se->values.swap(nv);
     se->cap = cap;
   }
   const hipMemcpyKind kind = device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
@@ -1160,7 +1285,7 @@ Status batched_sessions(const kivi_session* const* sessions, size_t n, const flo
   if (ws_floats > 0 && gq * core.head_dim <= kMaxGqD) {
     AttnSync& sync_ = st->batch;
     std::lock_guard<std::mutex> lock(sync_.mu);
-    KIVI_TRY(sync_.reserve(ws_floats * sizeof(float)));
+    KIVI_TRY(sync_.reserve(ws_floats * sizeof(float), s));
     KIVI_TRY(sync_.before(s));
     HIP_TRY(launch_sessions_attention(sp, sync_.workspace.as<float>(), s), "sessions attention");
     KIVI_TRY(sync_.after(s));
@@ -1223,8 +1348,8 @@ Status quantize(const float* data, size_t data_len, size_t batch, size_t heads, 
                             : units * tokens * (head_dim / group_size) * 2;
   hipStream_t s = device ? stream : nullptr;
   // the quantize launch writes every word and every (scale, zero) pair
-  KIVI_TRY(q->codes.alloc(q->n_codes * 4, "quantized codes"));
-  KIVI_TRY(q->params.alloc(q->n_params * 4, "quantized params"));
+  KIVI_TRY(q->codes.alloc(q->n_codes * 4, s, "quantized codes"));
+  KIVI_TRY(q->params.alloc(q->n_params * 4, s, "quantized params"));
   const float* src = data;
   Scratch staging;
   if (!device) {
@@ -1347,10 +1472,8 @@ Status guard_push(kivi_guard* g, const float* keys, const float* values, size_t 
       HIP_TRY(copy_units(nv.p, cap * D * 4, g->tv.p, g->cap * D * 4, g->seq * D * 4,
                          static_cast<uint32_t>(units), s), "guard tape");
     }
-    std::swap(g->tk.p, nk.p);
-    std::swap(g->tk.bytes, nk.bytes);
-    std::swap(g->tv.p, nv.p);
-    std::swap(g->tv.bytes, nv.bytes);
+    g->tk.swap(nk);
+    g->tv.swap(nv);
     g->cap = cap;
   }
   HIP_TRY(hipMemcpy2DAsync(g->tk.as<float>() + g->seq * D, g->cap * D * 4, keys, n * D * 4, n * D * 4,
@@ -1473,6 +1596,7 @@ void kivi_cache_free(kivi_cache* cache) {
   (void)cache->settle();
   (void)hipStreamSynchronize(cache->core.stream);
   (void)cache->attn.drain();
+  QuietDevice quiet;
   delete cache;
 }
 
@@ -1680,7 +1804,7 @@ void kivi_prefix_release(kivi_prefix* prefix) {
   if (prefix == nullptr) return;
   if (prefix->refs.fetch_sub(1, std::memory_order_acq_rel) == 1) {
     DeviceScope scope(prefix->state->core.device);
-    (void)hipDeviceSynchronize();
+    QuietDevice quiet;
     delete prefix;
   }
 }
@@ -1735,7 +1859,7 @@ void kivi_session_free(kivi_session* s) {
   kivi_prefix* p = s->prefix;
   {
     DeviceScope scope(p->state->core.device);
-    (void)hipDeviceSynchronize();
+    QuietDevice quiet;
     delete s;
   }
   kivi_prefix_release(p);
@@ -1817,6 +1941,7 @@ void kivi_runtime_free(kivi_runtime* rt) {
   (void)rt->cache.settle();
   (void)hipStreamSynchronize(rt->cache.core.stream);
   (void)rt->cache.attn.drain();
+  QuietDevice quiet;
   delete rt;
 }
 
@@ -1884,6 +2009,10 @@ void kivi_guard_free(kivi_guard* guard) {
     DeviceScope scope(guard->cache->core.device);
     (void)hipStreamSynchronize(guard->cache->core.stream);
     (void)guard->dense.drain();
+    QuietDevice quiet;
+    guard->tk.release();
+    guard->tv.release();
+    guard->dense.workspace.release();
   }
   kivi_cache_free(guard->cache);
   delete guard;
@@ -2028,7 +2157,7 @@ kivi_status kivi_quantize_per_token_device(const float* data, size_t data_len, s
 void kivi_quantized_free(kivi_quantized* q) {
   if (q == nullptr) return;
   DeviceScope scope(q->device);
-  (void)hipDeviceSynchronize();
+  QuietDevice quiet;
   delete q;
 }
 
