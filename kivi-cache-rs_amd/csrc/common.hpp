@@ -231,6 +231,22 @@ hipError_t launch_dequant_cache(const CacheView& c, const SeqState& s, float* ke
 // raised once to the largest size asked for so far, from any thread.
 hipError_t raise_lds_limit(const void* kernel, size_t bytes);
 
+// One block per unit of an array to write: dst_n 16-byte words, the first min(src_n, dst_n) of them
+// from src (null: none), the rest zero. Pitches and counts in 16-byte words, pointers 16-byte
+// aligned.
+struct UnitArray {
+  void* dst;
+  const void* src;
+  uint64_t dst_pitch, src_pitch;
+  uint64_t dst_n, src_n;
+};
+constexpr uint32_t kMaxUnitArrays = 4;
+struct UnitArrays {
+  UnitArray a[kMaxUnitArrays];
+  uint32_t count;
+};
+hipError_t launch_fill_units(const UnitArrays& a, uint32_t units, hipStream_t stream);
+
 // Copy `units` blocks of `bytes` from src (pitch src_pitch) to dst (pitch dst_pitch).
 hipError_t copy_units(void* dst, size_t dst_pitch, const void* src, size_t src_pitch, size_t bytes,
                       uint32_t units, hipStream_t stream);

@@ -483,9 +483,16 @@ struct CacheCore {
   Status init(hipStream_t s) {
     set_geometry();
     const size_t rbytes = (size_t)geo.units * geo.R * geo.D * sizeof(float);
-    KIVI_TRY(kres.alloc_zero(rbytes, s, "key residual"));
-    KIVI_TRY(vring.alloc_zero(rbytes, s, "value window"));
-    KIVI_TRY(smax.alloc_zero((size_t)geo.units * kMaxUnitWords * sizeof(uint32_t), s, "scale maxima"));
+    KIVI_TRY(kres.alloc(rbytes, s, "key residual"));
+    KIVI_TRY(vring.alloc(rbytes, s, "value window"));
+    KIVI_TRY(smax.alloc((size_t)geo.units * kMaxUnitWords * sizeof(uint32_t), s, "scale maxima"));
+    UnitArrays fill{};
+    const uint64_t rows = geo.residual_unit() / 4, maxima = kMaxUnitWords / 4;
+    fill.count = 3;
+    fill.a[0] = UnitArray{kres.p, nullptr, rows, 0, rows, 0};
+    fill.a[1] = UnitArray{vring.p, nullptr, rows, 0, rows, 0};
+    fill.a[2] = UnitArray{smax.p, nullptr, maxima, 0, maxima, 0};
+    HIP_TRY(launch_fill_units(fill, geo.units, s), "cache init");
     return Status{};
   }
 
@@ -496,21 +503,21 @@ struct CacheCore {
     Geometry ng = geo;
     ng.cap = want;
     DevBuf nkc, nkp, nvc, nvp;
-    KIVI_TRY(nkc.alloc_zero(ng.kcodes_unit() * ng.units * 4, s, "key codes"));
-    KIVI_TRY(nkp.alloc_zero(ng.kparams_unit() * ng.units * 4, s, "key params"));
-    KIVI_TRY(nvc.alloc_zero(ng.vcodes_unit() * ng.units * 4, s, "value codes"));
-    KIVI_TRY(nvp.alloc_zero(ng.vparams_unit() * ng.units * 4, s, "value params"));
-    if (geo.cap > 0) {
-      HIP_TRY(copy_units(nkc.p, ng.kcodes_unit() * 4, kcodes.p, geo.kcodes_unit() * 4,
-                         geo.kcodes_unit() * 4, geo.units, s), "grow key codes");
-      HIP_TRY(copy_units(nkp.p, ng.kparams_unit() * 4, kparams.p, geo.kparams_unit() * 4,
-                         geo.kparams_unit() * 4, geo.units, s), "grow key params");
-      HIP_TRY(copy_units(nvc.p, ng.vcodes_unit() * 4, vcodes.p, geo.vcodes_unit() * 4,
-                         geo.vcodes_unit() * 4, geo.units, s), "grow value codes");
-      HIP_TRY(copy_units(nvp.p, ng.vparams_unit() * 4, vparams.p, geo.vparams_unit() * 4,
-                         geo.vparams_unit() * 4, geo.units, s), "grow value params");
-      HIP_TRY(hipStreamSynchronize(s), "grow");
-    }
+    KIVI_TRY(nkc.alloc(ng.kcodes_unit() * ng.units * 4, s, "key codes"));
+    KIVI_TRY(nkp.alloc(ng.kparams_unit() * ng.units * 4, s, "key params"));
+    KIVI_TRY(nvc.alloc(ng.vcodes_unit() * ng.units * 4, s, "value codes"));
+    KIVI_TRY(nvp.alloc(ng.vparams_unit() * ng.units * 4, s, "value params"));
+    // a unit's blocks are whole 16-byte words (cap is a multiple of 64 and of G)
+    UnitArrays fill{};
+    auto add = [&](const DevBuf& dst, uint64_t to, const DevBuf& src, uint64_t from) {
+      fill.a[fill.count++] = UnitArray{dst.p, src.p, to / 4, from / 4, to / 4, from / 4};
+    };
+    add(nkc, ng.kcodes_unit(), kcodes, geo.kcodes_unit());
+    add(nkp, ng.kparams_unit(), kparams, geo.kparams_unit());
+    add(nvc, ng.vcodes_unit(), vcodes, geo.vcodes_unit());
+    add(nvp, ng.vparams_unit(), vparams, geo.vparams_unit());
+    HIP_TRY(launch_fill_units(fill, geo.units, s), "grow arenas");
+    if (geo.cap > 0) HIP_TRY(hipStreamSynchronize(s), "grow");
     kcodes.swap(nkc);
     kparams.swap(nkp);
     vcodes.swap(nvc);
@@ -674,18 +681,19 @@ struct CacheCore {
       const uint64_t gran = granule();
       Geometry ng = geo;
       ng.cap = (used + gran - 1) / gran * gran;
-      KIVI_TRY(dst.kcodes.alloc_zero(ng.kcodes_unit() * ng.units * 4, s, "prefix key codes"));
-      KIVI_TRY(dst.kparams.alloc_zero(ng.kparams_unit() * ng.units * 4, s, "prefix key params"));
-      KIVI_TRY(dst.vcodes.alloc_zero(ng.vcodes_unit() * ng.units * 4, s, "prefix value codes"));
-      KIVI_TRY(dst.vparams.alloc_zero(ng.vparams_unit() * ng.units * 4, s, "prefix value params"));
-      HIP_TRY(copy_units(dst.kcodes.p, ng.kcodes_unit() * 4, kcodes.p, geo.kcodes_unit() * 4,
-                         ng.kcodes_unit() * 4, geo.units, s), "prefix copy");
-      HIP_TRY(copy_units(dst.kparams.p, ng.kparams_unit() * 4, kparams.p, geo.kparams_unit() * 4,
-                         ng.kparams_unit() * 4, geo.units, s), "prefix copy");
-      HIP_TRY(copy_units(dst.vcodes.p, ng.vcodes_unit() * 4, vcodes.p, geo.vcodes_unit() * 4,
-                         ng.vcodes_unit() * 4, geo.units, s), "prefix copy");
-      HIP_TRY(copy_units(dst.vparams.p, ng.vparams_unit() * 4, vparams.p, geo.vparams_unit() * 4,
-                         ng.vparams_unit() * 4, geo.units, s), "prefix copy");
+      KIVI_TRY(dst.kcodes.alloc(ng.kcodes_unit() * ng.units * 4, s, "prefix key codes"));
+      KIVI_TRY(dst.kparams.alloc(ng.kparams_unit() * ng.units * 4, s, "prefix key params"));
+      KIVI_TRY(dst.vcodes.alloc(ng.vcodes_unit() * ng.units * 4, s, "prefix value codes"));
+      KIVI_TRY(dst.vparams.alloc(ng.vparams_unit() * ng.units * 4, s, "prefix value params"));
+      UnitArrays fill{};
+      auto add = [&](const DevBuf& to, uint64_t n, const DevBuf& from, uint64_t pitch) {
+        fill.a[fill.count++] = UnitArray{to.p, from.p, n / 4, pitch / 4, n / 4, n / 4};
+      };
+      add(dst.kcodes, ng.kcodes_unit(), kcodes, geo.kcodes_unit());
+      add(dst.kparams, ng.kparams_unit(), kparams, geo.kparams_unit());
+      add(dst.vcodes, ng.vcodes_unit(), vcodes, geo.vcodes_unit());
+      add(dst.vparams, ng.vparams_unit(), vparams, geo.vparams_unit());
+      HIP_TRY(launch_fill_units(fill, geo.units, s), "prefix copy");
       dst.geo.cap = ng.cap;
     }
     return Status{};
@@ -1216,15 +1224,21 @@ Status session_append(kivi_session* se, const float* keys, size_t keys_len, cons
     se->values.swap(nv);
     se->cap = cap;
   }
-  const hipMemcpyKind kind = device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
   const size_t row = seq_len * D * 4;
+  if (device) {
+    HIP_TRY(copy_units(se->keys.as<float>() + se->len * D, se->cap * D * 4, keys, row, row,
+                       static_cast<uint32_t>(units), s), "suffix append");
+    HIP_TRY(copy_units(se->values.as<float>() + se->len * D, se->cap * D * 4, values, row, row,
+                       static_cast<uint32_t>(units), s), "suffix append");
+    se->len = new_len;
+    return Status{};
+  }
   HIP_TRY(hipMemcpy2DAsync(se->keys.as<float>() + se->len * D, se->cap * D * 4, keys, row, row,
-                           units, kind, s), "suffix append");
+                           units, hipMemcpyHostToDevice, s), "suffix append");
   HIP_TRY(hipMemcpy2DAsync(se->values.as<float>() + se->len * D, se->cap * D * 4, values, row, row,
-                           units, kind, s), "suffix append");
+                           units, hipMemcpyHostToDevice, s), "suffix append");
   se->len = new_len;
-  if (!device) return sync(s, "session append");
-  return Status{};
+  return sync(s, "session append");
 }
 
 Status batched_sessions(const kivi_session* const* sessions, size_t n, const float* queries,
