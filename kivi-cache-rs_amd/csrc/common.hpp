@@ -205,7 +205,7 @@ hipError_t launch_quant_values(const CacheView& c, RowSource ring, uint32_t n_ri
 // src/cache.rs:382-484, without a key flush): key row -> residual slot `kslot`; when `evict`,
 // the window row in slot `vslot` (stream token `vq`) is quantized into the packed values
 // first; the value row then goes to slot `vslot`. keys/values are [units][D]. Needs
-// D % 64 == 0, D <= 256 and G dividing 64 (returns hipErrorNotSupported otherwise).
+// D <= 1024 and G dividing 64 (returns hipErrorNotSupported otherwise).
 hipError_t launch_decode_append(const CacheView& c, const float* keys, const float* values,
                                 uint32_t kslot, uint32_t vslot, bool evict, uint64_t vq,
                                 hipStream_t stream);

@@ -231,16 +231,21 @@ __global__ void __launch_bounds__(kThreads) k_fill_units(UnitArrays a, uint32_t 
 }
 
 // One decode token (see launch_decode_append): one workgroup per unit, thread d owns channel
-// d. The value group min/max (src/quant.rs:349-375) reduces over the G lanes of a channel
+// d (head_dim rounded up to whole waves; the threads past it hold whole groups' lanes and write
+// nothing). The value group min/max (src/quant.rs:349-375) reduces over the G lanes of a channel
 // group by shuffles (G divides 64). Each channel's code word is read, OR-ed and written by
 // its own thread (the words of a 64-token block fill across appends; later tokens' bits are
-// still zero).
-__global__ void __launch_bounds__(256)
+// still zero). Latency-bound: one launch in place of a residual copy, an eviction and a window copy
+// (head_dims other than 64, 128, 192 and 256 took those: a decode step of 16 units at
+// head_dim 96, 2000 tokens, 32.3 -> 23.9 us).
+__global__ void __launch_bounds__(1024)
     k_decode_append(CacheView c, const float* keys, const float* values, uint32_t kslot,
                     uint32_t vslot, uint32_t evict, uint64_t vq) {
   const Geometry& geo = c.geo;
-  const uint32_t unit = blockIdx.x, d = threadIdx.x, D = geo.D, R = geo.R;
-  c.kres[((uint64_t)unit * R + kslot) * D + d] = keys[(uint64_t)unit * D + d];
+  const uint32_t unit = blockIdx.x, D = geo.D, R = geo.R;
+  const bool live = threadIdx.x < D;
+  const uint32_t d = live ? threadIdx.x : threadIdx.x & (geo.G - 1);  // any whole group
+  if (live) c.kres[((uint64_t)unit * R + kslot) * D + d] = keys[(uint64_t)unit * D + d];
   const float v = values[(uint64_t)unit * D + d];
   float* slot = c.vring + ((uint64_t)unit * R + vslot) * D + d;
   if (evict) {
@@ -259,21 +264,25 @@ __global__ void __launch_bounds__(256)
     const uint64_t tb = vq / kValueBlock;
     const uint32_t tt = static_cast<uint32_t>(vq % kValueBlock), ppw = geo.ppw(), vw = geo.vwords_per_channel();
     float2* params = reinterpret_cast<float2*>(c.vparams + unit * geo.vparams_unit());
-    if (d % G == 0) params[(tb * geo.ncg() + d / G) * kValueBlock + tt] = make_float2(scale, mn);
-    uint32_t* w = c.vcodes + unit * geo.vcodes_unit() + tb * D * vw + (uint64_t)d * vw + tt / ppw;
-    *w = (tt % ppw == 0 ? 0u : *w) | (code << code_shift(bits, tt % ppw));
-    // per-wave maxima of the scale and |x| (every lane holds its group's), one atomic each
-    float sm = scale, am = fmaxf(fabsf(mn), fabsf(mx));
+    if (live) {
+      if (d % G == 0) params[(tb * geo.ncg() + d / G) * kValueBlock + tt] = make_float2(scale, mn);
+      uint32_t* w = c.vcodes + unit * geo.vcodes_unit() + tb * D * vw + (uint64_t)d * vw + tt / ppw;
+      *w = (tt % ppw == 0 ? 0u : *w) | (code << code_shift(bits, tt % ppw));
+    }
+    // per-wave maxima of the scale and |x| (every lane holds a group's), one atomic each
+    float sm = fmaxf(0.f, scale), am = fmaxf(0.f, fmaxf(fabsf(mn), fabsf(mx)));  // a NaN raises nothing
     for (int o = 32; o > 0; o >>= 1) {
       sm = fmaxf(sm, __shfl_xor(sm, o));
       am = fmaxf(am, __shfl_xor(am, o));
     }
-    if (d % 64 == 0) {
+    if (threadIdx.x % 64 == 0) {
       atomicMax(max_slot(c, unit, 0) + kMaxValueScale, __float_as_uint(sm));
       atomicMax(max_slot(c, unit, 0) + kMaxValueAbs, __float_as_uint(am));
     }
+    // a thread past head_dim read another thread's slot: every read before the writes below
+    if (D % 64 != 0) __syncthreads();
   }
-  *slot = v;
+  if (live) *slot = v;
 }
 
 // Workgroup (unit, kind): kind 0 scans the key residual rows, kind 1 the value window rows.
@@ -1748,8 +1757,8 @@ hipError_t launch_decode_append(const CacheView& c, const float* keys, const flo
                                 uint32_t kslot, uint32_t vslot, bool evict, uint64_t vq,
                                 hipStream_t stream) {
   const Geometry& g = c.geo;
-  if (g.D % 64 != 0 || g.D > 256 || 64 % g.G != 0) return hipErrorNotSupported;
-  k_decode_append<<<g.units, g.D, 0, stream>>>(c, keys, values, kslot, vslot, evict ? 1u : 0u, vq);
+  if (g.D > 1024 || 64 % g.G != 0) return hipErrorNotSupported;
+  k_decode_append<<<g.units, (g.D + 63) / 64 * 64, 0, stream>>>(c, keys, values, kslot, vslot, evict ? 1u : 0u, vq);
   return hipGetLastError();
 }
 

@@ -67,3 +67,23 @@ def test_codec_matches_oracle(amd, oracle, case, off):
             assert same(got.codes(), want.codes()) and same(got.scale_zero(), want.scale_zero())
     finally:
         mem.free()
+
+
+@pytest.mark.parametrize("bits,group,dim", [
+    (8, 4, 4), (4, 8, 24), (2, 16, 16), (2, 16, 80), (4, 32, 96), (8, 16, 112), (4, 64, 320), (8, 16, 1024), (2, 64, 1024)])
+def test_single_token_appends_match_oracle(amd, oracle, bits, group, dim):
+    """One-launch appends (copy, eviction, window write) of head_dims that are no whole waves and of
+    the widest, across a window's fill, evictions and key flushes."""
+    rng = np.random.default_rng(6400 + dim)
+    cfg, units = KiviConfig(bits, group, group), 2
+    a, o = KiviCache(amd, cfg, 1, units, dim), KiviCache(oracle, cfg, 1, units, dim)
+    for step in range(3 * group + 70):
+        k, v = rows(rng, (units, 1, dim), 0), rows(rng, (units, 1, dim), 0)
+        k[np.isinf(k)] = 0
+        v[np.isinf(v)] = np.inf if step == 7 else 0
+        a.append(k, v, 1)
+        o.append(k, v, 1)
+    for got, want, name in zip(a.export_streams(), o.export_streams(), ("key codes", "key params", "value codes", "value params")):
+        assert same(got, want), name
+    for got, want in zip(a.dequantize(), o.dequantize()):
+        assert same(got[~np.isnan(want)], want[~np.isnan(want)])
