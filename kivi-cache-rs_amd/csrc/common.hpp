@@ -352,6 +352,8 @@ struct SessionsProblem {
   float scale;
 };
 size_t sessions_workspace_floats(const SessionsProblem& p);
+// Whether the call's sessions only share launches, each with the workgroups of its own attention.
+bool sessions_one_by_one(const SessionsProblem& p);
 hipError_t launch_sessions_attention(const SessionsProblem& p, float* workspace,
                                      hipStream_t stream);
 

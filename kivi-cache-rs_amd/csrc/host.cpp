@@ -1296,14 +1296,32 @@ Status batched_sessions(const kivi_session* const* sessions, size_t n, const flo
   sp.scale = scale;
   const size_t gq = num_q_heads / core.heads;
   const size_t ws_floats = n <= UINT32_MAX ? sessions_workspace_floats(sp) : 0;
-  if (ws_floats > 0 && gq * core.head_dim <= kMaxGqD) {
+  // Sessions that only share launches also run one by one, each in its own workspace: one alone, and
+  // where the launch's workspace cannot grow, under capture or without the memory.
+  const bool each = ws_floats > 0 && sessions_one_by_one(sp);
+  bool batched = ws_floats > 0 && gq * core.head_dim <= kMaxGqD && !(each && n == 1);
+  if (batched) {
     AttnSync& sync_ = st->batch;
     std::lock_guard<std::mutex> lock(sync_.mu);
-    KIVI_TRY(sync_.reserve(ws_floats * sizeof(float), s));
-    KIVI_TRY(sync_.before(s));
-    HIP_TRY(launch_sessions_attention(sp, sync_.workspace.as<float>(), s), "sessions attention");
-    KIVI_TRY(sync_.after(s));
-  } else {
+    const size_t bytes = ws_floats * sizeof(float);
+    if (each && bytes > sync_.workspace.bytes) {
+      hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+      HIP_TRY(hipStreamIsCapturing(s, &capture), "sessions capture status");
+      batched = capture == hipStreamCaptureStatusNone;
+    }
+    if (batched) {
+      const Status grown = sync_.reserve(bytes, s);
+      if (!grown.ok() && !each) return grown;
+      batched = grown.ok();
+      if (!batched) (void)hipGetLastError();
+    }
+    if (batched) {
+      KIVI_TRY(sync_.before(s));
+      HIP_TRY(launch_sessions_attention(sp, sync_.workspace.as<float>(), s), "sessions attention");
+      KIVI_TRY(sync_.after(s));
+    }
+  }
+  if (!batched) {
     for (size_t i = 0; i < n; ++i) {
       kivi_session* se = const_cast<kivi_session*>(sessions[i]);  // its workspace only
       KIVI_TRY(attend(core, se->attn, se->keys.as<float>(), se->values.as<float>(), se->len,

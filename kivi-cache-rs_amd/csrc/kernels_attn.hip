@@ -1324,6 +1324,11 @@ __device__ __forceinline__ void row_split(const AttnArgs& a, uint32_t unit, uint
   const uint32_t b = unit / a.heads, kvh = unit % a.heads;
   const uint32_t lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   const uint64_t t0 = a.t_begin + (uint64_t)split * S;
+  if (t0 >= a.total) {  // a batched session shorter than the longest: an empty partial
+    float* part = a.ws + (((uint64_t)unit * a.nsplit_total + a.nsplit_fast + a.nsplit_win + split) * gq + h0) * (D + 2);
+    for (uint32_t i = threadIdx.x; i < nh * (D + 2); i += kThreads) part[i] = i % (D + 2) == D ? -INFINITY : 0.f;
+    return;
+  }
   const uint32_t ntok = static_cast<uint32_t>(std::min<uint64_t>(S, a.total - t0));
   // the split's packed tokens [0, npk) / [0, npv), its tokens before the suffix [0, nseq), and the
   // first token's offset into the residual, the window and the suffix
@@ -1505,10 +1510,14 @@ __device__ __forceinline__ void row_split(const AttnArgs& a, uint32_t unit, uint
 }
 
 template <int BITS>
+__device__ __forceinline__ void rows_block(const AttnArgs& a, uint32_t block, float* lds) {
+  const uint32_t vu = block / a.nsplit_gen;
+  row_split<BITS>(a, vu / a.hgroups_rows, block % a.nsplit_gen, vu % a.hgroups_rows, lds);
+}
+template <int BITS>
 __global__ void __launch_bounds__(kThreads) k_attn_rows(AttnArgs a) {
   extern __shared__ float lds[];
-  const uint32_t vu = blockIdx.x / a.nsplit_gen;
-  row_split<BITS>(a, vu / a.hgroups_rows, blockIdx.x % a.nsplit_gen, vu % a.hgroups_rows, lds);
+  rows_block<BITS>(a, blockIdx.x, lds);
 }
 
 // ------------------------------------------------------------------ lane splits
@@ -1765,16 +1774,20 @@ __device__ __forceinline__ void lane_split(const AttnArgs& a, uint32_t unit, uin
 // The row splits over the tokens after the packed chunks come first in the grid (their latency
 // overlaps the packed ones), then the lane splits of every (unit, head group).
 template <int BITS, int HP>
-__global__ void __launch_bounds__(kThreads, HP == 4 || (HP == 2 && BITS == 8) ? 3 : 4) k_attn_lanes(AttnArgs a) {
-  extern __shared__ float lds[];
+__device__ __forceinline__ void lanes_block(const AttnArgs& a, uint32_t block, float* lds) {
   const uint32_t ngen = a.units * a.hgroups_rows * a.nsplit_gen;
-  if (blockIdx.x < ngen) {
-    const uint32_t vr = blockIdx.x / a.nsplit_gen;
-    row_split<BITS>(a, vr / a.hgroups_rows, blockIdx.x % a.nsplit_gen, vr % a.hgroups_rows, lds);
+  if (block < ngen) {
+    rows_block<BITS>(a, block, lds);
     return;
   }
-  const uint32_t blk = blockIdx.x - ngen, vu = blk / a.nsplit_fast;
+  const uint32_t blk = block - ngen, vu = blk / a.nsplit_fast;
   lane_split<BITS, HP>(a, vu / a.hgroups, blk % a.nsplit_fast, vu % a.hgroups, lds);
+}
+constexpr int lane_min_groups(int bits, int hp) { return hp == 4 || (hp == 2 && bits == 8) ? 3 : 4; }
+template <int BITS, int HP>
+__global__ void __launch_bounds__(kThreads, lane_min_groups(BITS, HP)) k_attn_lanes(AttnArgs a) {
+  extern __shared__ float lds[];
+  lanes_block<BITS, HP>(a, blockIdx.x, lds);
 }
 
 // ------------------------------------------------------------------ chunk launch
@@ -1820,6 +1833,29 @@ __global__ void __launch_bounds__(kThreads, SMALL ? 2 : fast_min_groups(BITS, NR
   } else {
     mfma_split<BITS, NRS, fast_cpw(BITS, NRS), false, D>(a, vu / a.hgroups, blk % a.nsplit_fast, vu % a.hgroups, lds);
   }
+}
+
+// Block `block` of the launch above for one session of a batched call. (k_attn_mfma keeps its own
+// copy: through this function the compiler scheduled <2,1,128> differently, 111.9 -> 115.6 us at 128
+// units x 32768 tokens.)
+template <int BITS, int NRS, int D>
+__device__ __forceinline__ void mfma_block(const AttnArgs& a, uint32_t block, float* lds) {
+  const uint32_t nwin = a.units * a.hgroups * a.nsplit_win;
+  const uint32_t ngen = a.units * a.hgroups_rows * a.nsplit_gen;
+  if constexpr (D == 128) {
+    if (block < nwin) {
+      const uint32_t vu = block / a.nsplit_win;
+      mfma_split<BITS, NRS, 1, true, D>(a, vu / a.hgroups, block % a.nsplit_win, vu % a.hgroups, lds);
+      return;
+    }
+  } else {
+    if (block < ngen) {
+      rows_block<BITS>(a, block, lds);
+      return;
+    }
+  }
+  const uint32_t blk = block - nwin - ngen, vu = blk / a.nsplit_fast;
+  mfma_split<BITS, NRS, fast_cpw(BITS, NRS), false, D>(a, vu / a.hgroups, blk % a.nsplit_fast, vu % a.hgroups, lds);
 }
 
 // ------------------------------------------------------------------ eight-head 16x16x32 path
@@ -2689,6 +2725,26 @@ __global__ void __launch_bounds__(kThreads, kWide16Blocks) k_attn_sessions(AttnA
   }
   const uint32_t blk = blockIdx.x - nwin, vu = blk / a.nsplit_fast;
   wide16_split<BITS, true>(a, vu / a.hgroups_fast, blk % a.nsplit_fast, vu % a.hgroups_fast, lds);
+}
+
+// Batched sessions at the other shapes: the single-session launch once per session, the sessions of
+// one block index side by side, so that a prefix chunk is read from HBM once. Bound as those launches
+// are; what it saves is two launches per session. 8 units: 8 sessions x 10007 tokens at head_dim 96
+// 175 -> 52 us; 20 x 20007 at head_dim 64 268 -> 52; 40 x 10007 at G = 64 535 -> 85.
+template <int BITS, int HP>
+__global__ void __launch_bounds__(kThreads, lane_min_groups(BITS, HP)) k_sessions_lanes(AttnArgs a, SessionTable t) {
+  extern __shared__ float lds[];
+  lanes_block<BITS, HP>(session_args(a, t, blockIdx.x % a.nsess), blockIdx.x / a.nsess, lds);
+}
+template <int BITS>
+__global__ void __launch_bounds__(kThreads) k_sessions_rows(AttnArgs a, SessionTable t) {
+  extern __shared__ float lds[];
+  rows_block<BITS>(session_args(a, t, blockIdx.x % a.nsess), blockIdx.x / a.nsess, lds);
+}
+template <int BITS, int NRS, int D>
+__global__ void __launch_bounds__(kThreads, fast_min_groups(BITS, NRS, D)) k_sessions_mfma(AttnArgs a, SessionTable t) {
+  extern __shared__ float lds[];
+  mfma_block<BITS, NRS, D>(session_args(a, t, blockIdx.x % a.nsess), blockIdx.x / a.nsess, lds);
 }
 
 // Session suffixes of the shared-prefix form (fp32 rows, head_dim 128, GQA <= 8): one
@@ -3708,7 +3764,11 @@ uint32_t level_splits(uint32_t base, uint32_t most, uint32_t units, uint32_t chu
 // tokens, or of 16 to 64 behind matrix-core chunks).
 enum class SplitPlan { kUsual, kFewest, kCounted };
 
-AttnArgs make_args_as(const AttnProblem& p, float* ws, SplitPlan plan) {
+// `sessions` problems like p share the launch: the f32 splits (lanes, rows) may be that much longer
+// (8 sessions x 10007 tokens at head_dim 96: 71 -> 52 us). The matrix-core splits keep to one
+// problem's: their error grows with the chunks a wave adds up (22 sessions x 30616 tokens at
+// head_dim 256, 4 bits: 1.8e-6 at 4 chunks per wave, 3.4e-6 at 8, for 235 against 232 us).
+AttnArgs make_args_as(const AttnProblem& p, float* ws, SplitPlan plan, uint32_t sessions) {
   AttnArgs a{};
   a.c = p.cache;
   a.st = p.st;
@@ -3750,7 +3810,7 @@ AttnArgs make_args_as(const AttnProblem& p, float* ws, SplitPlan plan) {
   if (lanes) {
     // up to 16 chunks per split, fewer (down to 4, which fill the value phase's 16-lane rows)
     // while the launch would have fewer than kLaneGroups workgroups; then evened out
-    const uint32_t vu = p.cache.geo.units * a.hgroups;
+    const uint32_t vu = p.cache.geo.units * a.hgroups * sessions;
     uint32_t cps = kLaneChunks;
     while (plan == SplitPlan::kUsual && cps > 4 && (uint64_t)vu * ((a.chunk_end + cps - 1) / cps) < kLaneGroups) cps /= 2;
     a.nsplit_fast = (a.chunk_end + cps - 1) / cps;
@@ -3779,7 +3839,7 @@ AttnArgs make_args_as(const AttnProblem& p, float* ws, SplitPlan plan) {
     while (a.S > 16 && (uint64_t)p.cache.geo.units * ((rest + a.S - 1) / a.S) < 1024) a.S >>= 1;
   }
   if (a.hgroups_rows != 0 && plan == SplitPlan::kUsual) {
-    const uint64_t rest = a.total - a.t_begin, vu = (uint64_t)p.cache.geo.units * a.hgroups_rows;
+    const uint64_t rest = a.total - a.t_begin, vu = (uint64_t)p.cache.geo.units * a.hgroups_rows * sessions;
     const uint32_t pass = std::min(64u, std::max(16u, row_pass(p.cache.geo.D)));
     auto splits = [&](uint32_t S) { return (rest + S - 1) / S; };
     a.S = pass;
@@ -3803,11 +3863,11 @@ uint64_t workspace_floats(const AttnArgs& a) {
 // The lane and row splits can take more partials than the counted plan; a call whose counted
 // partials fit the static workspace keeps to a plan that does too, so that the allocation-free
 // attention takes (and refuses) the same calls whatever splits pay.
-AttnArgs make_args(const AttnProblem& p, float* ws) {
-  const AttnArgs a = make_args_as(p, ws, SplitPlan::kUsual);
+AttnArgs make_args(const AttnProblem& p, float* ws, uint32_t sessions = 1) {
+  const AttnArgs a = make_args_as(p, ws, SplitPlan::kUsual, sessions);
   if (workspace_floats(a) <= kStaticWorkspaceFloats) return a;
   for (SplitPlan plan : {SplitPlan::kFewest, SplitPlan::kCounted}) {
-    const AttnArgs f = make_args_as(p, ws, plan);
+    const AttnArgs f = make_args_as(p, ws, plan, sessions);
     if (workspace_floats(f) <= kStaticWorkspaceFloats) return f;
   }
   return a;
@@ -3988,7 +4048,7 @@ size_t attention_workspace_floats(const AttnProblem& p) {
 }
 
 size_t attention_counted_floats(const AttnProblem& p) {
-  return workspace_floats(make_args_as(p, nullptr, SplitPlan::kCounted));
+  return workspace_floats(make_args_as(p, nullptr, SplitPlan::kCounted, 1));
 }
 
 hipError_t launch_attention(const AttnProblem& p, float* workspace, hipStream_t stream) {
@@ -4032,7 +4092,7 @@ namespace {
 
 // Arguments of one launch group as one problem over the prefix (the window range is sized
 // for the group's longest suffix; each session clips it to its own).
-AttnArgs make_session_args(const SessionsProblem& sp, uint32_t nsess, uint64_t max_suffix, float* ws) {
+AttnProblem session_problem(const SessionsProblem& sp, uint64_t max_suffix) {
   AttnProblem p{};
   p.cache = sp.cache;
   p.st = sp.st;
@@ -4044,28 +4104,40 @@ AttnArgs make_session_args(const SessionsProblem& sp, uint32_t nsess, uint64_t m
   p.heads = sp.heads;
   p.batch = sp.batch;
   p.scale = sp.scale;
-  AttnArgs a = make_args(p, ws);
+  return p;
+}
+
+void set_session_strides(const SessionsProblem& sp, uint32_t nsess, AttnArgs& a) {
+  a.nsess = nsess;
+  a.q_sess_stride = (uint64_t)sp.batch * sp.qh * sp.cache.geo.D;
+  a.ws_sess_stride = (uint64_t)sp.cache.geo.units * a.nsplit_total * a.gq * (sp.cache.geo.D + 2);
+}
+
+AttnArgs make_session_args(const SessionsProblem& sp, uint32_t nsess, uint64_t max_suffix, float* ws) {
+  AttnArgs a = make_args(session_problem(sp, max_suffix), ws);
   // packed splits: 16 rows each, at most kWide16Cpw chunks per wave, at least kFastGroups workgroups
   a.hgroups_fast = (nsess * a.gq + kWide16Heads - 1) / kWide16Heads;
   const uint32_t vu = a.units * a.hgroups_fast, most = (a.chunk_end + 3) / 4;
   const uint32_t fewest = (a.chunk_end + 4 * kWide16Cpw - 1) / (4 * kWide16Cpw);
   a.nsplit_fast = level_splits(std::min(most, std::max(fewest, (kFastGroups + vu - 1) / vu)), most, vu, a.chunk_end);
   a.nsplit_total = a.nsplit_fast + a.nsplit_win + a.nsplit_gen;
-  a.nsess = nsess;
-  a.q_sess_stride = (uint64_t)sp.batch * sp.qh * sp.cache.geo.D;
-  a.ws_sess_stride = (uint64_t)sp.cache.geo.units * a.nsplit_total * a.gq * (sp.cache.geo.D + 2);
+  set_session_strides(sp, nsess, a);
   return a;
 }
 
-bool sessions_supported(const SessionsProblem& sp) {
-  AttnProblem p{};
-  p.cache = sp.cache;
-  p.st = sp.st;
-  p.qh = sp.qh;
-  p.heads = sp.heads;
-  // the batched-sessions kernels take head_dim 128, G = 32 and GQA <= 8
-  return sp.n > 0 && fast_eligible(p) && sp.st.kq > 0 && sp.cache.geo.D == 128 && sp.cache.geo.G == 32 &&
-         sp.qh / sp.heads <= 8;
+// The kernels of a batched call: none (the sessions run one by one), the row forms of head_dim 128,
+// G = 32 and GQA <= 8 with packed keys (16 rows per pass, or the GEMM form), or the single-session
+// launch once per session. None at head_dims the row splits do not take, for an empty prefix (a
+// session without a suffix would have no token) and for the eight- and sixteen-head kernels' units
+// above GQA 8.
+enum class SessionForm { kNone, kRows, kEach };
+SessionForm session_form(const SessionsProblem& sp) {
+  const AttnProblem p = session_problem(sp, 0);
+  const Geometry& g = sp.cache.geo;
+  if (sp.n == 0 || sp.seq == 0 || g.D % 16 != 0) return SessionForm::kNone;
+  if (fast_eligible(p) && sp.st.kq > 0 && g.D == 128 && g.G == 32)
+    return sp.qh / sp.heads <= 8 ? SessionForm::kRows : SessionForm::kNone;
+  return SessionForm::kEach;
 }
 
 uint64_t longest_suffix(const SessionsProblem& sp, uint32_t first, uint32_t count) {
@@ -4113,6 +4185,58 @@ AttnArgs make_shared_args(const SessionsProblem& sp, uint32_t nsess, uint64_t ma
 struct GroupBytes {
   double prefix, suffixes, queries;
 };
+
+// The single-session launch of `a` once per session.
+hipError_t launch_each(const AttnArgs& a, const SessionTable& t, const GroupBytes& by, hipStream_t stream) {
+  const uint32_t D = a.c.geo.D, bits = a.c.geo.bits;
+  const uint32_t grid =
+      a.nsess * a.units * (a.hgroups * (a.nsplit_win + a.nsplit_fast) + a.hgroups_rows * a.nsplit_gen);
+  const size_t rows = a.nsplit_gen > 0 ? row_lds_floats(D, a.S) : 0;
+  TimedLaunch timed(KIVI_KERNEL_ATTN_SESSIONS, stream, by.prefix + by.suffixes + by.queries);
+  auto launch = [&](auto kernel, size_t floats) {
+    const size_t lds = std::max(floats, rows) * sizeof(float);
+    const hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(kernel), lds);
+    if (e != hipSuccess) return e;
+    kernel<<<grid, kThreads, lds, stream>>>(a, t);
+    return hipGetLastError();
+  };
+  if (a.lane_cps != 0) {
+    const uint32_t hp = lane_heads(a.gq);
+    switch (bits * 10 + hp) {
+      case 21: return launch(k_sessions_lanes<2, 1>, lane_lds_floats(1));
+      case 22: return launch(k_sessions_lanes<2, 2>, lane_lds_floats(2));
+      case 24: return launch(k_sessions_lanes<2, 4>, lane_lds_floats(4));
+      case 41: return launch(k_sessions_lanes<4, 1>, lane_lds_floats(1));
+      case 42: return launch(k_sessions_lanes<4, 2>, lane_lds_floats(2));
+      case 44: return launch(k_sessions_lanes<4, 4>, lane_lds_floats(4));
+      case 81: return launch(k_sessions_lanes<8, 1>, lane_lds_floats(1));
+      case 82: return launch(k_sessions_lanes<8, 2>, lane_lds_floats(2));
+      case 84: return launch(k_sessions_lanes<8, 4>, lane_lds_floats(4));
+      default: return hipErrorInvalidValue;
+    }
+  }
+  if (a.nsplit_fast == 0 && a.nsplit_win == 0) {
+    switch (bits) {
+      case 2: return launch(k_sessions_rows<2>, 0);
+      case 4: return launch(k_sessions_rows<4>, 0);
+      case 8: return launch(k_sessions_rows<8>, 0);
+      default: return hipErrorInvalidValue;
+    }
+  }
+  const int nrs = fast_nrs(D, a.gq), nh = 4 * nrs;
+  const size_t logits = (size_t)4 * nh * ((a.nsplit_fast > 0 ? fast_cpw(static_cast<int>(bits), nrs) : 1) * 64 + kRowPad);
+  const size_t floats = std::max(logits, (size_t)4 * nh * (D + 2));
+#define KIVI_SM(B, N, DD) \
+  case DD * 100 + B * 10 + N: return launch(k_sessions_mfma<B, N, DD>, floats);
+  switch (D * 100 + bits * 10 + nrs) {
+    KIVI_SM(2, 1, 64) KIVI_SM(2, 2, 64) KIVI_SM(4, 1, 64) KIVI_SM(4, 2, 64) KIVI_SM(8, 1, 64) KIVI_SM(8, 2, 64)
+    KIVI_SM(2, 1, 128) KIVI_SM(2, 2, 128) KIVI_SM(4, 1, 128) KIVI_SM(4, 2, 128) KIVI_SM(8, 1, 128) KIVI_SM(8, 2, 128)
+    KIVI_SM(2, 1, 192) KIVI_SM(4, 1, 192) KIVI_SM(8, 1, 192)
+    KIVI_SM(2, 1, 256) KIVI_SM(4, 1, 256) KIVI_SM(8, 1, 256)
+    default: return hipErrorInvalidValue;
+  }
+#undef KIVI_SM
+}
 
 template <int BITS, int NRS>
 hipError_t launch_sessions(const AttnArgs& a, const SessionTable& t, const GroupBytes& by,
@@ -4171,33 +4295,47 @@ namespace {
 
 // Launch group [first, first + count): its form and arguments (queries, outputs and the
 // window range of that group).
-AttnArgs group_args(const SessionsProblem& p, uint32_t first, uint32_t count, float* ws, bool* shared) {
+AttnArgs group_args(const SessionsProblem& p, uint32_t first, uint32_t count, float* ws, bool each, bool* shared) {
   SessionsProblem gp = p;
   gp.queries = p.queries + (uint64_t)first * p.batch * p.qh * p.cache.geo.D;
   gp.out = p.out + (uint64_t)first * p.batch * p.qh * p.cache.geo.D;
-  *shared = use_shared(p, count);
   const uint64_t longest = longest_suffix(p, first, count);
+  *shared = !each && use_shared(p, count);
+  if (each) {
+    AttnArgs a = make_args(session_problem(gp, longest), ws, count);
+    set_session_strides(gp, count, a);
+    return a;
+  }
   return *shared ? make_shared_args(gp, count, longest, ws) : make_session_args(gp, count, longest, ws);
 }
+
+// Partials a batched call of single-session launches may take (256 MB); larger ones run one by one,
+// each session in its own workspace.
+constexpr size_t kEachFloats = (size_t)64 << 20;
 
 }  // namespace
 
 size_t sessions_workspace_floats(const SessionsProblem& p) {
-  if (!sessions_supported(p)) return 0;
+  const SessionForm form = session_form(p);
+  if (form == SessionForm::kNone) return 0;
   // every launch group reuses the workspace from its start
   size_t most = 0;
   for (uint32_t first = 0; first < p.n; first += kMaxLaunchSessions) {
     const uint32_t count = std::min(kMaxLaunchSessions, p.n - first);
     bool shared;
-    const AttnArgs a = group_args(p, first, count, nullptr, &shared);
+    const AttnArgs a = group_args(p, first, count, nullptr, form == SessionForm::kEach, &shared);
     most = std::max(most, (size_t)count * a.ws_sess_stride);
   }
-  return most;
+  return form == SessionForm::kEach && most > kEachFloats ? 0 : most;
 }
+
+bool sessions_one_by_one(const SessionsProblem& p) { return session_form(p) == SessionForm::kEach; }
 
 hipError_t launch_sessions_attention(const SessionsProblem& p, float* workspace,
                                      hipStream_t stream) {
-  if (!sessions_supported(p)) return hipErrorNotSupported;
+  const SessionForm form = session_form(p);
+  if (form == SessionForm::kNone) return hipErrorNotSupported;
+  const bool each = form == SessionForm::kEach;
   const Geometry& g = p.cache.geo;
   for (uint32_t first = 0; first < p.n; first += kMaxLaunchSessions) {
     const uint32_t count = std::min(kMaxLaunchSessions, p.n - first);
@@ -4208,7 +4346,7 @@ hipError_t launch_sessions_attention(const SessionsProblem& p, float* workspace,
       suffix_rows += 2.0 * (double)t.d[i].len;
     }
     bool shared;
-    const AttnArgs a = group_args(p, first, count, workspace, &shared);
+    const AttnArgs a = group_args(p, first, count, workspace, each, &shared);
     // algorithmic bytes: the prefix once, every session's suffix, the queries
     const double key_tok = g.D * g.bits / 8.0 + g.D * 8.0 / g.G;
     const double val_tok = g.D * g.bits / 8.0 + g.ncg() * 8.0;
@@ -4218,7 +4356,8 @@ hipError_t launch_sessions_attention(const SessionsProblem& p, float* workspace,
                         g.units * suffix_rows * row, count * (double)a.q_sess_stride * 4.0};
     hipError_t e = hipSuccess;
     const int nrs = a.gq <= 4 ? 1 : 2;
-    switch (g.bits * 10 + nrs) {
+    if (each) e = launch_each(a, t, by, stream);
+    else switch (g.bits * 10 + nrs) {
       case 21: e = shared ? launch_shared<2, 1>(a, t, by, stream) : launch_sessions<2, 1>(a, t, by, stream); break;
       case 22: e = shared ? launch_shared<2, 2>(a, t, by, stream) : launch_sessions<2, 2>(a, t, by, stream); break;
       case 41: e = shared ? launch_shared<4, 1>(a, t, by, stream) : launch_sessions<4, 1>(a, t, by, stream); break;

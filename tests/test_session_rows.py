@@ -12,10 +12,13 @@ matrix-core paths form products of 22 bits, 1e-4 at inputs of unit variance; a s
 logits are scaled by s may be off by s times that of its largest value (first order in the logits).
 """
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import kivi
+from helpers import DeviceArrays
 from kivi import KiviCache, KiviConfig
 
 pytestmark = pytest.mark.gpu
@@ -36,13 +39,42 @@ CASES[6] = (2, 1, 2, 1, 1500, 64 + 33)  # 64 rows in a first launch group, 33 in
 CASES.append((4, 1, 2, 2, 1500, 49))    # 98 rows: the GEMM form
 
 
+# Other shapes: one launch for all sessions, each as its single-session launch. Lane splits, row splits
+# alone (no packed chunk; a group of 8), the matrix-core chunks of other head_dims (with row splits
+# behind them) and of groups of 64 (with window chunks), suffixes from empty to several splits.
+OTHER = [
+    # bits, group, dim, batch, kv heads, query heads per KV head, prefix tokens, sessions
+    (4, 32, 96, 1, 2, 1, 900, 5),
+    (2, 16, 80, 2, 1, 4, 1500, 3),
+    (8, 16, 128, 1, 2, 7, 700, 66),     # two launch groups
+    (2, 32, 128, 1, 2, 4, 20, 4),       # no packed keys
+    (4, 8, 64, 1, 2, 3, 500, 3),
+    (2, 32, 64, 1, 3, 4, 1300, 6),
+    (4, 64, 256, 1, 1, 5, 800, 3),
+    (8, 32, 192, 1, 1, 2, 640, 4),
+    (2, 64, 128, 1, 2, 4, 1000, 5),
+    (4, 128, 128, 2, 1, 8, 900, 3),
+    (4, 8, 24, 1, 2, 3, 300, 3),        # generic splits: the sessions one by one
+]
+
+
+@pytest.mark.parametrize("case", OTHER)
+def test_sessions_of_other_shapes_against_dense(amd, case):
+    bits, group, dim, batch, heads, gq, n, count = case
+    run(amd, bits, group, 2 * group, dim, batch, heads, gq, n, count, 1.0)
+
+
 @pytest.mark.parametrize("spread", [1.0, 1e6])
 @pytest.mark.parametrize("case", CASES)
 def test_rows_of_sessions_against_dense(amd, case, spread):
     bits, batch, heads, gq, n, count = case
-    dim, qh = 128, heads * gq
+    run(amd, bits, 32, 64, 128, batch, heads, gq, n, count, spread)
+
+
+def run(amd, bits, group, residual, dim, batch, heads, gq, n, count, spread):
+    qh = heads * gq
     rng = np.random.default_rng(5100 + n + count)
-    cache = KiviCache(amd, KiviConfig(bits, 32, 64), batch, heads, dim)
+    cache = KiviCache(amd, KiviConfig(bits, group, residual), batch, heads, dim)
     k, v = (rng.standard_normal((batch, heads, n, dim)).astype(np.float32) for _ in range(2))
     cache.append(k, v, n)
     kd, vd = (x.reshape(batch, heads, n, dim).astype(np.float64) for x in cache.dequantize())
@@ -66,3 +98,47 @@ def test_rows_of_sessions_against_dense(amd, case, spread):
         w = np.exp(logits - logits.max(-1, keepdims=True))
         want = (w / w.sum(-1, keepdims=True)) @ vv
         assert np.abs(got[i] - want).max() < 1e-4, f"session {i}"
+
+
+def test_batch_captured_after_single_calls(amd):
+    """Each session's own call has sized its workspace; a capture of all of them as one batch finds no
+    workspace for a shared launch, runs them one by one and replays to the eager batch's rows."""
+    hip = C.CDLL("libamdhip64.so.7")
+    rng = np.random.default_rng(77)
+    heads, gq, dim, n, count = 2, 2, 96, 900, 3
+    qh, per = heads * gq, heads * gq * dim
+    cache = KiviCache(amd, KiviConfig(4, 32, 64), 1, heads, dim)
+    k, v = (rng.standard_normal((heads, n, dim)).astype(np.float32) for _ in range(2))
+    cache.append(k, v, n)
+    prefix = cache.share_prefix()
+    sessions = [prefix.session() for _ in range(count)]
+    mem = DeviceArrays()
+    q = rng.standard_normal(count * per).astype(np.float32)
+    dq, out = mem.upload(q), mem.empty(count * per)
+    stream, graph, exe = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamCreate(C.byref(stream)) == 0
+
+    def call(which, q_ptr, rows):
+        kivi.sessions_attention_device(amd, which, q_ptr, rows, qh, 0.1, out, rows, stream.value)
+
+    for s in sessions:
+        call([s], dq, per)
+    assert hip.hipStreamSynchronize(stream) == 0
+    assert hip.hipStreamBeginCapture(stream, 0) == 0
+    try:
+        call(sessions, dq, count * per)
+    finally:
+        rc = hip.hipStreamEndCapture(stream, C.byref(graph))
+    assert rc == 0
+    assert hip.hipGraphInstantiate(C.byref(exe), graph, None, None, C.c_size_t(0)) == 0
+    want = kivi.sessions_attention(amd, sessions, q, qh, 0.1)
+    for _ in range(3):
+        assert hip.hipMemcpy(C.c_void_p(out), np.zeros(count * per, np.float32).ctypes.data_as(C.c_void_p),
+                             C.c_size_t(4 * count * per), 1) == 0
+        assert hip.hipGraphLaunch(exe, stream) == 0
+        assert hip.hipStreamSynchronize(stream) == 0
+        got = mem.download(out, count * per)  # other splits than the batch's: twice the bar above
+        assert np.abs(got - np.asarray(want).reshape(-1)).max() < 2e-4
+    assert hip.hipGraphExecDestroy(exe) == 0 and hip.hipGraphDestroy(graph) == 0
+    assert hip.hipStreamDestroy(stream) == 0
+    mem.free()
