@@ -26,6 +26,8 @@
 //    its grid.
 //  * k_attn_shared / k_attn_sessions / k_attn_suffix — batched sessions over one shared
 //    prefix (the prefix read once for all sessions).
+//  * k_sessions_lanes / k_sessions_rows / k_sessions_mfma — batched sessions at other shapes: the
+//    splits below, or the matrix-core ones, of every session in one launch.
 //  * k_attn_lanes — packed chunks of the other head_dims and groups that are multiples of 16, in
 //    f32 on the vector ALU, with row splits for the tokens after them.
 //  * k_attn_rows — row splits alone: caches without a packed chunk, the quality guard's fp32
@@ -2730,7 +2732,7 @@ __global__ void __launch_bounds__(kThreads, kWide16Blocks) k_attn_sessions(AttnA
 // Batched sessions at the other shapes: the single-session launch once per session, the sessions of
 // one block index side by side, so that a prefix chunk is read from HBM once. Bound as those launches
 // are; what it saves is two launches per session. 8 units: 8 sessions x 10007 tokens at head_dim 96
-// 175 -> 52 us; 20 x 20007 at head_dim 64 268 -> 52; 40 x 10007 at G = 64 535 -> 85.
+// 175 -> 52 us; 20 x 20007 at head_dim 64 333 -> 65; 40 x 10007 at G = 64 535 -> 120.
 template <int BITS, int HP>
 __global__ void __launch_bounds__(kThreads, lane_min_groups(BITS, HP)) k_sessions_lanes(AttnArgs a, SessionTable t) {
   extern __shared__ float lds[];
