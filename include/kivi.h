@@ -300,7 +300,10 @@ kivi_status kivi_session_attention(const kivi_session* session, const float* que
  * (src/prefix.rs:228-289). queries/out are [n][batch][num_q_heads][head_dim]. Device
  * pointers for queries/out, enqueued on `stream`. The split workspace belongs to the
  * prefix: batched calls on one prefix are ordered after each other (a call on another
- * stream waits for the previous call's stream, which must still exist). The sessions'
+ * stream waits for the previous call's stream, which must still exist). Under stream capture
+ * the sessions run one by one in their own workspaces, as their own calls do, except at head_dim
+ * 128, group 32 and up to eight query heads per KV head with packed keys, where a graph keeps
+ * the prefix's workspace (a later eager batch that needs a larger one frees it). The sessions'
  * suffixes must not be appended to while a call that reads them is in flight. */
 kivi_status kivi_sessions_attention_device(const kivi_session* const* sessions, size_t n,
                                            const float* queries, size_t queries_len,

@@ -1296,25 +1296,35 @@ Status batched_sessions(const kivi_session* const* sessions, size_t n, const flo
   sp.scale = scale;
   const size_t gq = num_q_heads / core.heads;
   const size_t ws_floats = n <= UINT32_MAX ? sessions_workspace_floats(sp) : 0;
-  // Sessions that only share launches also run one by one, each in its own workspace: one alone, and
-  // where the launch's workspace cannot grow, under capture or without the memory.
+  // Sessions that only share launches also run one by one, each in its own workspace: one alone,
+  // without the memory for the launch's workspace, and under capture, where a graph holds its own
+  // sessions' workspaces and not the prefix's, which every other batch of the prefix writes, orders
+  // and may grow. An eager batch sizes and orders the sessions' own too, so that a capture of them
+  // on its stream allocates nothing and waits for no other stream.
   const bool each = ws_floats > 0 && sessions_one_by_one(sp);
   bool batched = ws_floats > 0 && gq * core.head_dim <= kMaxGqD && !(each && n == 1);
+  if (batched && each) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    HIP_TRY(hipStreamIsCapturing(s, &capture), "sessions capture status");
+    batched = capture == hipStreamCaptureStatusNone;
+    for (size_t i = 0; batched && i < n; ++i) {
+      kivi_session* se = const_cast<kivi_session*>(sessions[i]);  // its workspace only
+      AttnProblem p;
+      KIVI_TRY(attention_problem(core, descs[i].k, descs[i].v, descs[i].len, descs[i].stride, dq + i * per, num_q_heads,
+                                 scale, dout + i * per, false, &p));
+      std::lock_guard<std::mutex> lock(se->attn.mu);
+      KIVI_TRY(se->attn.reserve(attention_workspace_floats(p) * sizeof(float), s));
+      KIVI_TRY(se->attn.before(s));  // the session's latest stream is the batch's, as after a call of its own
+      KIVI_TRY(se->attn.after(s));
+    }
+  }
   if (batched) {
     AttnSync& sync_ = st->batch;
     std::lock_guard<std::mutex> lock(sync_.mu);
-    const size_t bytes = ws_floats * sizeof(float);
-    if (each && bytes > sync_.workspace.bytes) {
-      hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-      HIP_TRY(hipStreamIsCapturing(s, &capture), "sessions capture status");
-      batched = capture == hipStreamCaptureStatusNone;
-    }
-    if (batched) {
-      const Status grown = sync_.reserve(bytes, s);
-      if (!grown.ok() && !each) return grown;
-      batched = grown.ok();
-      if (!batched) (void)hipGetLastError();
-    }
+    const Status grown = sync_.reserve(ws_floats * sizeof(float), s);
+    if (!grown.ok() && !each) return grown;
+    batched = grown.ok();
+    if (!batched) (void)hipGetLastError();
     if (batched) {
       KIVI_TRY(sync_.before(s));
       HIP_TRY(launch_sessions_attention(sp, sync_.workspace.as<float>(), s), "sessions attention");
