@@ -352,6 +352,9 @@ struct SessionsProblem {
   float scale;
 };
 size_t sessions_workspace_floats(const SessionsProblem& p);
+// Floats to grow the workspace to: enough for any batch of no more sessions and no longer suffixes
+// (fewer rows can take more splits each), so that such a batch needs no growth, under capture say.
+size_t sessions_reserve_floats(const SessionsProblem& p);
 // Whether the call's sessions only share launches, each with the workgroups of its own attention.
 bool sessions_one_by_one(const SessionsProblem& p);
 hipError_t launch_sessions_attention(const SessionsProblem& p, float* workspace,

@@ -1321,7 +1321,8 @@ Status batched_sessions(const kivi_session* const* sessions, size_t n, const flo
   if (batched) {
     AttnSync& sync_ = st->batch;
     std::lock_guard<std::mutex> lock(sync_.mu);
-    const Status grown = sync_.reserve(ws_floats * sizeof(float), s);
+    const bool fits = ws_floats * sizeof(float) <= sync_.workspace.bytes;
+    const Status grown = fits ? Status{} : sync_.reserve(sessions_reserve_floats(sp) * sizeof(float), s);
     if (!grown.ok() && !each) return grown;
     batched = grown.ok();
     if (!batched) (void)hipGetLastError();

@@ -4331,6 +4331,18 @@ size_t sessions_workspace_floats(const SessionsProblem& p) {
   return form == SessionForm::kEach && most > kEachFloats ? 0 : most;
 }
 
+size_t sessions_reserve_floats(const SessionsProblem& p) {
+  size_t most = sessions_workspace_floats(p);
+  if (session_form(p) != SessionForm::kRows) return most;
+  const uint64_t longest = longest_suffix(p, 0, p.n);
+  for (uint32_t count = 1; count <= std::min(kMaxLaunchSessions, p.n); ++count) {
+    const AttnArgs a = use_shared(p, count) ? make_shared_args(p, count, longest, nullptr)
+                                            : make_session_args(p, count, longest, nullptr);
+    most = std::max(most, (size_t)count * a.ws_sess_stride);
+  }
+  return most;
+}
+
 bool sessions_one_by_one(const SessionsProblem& p) { return session_form(p) == SessionForm::kEach; }
 
 hipError_t launch_sessions_attention(const SessionsProblem& p, float* workspace,

@@ -146,3 +146,24 @@ def test_graphs_of_disjoint_sessions_replay_side_by_side(amd, bits, group, dim, 
     for exe, s in zip(graphs, streams):
         assert r.hip.hipGraphExecDestroy(exe) == 0 and r.hip.hipStreamDestroy(s) == 0
     r.mem.free()
+
+
+@pytest.mark.parametrize("gq,most", [(1, 9), (2, 9), (4, 5), (8, 3)])
+def test_fewer_sessions_than_warmed(amd, gq, most):
+    """head_dim 128 and group 32, where a graph keeps the prefix's workspace: an eager batch sizes it for
+    every smaller batch of the prefix too (fewer rows take more splits of the chunks)."""
+    r = Rig(amd, 2, 32, 128, 8, gq, 10007)
+    sessions = r.sessions([0, 17, 70, 140, 30, 9, 0, 64, 5][:most])
+    stream = r.stream()
+    r.batch(sessions).eager(stream)
+    for count in range(most, 0, -1):
+        b = r.batch(sessions[:count])
+        exe = b.capture(stream)
+        for _ in range(3):
+            b.clear()
+            assert r.hip.hipGraphLaunch(exe, stream) == 0
+            r.wait(stream)
+            assert np.abs(b.result() - b.want).max() < 2e-4
+        assert r.hip.hipGraphExecDestroy(exe) == 0
+    assert r.hip.hipStreamDestroy(stream) == 0
+    r.mem.free()
