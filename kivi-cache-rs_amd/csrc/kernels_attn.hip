@@ -3834,7 +3834,8 @@ AttnArgs make_args_as(const AttnProblem& p, float* ws, SplitPlan plan, uint32_t 
   // Row splits: one pass of a workgroup (at least 16 tokens) while the launch has few workgroups,
   // doubled while four per CU remain.
   a.hgroups_rows = p.cache.geo.D % 16 == 0 ? (a.gq + kRowHeads - 1) / kRowHeads : 0u;
-  if (plan == SplitPlan::kFewest) a.S = kRowMaxTokens;
+  // (generic splits keep the tokens their LDS is bounded for, see split_tokens)
+  if (plan == SplitPlan::kFewest && a.hgroups_rows != 0) a.S = kRowMaxTokens;
   if (plan == SplitPlan::kCounted && fast && !fast_win) {
     a.S = std::max(32u, a.S / 4);
     const uint64_t rest = a.total - a.t_begin;
@@ -3989,6 +3990,8 @@ hipError_t dispatch_generic(const AttnArgs& a, hipStream_t stream) {
     return hipGetLastError();
   }
   const size_t lds = ((size_t)a.gq * a.c.geo.D + (size_t)a.gq * a.S) * sizeof(float);
+  const hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(&k_attn_generic), lds);
+  if (e != hipSuccess) return e;
   k_attn_generic<<<a.units * a.nsplit_gen, kThreads, lds, stream>>>(a);
   return hipGetLastError();
 }
