@@ -3761,16 +3761,17 @@ uint32_t level_splits(uint32_t base, uint32_t most, uint32_t units, uint32_t chu
   return steps(best) * 5 <= steps(base) * 4 ? best : base;
 }
 
-// How many splits a plan takes: what pays, as few as its kernels go, or the plan by which the
-// allocation-free attention counts a call's partials (no lane splits, the rest in splits of 256
-// tokens, or of 16 to 64 behind matrix-core chunks).
+// How many splits a plan takes: what pays, as few packed splits as its kernels go, or the plan by
+// which the allocation-free attention counts a call's partials (no lane splits, the rest in splits of
+// 256 tokens, or of 16 to 64 behind matrix-core chunks).
 enum class SplitPlan { kUsual, kFewest, kCounted };
 
 // `sessions` problems like p share the launch: the f32 splits (lanes, rows) may be that much longer
 // (8 sessions x 10007 tokens at head_dim 96: 71 -> 52 us). The matrix-core splits keep to one
 // problem's: their error grows with the chunks a wave adds up (22 sessions x 30616 tokens at
 // head_dim 256, 4 bits: 1.8e-6 at 4 chunks per wave, 3.4e-6 at 8, for 235 against 232 us).
-AttnArgs make_args_as(const AttnProblem& p, float* ws, SplitPlan plan, uint32_t sessions) {
+// `row_tokens`: the fewest tokens a row split takes.
+AttnArgs make_args_as(const AttnProblem& p, float* ws, SplitPlan plan, uint32_t sessions, uint32_t row_tokens = 0) {
   AttnArgs a{};
   a.c = p.cache;
   a.st = p.st;
@@ -3834,18 +3835,17 @@ AttnArgs make_args_as(const AttnProblem& p, float* ws, SplitPlan plan, uint32_t 
   // Row splits: one pass of a workgroup (at least 16 tokens) while the launch has few workgroups,
   // doubled while four per CU remain.
   a.hgroups_rows = p.cache.geo.D % 16 == 0 ? (a.gq + kRowHeads - 1) / kRowHeads : 0u;
-  // (generic splits keep the tokens their LDS is bounded for, see split_tokens)
-  if (plan == SplitPlan::kFewest && a.hgroups_rows != 0) a.S = kRowMaxTokens;
   if (plan == SplitPlan::kCounted && fast && !fast_win) {
     a.S = std::max(32u, a.S / 4);
     const uint64_t rest = a.total - a.t_begin;
     while (a.S > 16 && (uint64_t)p.cache.geo.units * ((rest + a.S - 1) / a.S) < 1024) a.S >>= 1;
   }
-  if (a.hgroups_rows != 0 && plan == SplitPlan::kUsual) {
+  // (Generic splits keep the tokens their LDS is bounded for, see split_tokens.)
+  if (a.hgroups_rows != 0 && plan != SplitPlan::kCounted) {
     const uint64_t rest = a.total - a.t_begin, vu = (uint64_t)p.cache.geo.units * a.hgroups_rows * sessions;
     const uint32_t pass = std::min(64u, std::max(16u, row_pass(p.cache.geo.D)));
     auto splits = [&](uint32_t S) { return (rest + S - 1) / S; };
-    a.S = pass;
+    a.S = std::max(pass, row_tokens);
     while (2 * a.S <= kRowMaxTokens && vu * splits(2 * a.S) >= kRowGroups) a.S *= 2;
   }
   a.nsplit_gen = static_cast<uint32_t>((a.total - a.t_begin + a.S - 1) / a.S);
@@ -3863,17 +3863,26 @@ uint64_t workspace_floats(const AttnArgs& a) {
   return (uint64_t)a.units * a.nsplit_total * a.gq * (a.c.geo.D + 2);
 }
 
-// The lane and row splits can take more partials than the counted plan; a call whose counted
-// partials fit the static workspace keeps to a plan that does too, so that the allocation-free
-// attention takes (and refuses) the same calls whatever splits pay.
-AttnArgs make_args(const AttnProblem& p, float* ws, uint32_t sessions = 1) {
-  const AttnArgs a = make_args_as(p, ws, SplitPlan::kUsual, sessions);
-  if (workspace_floats(a) <= kStaticWorkspaceFloats) return a;
-  for (SplitPlan plan : {SplitPlan::kFewest, SplitPlan::kCounted}) {
-    const AttnArgs f = make_args_as(p, ws, plan, sessions);
-    if (workspace_floats(f) <= kStaticWorkspaceFloats) return f;
-  }
-  return a;
+// The plan of one call. The usual plan can take more partials than the counted one (lane and row
+// splits, evened grids), and the allocation-free attention takes a call by the counted ones and gives
+// the bits of the allocating call. So where the counted partials fit the static workspace and the
+// usual ones don't, every entry point (not only that one) runs the plan with the most splits that
+// does fit: longer row splits first, then fewer packed ones. Calls that one refuses or cannot make
+// (a suffix) keep the usual plan. Measured, with the usual plan beside it: head_dim 1024, G = 8, four
+// heads, 32 units x 3500 tokens 557 us (440), 8 x 1200 81 (64; with 256-token row splits 362); head_dim
+// 256, 300 x 1500 62 (64; 80).
+AttnArgs make_args(const AttnProblem& p, float* ws) {
+  const AttnArgs a = make_args_as(p, ws, SplitPlan::kUsual, 1);
+  auto fits = [](const AttnArgs& x) { return workspace_floats(x) <= kStaticWorkspaceFloats; };
+  if (fits(a) || p.suffix_len != 0) return a;
+  const AttnArgs counted = make_args_as(p, ws, SplitPlan::kCounted, 1);
+  if (!fits(counted)) return a;
+  for (SplitPlan plan : {SplitPlan::kUsual, SplitPlan::kFewest})
+    for (uint32_t tokens = a.S; tokens <= kRowMaxTokens; tokens *= 2) {
+      const AttnArgs f = make_args_as(p, ws, plan, 1, tokens);
+      if (fits(f)) return f;
+    }
+  return counted;
 }
 
 // A launch whose waves own at most one packed chunk each (at head_dim 128, where the window
@@ -4119,7 +4128,7 @@ void set_session_strides(const SessionsProblem& sp, uint32_t nsess, AttnArgs& a)
 }
 
 AttnArgs make_session_args(const SessionsProblem& sp, uint32_t nsess, uint64_t max_suffix, float* ws) {
-  AttnArgs a = make_args(session_problem(sp, max_suffix), ws);
+  AttnArgs a = make_args_as(session_problem(sp, max_suffix), ws, SplitPlan::kUsual, 1);
   // packed splits: 16 rows each, at most kWide16Cpw chunks per wave, at least kFastGroups workgroups
   a.hgroups_fast = (nsess * a.gq + kWide16Heads - 1) / kWide16Heads;
   const uint32_t vu = a.units * a.hgroups_fast, most = (a.chunk_end + 3) / 4;
@@ -4307,7 +4316,7 @@ AttnArgs group_args(const SessionsProblem& p, uint32_t first, uint32_t count, fl
   const uint64_t longest = longest_suffix(p, first, count);
   *shared = !each && use_shared(p, count);
   if (each) {
-    AttnArgs a = make_args(session_problem(gp, longest), ws, count);
+    AttnArgs a = make_args_as(session_problem(gp, longest), ws, SplitPlan::kUsual, count);
     set_session_strides(gp, count, a);
     return a;
   }

@@ -56,3 +56,19 @@ GENERIC = [
 @pytest.mark.parametrize("bits,group,dim,units,gq,n,counted", GENERIC)
 def test_generic_splits_of_many_heads(amd, bits, group, dim, units, gq, n, counted):
     check(amd, bits, group, 2 * group, dim, units, gq, n, 1.4e-4, counted)
+
+
+AROUND_STATIC = [
+    # bits, group, residual, dim, units, query heads per KV head, tokens, bar, counted partials
+    (4, 64, 64, 256, 340, 4, 447, 1e-4, 340 * 5 * 4 * 258),   # an evened grid and its row splits
+    (4, 8, 32, 1024, 8, 4, 1200, 2e-5, 8 * 5 * 4 * 1026),     # row splits alone
+    (4, 16, 1024, 1024, 8, 4, 1500, 2e-5, 8 * 6 * 4 * 1026),  # lane splits before a long window
+    (4, 16, 16, 48, 1000, 32, 200, 2e-5, 1000 * 32 * 50),     # only the counted plan fits
+    (4, 8, 16, 48, 130, 12, 10000, 2e-5, 130 * 40 * 12 * 50),  # counted too large: the usual plan
+]
+
+
+@pytest.mark.parametrize("bits,group,residual,dim,units,gq,n,bar,counted", AROUND_STATIC)
+def test_plans_around_the_static_workspace(amd, bits, group, residual, dim, units, gq, n, bar, counted):
+    """Cases whose usual plan takes more partials than the static workspace holds."""
+    check(amd, bits, group, residual, dim, units, gq, n, bar, counted)
