@@ -253,6 +253,12 @@ __global__ void __launch_bounds__(1024)
     const float levels = static_cast<float>(geo.levels());
     const float x = *slot;  // stream token vq, the oldest of the window
     float mn = x, mx = x;
+    // a group of NaNs alone ends at the infinities, as in the longer appends of these head_dims (at
+    // 64, 128, 192 and 256 it stays NaN)
+    if (D % 64 != 0 || D > 256) {
+      mn = fminf(mn, INFINITY);
+      mx = fmaxf(mx, -INFINITY);
+    }
     for (uint32_t o = 1; o < G; o <<= 1) {
       mn = fminf(mn, __shfl_xor(mn, o));
       mx = fmaxf(mx, __shfl_xor(mx, o));

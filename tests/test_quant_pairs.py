@@ -87,3 +87,57 @@ def test_single_token_appends_match_oracle(amd, oracle, bits, group, dim):
         assert same(got, want), name
     for got, want in zip(a.dequantize(), o.dequantize()):
         assert same(got[~np.isnan(want)], want[~np.isnan(want)])
+
+
+# pair forms and one-launch appends at head_dims the wave forms do not take
+NAN_CASES = [(2, 16, 80), (4, 32, 96), (8, 16, 112), (4, 64, 320), (8, 128, 384), (2, 16, 1024)]
+
+
+def nan_rows(rng, shape, group):
+    """Single NaNs, whole channel groups of NaNs in some rows, and NaN-only channels over many rows."""
+    x = rng.standard_normal(shape).astype(np.float32)
+    flat = x.reshape(-1)
+    flat[rng.choice(flat.size, max(1, flat.size // 50), replace=False)] = np.nan
+    x[0, shape[1] // 3, :group] = np.nan
+    x[-1, -1, -group:] = np.nan
+    x[-1, :, 3] = np.nan
+    return x
+
+
+def same_or_nan(a, b):
+    a, b = np.asarray(a), np.asarray(b)
+    if a.dtype != np.float32:
+        return np.array_equal(a, b)
+    return np.array_equal(np.isnan(a), np.isnan(b)) and same(a[~np.isnan(a)], b[~np.isnan(b)])
+
+
+def check_streams(a, o):
+    for got, want, name in zip(a.export_streams(), o.export_streams(), ("key codes", "key params", "value codes", "value params")):
+        assert same_or_nan(got, want), name
+
+
+@pytest.mark.parametrize("bits,group,dim", NAN_CASES)
+def test_nans_are_passed_over(amd, oracle, bits, group, dim):
+    """A NaN takes no part in a group's minimum and maximum and gets code 0; a group of NaNs alone keeps
+    the reduction's initial values, zero +inf and scale -inf (src/quant.rs:303, 356: f32::min / max).
+    Long appends, the standalone codec, and the same rows token by token."""
+    rng = np.random.default_rng(6500 + dim)
+    cfg, units, n = KiviConfig(bits, group, group), 2, 4 * group
+    k, v = nan_rows(rng, (units, n, dim), group), nan_rows(rng, (units, n, dim), group)
+    a, o = KiviCache(amd, cfg, 1, units, dim), KiviCache(oracle, cfg, 1, units, dim)
+    for c in (a, o):
+        c.append(k, v, n)
+    check_streams(a, o)
+    for fn in (quantize_per_channel, quantize_per_token):
+        got, want = (fn(x, k, 1, units, n, dim, bits, group) for x in (amd, oracle))
+        assert same_or_nan(got.codes(), want.codes()) and same_or_nan(got.scale_zero(), want.scale_zero())
+    steps = min(n, 160)
+    a, o = KiviCache(amd, cfg, 1, units, dim), KiviCache(oracle, cfg, 1, units, dim)
+    for t in range(steps):
+        for c in (a, o):
+            c.append(np.ascontiguousarray(k[:, n - steps + t:n - steps + t + 1]),
+                     np.ascontiguousarray(v[:, n - steps + t:n - steps + t + 1]), 1)
+    for t in range(group):  # evict them all
+        for c in (a, o):
+            c.append(np.ones((units, 1, dim), np.float32), np.ones((units, 1, dim), np.float32), 1)
+    check_streams(a, o)
