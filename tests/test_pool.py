@@ -108,3 +108,131 @@ def test_allocating_calls_are_refused_under_capture(amd):
     assert c.sequence_length() == 100
     assert hip.hipStreamDestroy(stream) == 0
     mem.free()
+
+
+class Capture:
+    """A capture of the allocation-free attention on its own stream, begun by this thread; ``other`` runs
+    on another thread before it ends."""
+
+    def __init__(self, amd, mode):
+        self.hip, self.mode, self.mem = C.CDLL("libamdhip64.so.7"), mode, DeviceArrays()
+        self.cache = self.make(amd, 1)
+        q = np.random.default_rng(3).standard_normal(4 * 128).astype(np.float32)
+        self.n = q.size
+        self.dq, self.out, self.out2 = self.mem.upload(q), self.mem.empty(q.size), self.mem.empty(q.size)
+        self.streams = [C.c_void_p() for _ in range(2)]
+        for s in self.streams:
+            assert self.hip.hipStreamCreate(C.byref(s)) == 0
+        self.cache.attention_device(self.dq, self.n, 4, 0.1, self.out2, self.n, self.streams[1].value)
+        self.want = self.mem.download(self.out2, self.n)
+
+    @staticmethod
+    def make(amd, seed):
+        c = KiviCache(amd, KiviConfig(2, 32, 32), 1, 2, 128)
+        c.append(*rows(seed, 2, 300, 128), 300)
+        return c
+
+    def run(self, other):
+        graph, failure = C.c_void_p(), []
+
+        def work():
+            try:
+                other(self)
+            except BaseException as e:  # reported by the test's own thread
+                failure.append(e)
+
+        assert self.hip.hipStreamBeginCapture(self.streams[0], self.mode) == 0
+        self.cache.attention_device_noalloc(self.dq, self.n, 4, 0.1, self.out, self.n, self.streams[0].value)
+        t = threading.Thread(target=work)
+        t.start()
+        t.join()
+        rc = self.hip.hipStreamEndCapture(self.streams[0], C.byref(graph))
+        self.hip.hipGetLastError()
+        if failure:
+            raise failure[0]
+        return rc, graph
+
+
+@pytest.mark.parametrize("mode", [1, 2])  # thread-local, relaxed
+@pytest.mark.parametrize("what", ["cache", "growth", "session", "quantized"])
+def test_freeing_leaves_captures_of_other_threads_alone(amd, mode, what):
+    cap = Capture(amd, mode)
+    c = Capture.make(amd, 2)
+    k, v = rows(9, 2, 1000, 128)
+    dk, dv = cap.mem.upload(k.reshape(-1)), cap.mem.upload(v.reshape(-1))
+    held = [None if what == "growth" else c if what == "cache" else c.share_prefix().session() if what == "session"
+            else quantize_per_channel(amd, k[:, :992].copy(), 1, 2, 992, 128, 2, 32)]
+    if what == "cache":
+        del c
+
+    def other(cap):
+        if what == "growth":
+            c.append_device(dk, k.size, dv, v.size, 1000, cap.streams[1].value)
+        held.clear()
+
+    rc, graph = cap.run(other)
+    assert rc == 0
+    exe = C.c_void_p()
+    assert cap.hip.hipGraphInstantiate(C.byref(exe), graph, None, None, C.c_size_t(0)) == 0
+    for _ in range(3):
+        assert cap.hip.hipMemcpy(C.c_void_p(cap.out), np.zeros(cap.n, np.float32).ctypes.data_as(C.c_void_p),
+                                 C.c_size_t(4 * cap.n), 1) == 0
+        assert cap.hip.hipGraphLaunch(exe, cap.streams[0]) == 0
+        assert cap.hip.hipStreamSynchronize(cap.streams[0]) == 0
+        assert np.array_equal(cap.mem.download(cap.out, cap.n), cap.want)
+    assert cap.hip.hipGraphExecDestroy(exe) == 0 and cap.hip.hipGraphDestroy(graph) == 0
+    for s in cap.streams:
+        assert cap.hip.hipStreamDestroy(s) == 0
+    cap.mem.free()
+
+
+@pytest.mark.parametrize("replay", [False, True])
+def test_a_buffer_waits_for_every_stream_that_reads_it(amd, replay):
+    """Dense reconstructions on two streams, or by a graph's launch on another stream than it was captured
+    on, then the cache freed at once and its buffers taken by the next one."""
+    hip, mem = C.CDLL("libamdhip64.so.7"), DeviceArrays()
+    units, n, dim = 8, 20000, 128
+    cfg = KiviConfig(4, 32, 32)
+    k, v = rows(11, units, n, dim)
+    streams = [C.c_void_p() for _ in range(2)]
+    for s in streams:
+        assert hip.hipStreamCreateWithFlags(C.byref(s), 1) == 0  # non-blocking
+    dk, dv = mem.upload(k.reshape(-1)), mem.upload(v.reshape(-1))
+    outs = [(mem.alloc(k.size), mem.alloc(k.size)) for _ in streams]
+
+    def filled():
+        c = KiviCache(amd, cfg, 1, units, dim)
+        c.reserve(n)
+        return c
+
+    c = filled()
+    c.append(k, v, n)
+    want = [np.asarray(x).view(np.uint32).copy() for x in c.dequantize()]
+    for _ in range(4):
+        if replay:
+            graph, exe = C.c_void_p(), C.c_void_p()
+            assert hip.hipStreamBeginCapture(streams[0], 1) == 0
+            c.dequantize_device(outs[0][0], k.size, outs[0][1], k.size, streams[0].value)
+            assert hip.hipStreamEndCapture(streams[0], C.byref(graph)) == 0
+            assert hip.hipGraphInstantiate(C.byref(exe), graph, None, None, C.c_size_t(0)) == 0
+            for _ in range(8):
+                assert hip.hipGraphLaunch(exe, streams[1]) == 0
+        else:
+            for _ in range(8):
+                for s, (a, b) in zip(streams, outs):
+                    c.dequantize_device(a, k.size, b, k.size, s.value)
+        del c
+        c = filled()  # the same sizes: the buffers just given back
+        c.append_device(dv, k.size, dk, k.size, n, streams[0].value)
+        assert hip.hipDeviceSynchronize() == 0
+        for a, b in outs[:1] if replay else outs:
+            for ptr, x in ((a, want[0]), (b, want[1])):
+                assert np.array_equal(mem.download(ptr, k.size).view(np.uint32), x.reshape(-1))
+        if replay:
+            assert hip.hipGraphExecDestroy(exe) == 0 and hip.hipGraphDestroy(graph) == 0
+        del c
+        c = filled()
+        c.append(k, v, n)
+    for s in streams:
+        assert hip.hipStreamDestroy(s) == 0
+    mem.free()
