@@ -237,6 +237,13 @@ struct DeviceScope {
   }
 };
 
+// The outcome of a call whose failure is nothing to report: a refused free or wait, as under capture.
+// Takes the error out of HIP's last-error state, which the next launch would report as its own.
+bool tolerated(hipError_t e) {
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e == hipSuccess;
+}
+
 // Device memory the library's objects gave back, kept for the next ones: a request that makes and
 // frees a cache spent more on hipMalloc and hipFree (page mapping, 20-300 us each) than on its
 // kernels (16 x 8 units x 32768 tokens prefilled and exported: 1100 of 2370 us). Per device, at most
@@ -286,7 +293,7 @@ class DevicePool {
       std::lock_guard<std::mutex> lock(mu_);
       blocks_.push_back(Block{p, n, device});
     } catch (...) {
-      (void)hipFree(p);
+      (void)tolerated(hipFree(p));
       return;
     }
     (void)trim(device, kPoolBytes, kPoolBlocks);
@@ -318,7 +325,7 @@ class DevicePool {
         p = blocks_[oldest].p;
         blocks_.erase(blocks_.begin() + oldest);
       }
-      (void)hipFree(p);
+      (void)tolerated(hipFree(p));
       any = true;
     }
   }
@@ -330,7 +337,7 @@ class DevicePool {
 // hundred launches.
 bool wait_device() {
   void* p = nullptr;
-  return hipMalloc(&p, 256) == hipSuccess && hipFree(p) == hipSuccess;
+  return tolerated(hipMalloc(&p, 256)) && tolerated(hipFree(p));
 }
 
 // Waits for all work on the current device once (`idle`: the caller knows that none of it uses the
@@ -371,7 +378,7 @@ struct DevBuf {
       if (idle)
         DevicePool::get().give(p, block, device);
       else
-        (void)hipFree(p);
+        (void)tolerated(hipFree(p));
     }
     p = nullptr;
     bytes = block = 0;
@@ -387,8 +394,7 @@ struct DevBuf {
     release();
     if (n == 0) return Status{};
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    const bool captured = hipStreamIsCapturing(s, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone;
-    if (captured) (void)hipGetLastError();
+    const bool captured = !tolerated(hipStreamIsCapturing(s, &capture)) || capture != hipStreamCaptureStatusNone;
     const hipError_t e = DevicePool::get().take(&p, n, captured, &device, &block);
     if (e != hipSuccess) {
       p = nullptr;
@@ -410,7 +416,7 @@ struct Scratch {
   void* p = nullptr;
   hipStream_t s = nullptr;
   ~Scratch() {
-    if (p != nullptr) (void)hipFreeAsync(p, s);
+    if (p != nullptr) (void)tolerated(hipFreeAsync(p, s));
   }
   Status get(size_t bytes, hipStream_t stream, const char* what) {
     s = stream;
@@ -846,10 +852,9 @@ struct DeviceCallOrder {
   bool any = false, one = true;
   void enter(hipStream_t s) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    const hipError_t e = hipStreamIsCapturing(s, &cs);
-    if (e != hipSuccess) (void)hipGetLastError();
+    const bool known = tolerated(hipStreamIsCapturing(s, &cs));
     std::lock_guard<std::mutex> lock(mu);
-    if ((any && s != only) || e != hipSuccess || cs != hipStreamCaptureStatusNone) one = false;
+    if ((any && s != only) || !known || cs != hipStreamCaptureStatusNone) one = false;
     any = true;
     only = s;
   }
@@ -881,8 +886,9 @@ struct kivi_cache {
   // Waits for the streams the cache knows; true when no work on its buffers is left anywhere.
   bool finish() {
     const bool settled = settle().ok();
-    const bool own = hipStreamSynchronize(core.stream) == hipSuccess;
+    const bool own = tolerated(hipStreamSynchronize(core.stream));
     const bool drained = attn.drain().ok();
+    if (!settled || !drained) (void)hipGetLastError();
     return settled && own && drained && dev.one;
   }
 };
@@ -2084,8 +2090,8 @@ void kivi_guard_free(kivi_guard* guard) {
   if (guard == nullptr) return;
   {
     DeviceScope scope(guard->cache->core.device);
-    (void)hipStreamSynchronize(guard->cache->core.stream);
-    (void)guard->dense.drain();
+    (void)tolerated(hipStreamSynchronize(guard->cache->core.stream));
+    if (!guard->dense.drain().ok()) (void)hipGetLastError();
     QuietDevice quiet;
     guard->tk.release();
     guard->tv.release();

@@ -236,3 +236,26 @@ def test_a_buffer_waits_for_every_stream_that_reads_it(amd, replay):
     for s in streams:
         assert hip.hipStreamDestroy(s) == 0
     mem.free()
+
+
+@pytest.mark.parametrize("what", ["session", "quantized", "prefix"])
+def test_a_refused_free_leaves_no_error_behind(amd, what):
+    """An object freed while another thread captures in global mode (which refuses to free memory): the
+    freeing thread's next call on another cache succeeds."""
+    cap = Capture(amd, 0)
+    k = rows(9, 2, 992, 128)[0]
+    prefix = Capture.make(amd, 2).share_prefix()
+    held = [prefix.session() if what == "session" else quantize_per_channel(amd, k, 1, 2, 992, 128, 2, 32)
+            if what == "quantized" else prefix]
+    del prefix
+
+    def other(cap):
+        held.clear()
+        cap.cache.attention_device(cap.dq, cap.n, 4, 0.1, cap.out2, cap.n, cap.streams[1].value)
+
+    assert np.array_equal(cap.mem.download(cap.out2, cap.n), cap.want)
+    cap.run(other)  # global mode: the refusal may have ended the capture
+    assert np.array_equal(cap.mem.download(cap.out2, cap.n), cap.want)
+    for s in cap.streams:
+        assert cap.hip.hipStreamDestroy(s) == 0
+    cap.mem.free()
