@@ -460,6 +460,12 @@ const char* kivi_status_name(int32_t code);
 int32_t kivi_abi_version(void);
 /* Number of usable HIP devices (0 when none); never fails. */
 int32_t kivi_device_count(void);
+/* Extension: device memory of freed objects (arenas, windows, suffixes, attention workspaces,
+ * quantized tensors, guard tapes) stays with the library for the next ones, at most 1 GiB and 256
+ * blocks per device, and is freed when an allocation of the library fails for want of memory. This
+ * call frees what is kept on the current device, for other allocators of the process, and returns
+ * its bytes (0 without a device). kivi_cache_device_bytes does not count it. */
+size_t kivi_release_pooled_memory(void);
 
 /* ---------------------------------------------------------------- kernel timing
  * Measurement hooks for benchmark harnesses; no counterpart in the reference, whose path

@@ -248,7 +248,7 @@ bool tolerated(hipError_t e) {
 // frees a cache spent more on hipMalloc and hipFree (page mapping, 20-300 us each) than on its
 // kernels (16 x 8 units x 32768 tokens prefilled and exported: 1100 of 2370 us). Per device, at most
 // kPoolBytes in kPoolBlocks blocks; past that the oldest are freed at once, and all of a device's
-// are when an allocation there fails. A block is only given back while the device is idle (see
+// are when an allocation there fails (the pool's own or a call's scratch). A block is only given back while the device is idle (see
 // QuietDevice), as hipFree would have waited for, so whoever takes it next may use it on any
 // stream. Any thread may take and give.
 class DevicePool {
@@ -282,12 +282,14 @@ class DevicePool {
     }
     *got = n;
     e = hipMalloc(p, n);
-    if (e == hipErrorOutOfMemory && !fresh && trim(*device, 0, 0)) {
+    if (e == hipErrorOutOfMemory && !fresh && empty(*device) > 0) {
       (void)hipGetLastError();
       e = hipMalloc(p, n);
     }
     return e;
   }
+  // Frees all it keeps for a device; the bytes.
+  size_t empty(int device) { return trim(device, 0, 0); }
   void give(void* p, size_t n, int device) {
     try {
       std::lock_guard<std::mutex> lock(mu_);
@@ -307,9 +309,9 @@ class DevicePool {
   };
   std::mutex mu_;
   std::vector<Block> blocks_;  // oldest first
-  // Frees a device's oldest blocks down to the limits; true when any was freed.
-  bool trim(int device, size_t bytes, size_t count) {
-    bool any = false;
+  // Frees a device's oldest blocks down to the limits; the bytes freed.
+  size_t trim(int device, size_t bytes, size_t count) {
+    size_t freed = 0;
     for (;;) {
       void* p = nullptr;
       {
@@ -321,12 +323,12 @@ class DevicePool {
           ++n;
           oldest = i;
         }
-        if (oldest == blocks_.size() || (held <= bytes && n <= count)) return any;
+        if (oldest == blocks_.size() || (held <= bytes && n <= count)) return freed;
         p = blocks_[oldest].p;
+        freed += blocks_[oldest].bytes;
         blocks_.erase(blocks_.begin() + oldest);
       }
       (void)tolerated(hipFree(p));
-      any = true;
     }
   }
 };
@@ -421,7 +423,16 @@ struct Scratch {
   Status get(size_t bytes, hipStream_t stream, const char* what) {
     s = stream;
     if (bytes == 0) return Status{};
-    HIP_TRY(hipMallocAsync(&p, bytes, stream), what);
+    hipError_t e = hipMallocAsync(&p, bytes, stream);
+    int device = 0;
+    if (e == hipErrorOutOfMemory && hipGetDevice(&device) == hipSuccess && DevicePool::get().empty(device) > 0) {
+      (void)hipGetLastError();
+      e = hipMallocAsync(&p, bytes, stream);
+    }
+    if (e != hipSuccess) {
+      p = nullptr;
+      return DevErr(e, what);
+    }
     return Status{};
   }
   template <class T>
@@ -2316,6 +2327,12 @@ const char* kivi_status_name(int32_t code) {
 }
 
 int32_t kivi_abi_version(void) { return KIVI_ABI_VERSION; }
+
+size_t kivi_release_pooled_memory(void) {
+  int device = 0;
+  if (device_count() <= 0 || !tolerated(hipGetDevice(&device))) return 0;
+  return DevicePool::get().empty(device);
+}
 
 int32_t kivi_device_count(void) { return device_count(); }
 

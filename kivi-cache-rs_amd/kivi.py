@@ -266,6 +266,7 @@ _SIGS = {
 # Entry points only the HIP library has (device pointers, streams, device queries).
 _DEVICE_SIGS = {
     "device_count": (C.c_int32, []),
+    "release_pooled_memory": (_SZ, []),
     "timing_enable": (None, [C.c_int32]),
     "timing_read": (C.c_int, [C.c_int32, C.POINTER(_KernelTiming), _ERRP]),
     "status_name": (C.c_char_p, [C.c_int32]),
@@ -925,6 +926,11 @@ class QuantizedTensor:
     def dequantize_device(self, out_ptr, out_len, stream=0):
         self._b.call("quantized_dequantize_device", self._h, C.c_void_p(out_ptr), out_len,
                      C.c_void_p(stream))
+
+
+def release_pooled_memory(backend):
+    """Frees the device memory the library keeps of freed objects; its bytes (HIP library only)."""
+    return backend["release_pooled_memory"]()
 
 
 def plan_device_bytes(backend, config, batch, num_kv_heads, head_dim, tokens):

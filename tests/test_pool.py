@@ -8,6 +8,7 @@ import threading
 import numpy as np
 import pytest
 
+import kivi
 from kivi import KiviCache, KiviConfig, KiviError, quantize_per_channel
 from helpers import DeviceArrays
 
@@ -259,3 +260,42 @@ def test_a_refused_free_leaves_no_error_behind(amd, what):
     for s in cap.streams:
         assert cap.hip.hipStreamDestroy(s) == 0
     cap.mem.free()
+
+
+def free_device_bytes(hip):
+    free, total = C.c_size_t(), C.c_size_t()
+    assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def test_kept_memory_can_be_taken_back(amd):
+    hip = C.CDLL("libamdhip64.so.7")
+    kivi.release_pooled_memory(amd)
+    assert kivi.release_pooled_memory(amd) == 0
+    before = free_device_bytes(hip)
+    c = KiviCache(amd, KiviConfig(8, 32, 32), 1, 8, 128)
+    c.reserve(200_000)
+    size = c.device_bytes()
+    del c
+    assert before - free_device_bytes(hip) >= size
+    assert kivi.release_pooled_memory(amd) >= size
+    assert before - free_device_bytes(hip) < size // 8
+
+
+def test_scratch_gets_the_kept_memory(amd):
+    """A host append whose staging fits the device only together with what the pool keeps."""
+    hip, mem = C.CDLL("libamdhip64.so.7"), DeviceArrays()
+    kivi.release_pooled_memory(amd)
+    units, n, dim = 8, 80000, 128  # 328 MB of staging for the keys, as much for the values
+    c = KiviCache(amd, KiviConfig(2, 32, 32), 1, units, dim)
+    c.reserve(n)
+    k = rows(21, units, n, dim)[0]
+    big = KiviCache(amd, KiviConfig(8, 32, 32), 1, 8, 128)
+    big.reserve(380_000)  # 973 MB
+    ballast = mem.alloc((free_device_bytes(hip) - (280 << 20)) // 4)
+    del big  # the pool's from here on
+    try:
+        c.append(k, k, n)
+    finally:
+        mem.free()
+    assert ballast and c.sequence_length() == n
