@@ -291,6 +291,10 @@ class DevicePool {
   // Frees all it keeps for a device; the bytes.
   size_t empty(int device) { return trim(device, 0, 0); }
   void give(void* p, size_t n, int device) {
+    if (n > kPoolBytes) {  // would push everything else out and then leave itself
+      (void)tolerated(hipFree(p));
+      return;
+    }
     try {
       std::lock_guard<std::mutex> lock(mu_);
       blocks_.push_back(Block{p, n, device});

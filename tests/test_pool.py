@@ -292,10 +292,29 @@ def test_scratch_gets_the_kept_memory(amd):
     k = rows(21, units, n, dim)[0]
     big = KiviCache(amd, KiviConfig(8, 32, 32), 1, 8, 128)
     big.reserve(380_000)  # 973 MB
-    ballast = mem.alloc((free_device_bytes(hip) - (280 << 20)) // 4)
+    mem.alloc((free_device_bytes(hip) - (280 << 20)) // 4)
+    for _ in range(64):  # what was free rounds down: leave 200 to 232 MiB
+        if free_device_bytes(hip) < 232 << 20:
+            break
+        mem.alloc(8 << 20)
     del big  # the pool's from here on
     try:
         c.append(k, k, n)
     finally:
         mem.free()
-    assert ballast and c.sequence_length() == n
+    assert c.sequence_length() == n
+
+
+def test_a_block_past_the_bound_leaves_the_others(amd):
+    """A tensor whose codes alone are above 1 GiB (1.5 GiB, with 96 MiB of parameters) freed after a small
+    one (64 + 4 MiB): the codes go back to the device, the rest stays."""
+    hip, mem = C.CDLL("libamdhip64.so.7"), DeviceArrays()
+    kivi.release_pooled_memory(amd)
+    n = 3 << 29
+    data = mem.alloc(n)
+    for elements in (1 << 26, n):
+        q = kivi.quantize_device(amd, False, data, elements, 1, 1, elements // 128, 128, 8, 128)
+        del q
+    assert kivi.release_pooled_memory(amd) == (64 + 4 + 96) << 20
+    assert hip.hipDeviceSynchronize() == 0
+    mem.free()
