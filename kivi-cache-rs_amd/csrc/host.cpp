@@ -244,6 +244,12 @@ bool tolerated(hipError_t e) {
   return e == hipSuccess;
 }
 
+// Whether p points into memory of device `dev` itself.
+bool on_device(const void* p, int dev) {
+  hipPointerAttribute_t a{};
+  return tolerated(hipPointerGetAttributes(&a, p)) && a.type == hipMemoryTypeDevice && a.device == dev;
+}
+
 // Device memory the library's objects gave back, kept for the next ones: a request that makes and
 // frees a cache spent more on hipMalloc and hipFree (page mapping, 20-300 us each) than on its
 // kernels (16 x 8 units x 32768 tokens prefilled and exported: 1100 of 2370 us). Per device, at most
@@ -1286,20 +1292,17 @@ Status session_append(kivi_session* se, const float* keys, size_t keys_len, cons
     se->cap = cap;
   }
   const size_t row = seq_len * D * 4;
-  if (device) {
-    HIP_TRY(copy_units(se->keys.as<float>() + se->len * D, se->cap * D * 4, keys, row, row,
-                       static_cast<uint32_t>(units), s), "suffix append");
-    HIP_TRY(copy_units(se->values.as<float>() + se->len * D, se->cap * D * 4, values, row, row,
-                       static_cast<uint32_t>(units), s), "suffix append");
-    se->len = new_len;
-    return Status{};
-  }
-  HIP_TRY(hipMemcpy2DAsync(se->keys.as<float>() + se->len * D, se->cap * D * 4, keys, row, row,
-                           units, hipMemcpyHostToDevice, s), "suffix append");
-  HIP_TRY(hipMemcpy2DAsync(se->values.as<float>() + se->len * D, se->cap * D * 4, values, row, row,
-                           units, hipMemcpyHostToDevice, s), "suffix append");
+  const hipMemcpyKind kind = device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
+  auto copy = [&](float* dst, const float* src) {
+    // a kernel's copy only from this device's own memory: another device's may not be mapped here
+    if (device && on_device(src, core.device))
+      return copy_units(dst, se->cap * D * 4, src, row, row, static_cast<uint32_t>(units), s);
+    return hipMemcpy2DAsync(dst, se->cap * D * 4, src, row, row, units, kind, s);
+  };
+  HIP_TRY(copy(se->keys.as<float>() + se->len * D, keys), "suffix append");
+  HIP_TRY(copy(se->values.as<float>() + se->len * D, values), "suffix append");
   se->len = new_len;
-  return sync(s, "session append");
+  return device ? Status{} : sync(s, "session append");
 }
 
 Status batched_sessions(const kivi_session* const* sessions, size_t n, const float* queries,

@@ -142,3 +142,39 @@ def test_batch_captured_after_single_calls(amd):
     assert hip.hipGraphExecDestroy(exe) == 0 and hip.hipGraphDestroy(graph) == 0
     assert hip.hipStreamDestroy(stream) == 0
     mem.free()
+
+
+@pytest.mark.parametrize("off", [0, 4])
+@pytest.mark.parametrize("pinned", [False, True])
+def test_suffix_rows_of_device_and_pinned_memory(amd, pinned, off):
+    """Suffixes appended from this device's memory (a kernel's copy, or the copy engine 4 bytes off) and
+    from pinned host memory (the copy engine): the rows of the host-pointer append."""
+    hip, mem = C.CDLL("libamdhip64.so.7"), DeviceArrays()
+    rng = np.random.default_rng(91)
+    heads, dim = 3, 128
+    cache = KiviCache(amd, KiviConfig(2, 32, 32), 1, heads, dim)
+    k, v = (rng.standard_normal((heads, 100, dim)).astype(np.float32) for _ in range(2))
+    cache.append(k, v, 100)
+    prefix = cache.share_prefix()
+    a, b = prefix.session(), prefix.session()
+    for n in (5, 1, 40, 3):
+        rows = [rng.standard_normal(heads * n * dim).astype(np.float32) for _ in range(2)]
+        ptrs, hosts = [], []
+        for x in rows:
+            x = np.concatenate([np.zeros(off // 4, np.float32), x])
+            if pinned:
+                p = C.c_void_p()
+                assert hip.hipHostMalloc(C.byref(p), C.c_size_t(x.nbytes), 0) == 0
+                C.memmove(p, x.ctypes.data, x.nbytes)
+                hosts.append(p)
+                ptrs.append(p.value + off)
+            else:
+                ptrs.append(mem.upload(x) + off)
+        a.append_device(ptrs[0], rows[0].size, ptrs[1], rows[1].size, n)
+        b.append(rows[0], rows[1], n)
+        assert hip.hipDeviceSynchronize() == 0
+        for p in hosts:
+            assert hip.hipHostFree(p) == 0
+    q = rng.standard_normal(2 * heads * dim).astype(np.float32)
+    assert np.array_equal(a.attention(q, 2 * heads, 0.1), b.attention(q, 2 * heads, 0.1))
+    mem.free()
