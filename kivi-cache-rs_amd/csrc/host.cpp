@@ -869,13 +869,14 @@ struct DeviceCallOrder {
   bool pending = false;
   // Whether every device-pointer call so far came on one stream and none under capture: then that
   // stream's end is the end of all of them (no other stream or graph launch has work of theirs).
+  // hipStreamPerThread names another stream in every thread, so it never counts as one.
   hipStream_t only = nullptr;
   bool any = false, one = true;
   void enter(hipStream_t s) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     const bool known = tolerated(hipStreamIsCapturing(s, &cs));
     std::lock_guard<std::mutex> lock(mu);
-    if ((any && s != only) || !known || cs != hipStreamCaptureStatusNone) one = false;
+    if ((any && s != only) || s == hipStreamPerThread || !known || cs != hipStreamCaptureStatusNone) one = false;
     any = true;
     only = s;
   }

@@ -239,6 +239,59 @@ def test_a_buffer_waits_for_every_stream_that_reads_it(amd, replay):
     mem.free()
 
 
+def test_a_buffer_waits_for_every_threads_own_stream(amd):
+    """Dense reconstructions of two threads on hipStreamPerThread (one handle, a stream per thread), then
+    the cache freed by a third and its buffers taken by the next one."""
+    hip, mem = C.CDLL("libamdhip64.so.7"), DeviceArrays()
+    units, n, dim, per_thread = 8, 20000, 128, 2
+    cfg = KiviConfig(4, 32, 32)
+    k, v = rows(11, units, n, dim)
+    stream = C.c_void_p()
+    assert hip.hipStreamCreateWithFlags(C.byref(stream), 1) == 0
+    dk, dv = mem.upload(k.reshape(-1)), mem.upload(v.reshape(-1))
+    outs = [(mem.alloc(k.size), mem.alloc(k.size)) for _ in range(2)]
+
+    def filled():
+        c = KiviCache(amd, cfg, 1, units, dim)
+        c.reserve(n)
+        return c
+
+    for _ in range(4):
+        c = filled()
+        c.append(k, v, n)
+        want = [np.asarray(x).view(np.uint32).copy() for x in c.dequantize()]
+        held, queued, freed, failure = [c], threading.Barrier(3), threading.Event(), []
+        del c
+
+        def read(out):
+            try:
+                for _ in range(8):
+                    held[0].dequantize_device(out[0], k.size, out[1], k.size, per_thread)
+            except BaseException as e:
+                failure.append(e)
+            queued.wait(60)
+            freed.wait(60)  # a thread's stream ends with the thread
+
+        threads = [threading.Thread(target=read, args=(o,)) for o in outs]
+        for t in threads:
+            t.start()
+        queued.wait(60)
+        held.clear()
+        c = filled()  # the same sizes: the buffers just given back
+        c.append_device(dv, k.size, dk, k.size, n, stream.value)
+        assert hip.hipDeviceSynchronize() == 0
+        freed.set()
+        for t in threads:
+            t.join()
+        assert not failure
+        for out in outs:
+            for ptr, x in zip(out, want):
+                assert np.array_equal(mem.download(ptr, k.size).view(np.uint32), x.reshape(-1))
+        del c
+    assert hip.hipStreamDestroy(stream) == 0
+    mem.free()
+
+
 @pytest.mark.parametrize("what", ["session", "quantized", "prefix"])
 def test_a_refused_free_leaves_no_error_behind(amd, what):
     """An object freed while another thread captures in global mode (which refuses to free memory): the
