@@ -336,8 +336,8 @@ struct SessionTable {
 };
 
 // n sessions sharing one prefix: the prefix's packed chunks serve all sessions' rows (session, head)
-// at once, 16 rows per pass over them or, from kSharedMinRows rows on, as a GEMM operand (which takes
-// the prefix window too); each session's suffix (and window) runs per session. Returns
+// at once, 16 rows per pass over them or, with many rows or a long prefix window, as a GEMM operand (which
+// takes the window too); each session's suffix (and window) runs per session. Returns
 // hipErrorNotSupported for shapes without the packed-chunk path (the caller then runs the sessions
 // one by one).
 struct SessionsProblem {

@@ -4165,18 +4165,12 @@ uint64_t longest_suffix(const SessionsProblem& sp, uint32_t first, uint32_t coun
   return m;
 }
 
-// Rows (sessions x GQA heads) from which one launch group takes the GEMM form. Below, groups of 16
-// rows on the 16x16x32 path: each costs a pass over the chunks, where the GEMM form dequantizes
-// them once but then costs nearly the same for 16 rows as for 128. Step times at 8 units, 2 bits:
-// 16 rows x 65536 tokens 35.3 us (GEMM form 165), 80 rows x 10007 40.7 (53.6), 128 rows x 30000
-// 102 (98), 256 rows x 65536 380 (221).
+// Rows (sessions x GQA heads) from which one launch group takes the GEMM form always, and the fewest
+// with which it may (see shared_pays).
 constexpr uint32_t kSharedMinRows = 97;
+constexpr uint32_t kSharedFewRows = 16;
 // Workgroups the GEMM form aims for (one per CU: 148 KB of LDS each).
 constexpr uint32_t kSharedTargetGroups = 256;
-
-bool use_shared(const SessionsProblem& sp, uint32_t nsess) {
-  return nsess * (sp.qh / sp.heads) >= kSharedMinRows;
-}
 
 // The GEMM form's splits: the packed chunks of a unit in nsplit contiguous ranges, nsplit a
 // multiple of 8 (the XCD count) where the chunks allow, so about kSharedTargetGroups
@@ -4184,8 +4178,7 @@ bool use_shared(const SessionsProblem& sp, uint32_t nsess) {
 // The GEMM form covers every prefix chunk, [0, ceil(seq/64)) (the fp32 band of the prefix
 // too, as the prefix's smax covers those rows); k_attn_suffix covers each session's suffix
 // [seq, seq + len) in runs of kSufTokens.
-AttnArgs make_shared_args(const SessionsProblem& sp, uint32_t nsess, uint64_t max_suffix, float* ws) {
-  AttnArgs a = make_session_args(sp, nsess, max_suffix, ws);
+AttnArgs make_shared_args(const SessionsProblem& sp, uint32_t nsess, uint64_t max_suffix, AttnArgs a) {
   const uint32_t rblocks = (nsess * a.gq + kShRows - 1) / kShRows;
   const uint32_t per = a.units * rblocks;
   uint32_t ns = (kSharedTargetGroups + per - 1) / per;
@@ -4197,6 +4190,42 @@ AttnArgs make_shared_args(const SessionsProblem& sp, uint32_t nsess, uint64_t ma
   a.nsplit_total = a.nsplit_fast + a.nsplit_win + a.nsplit_gen;
   a.ws_sess_stride = (uint64_t)sp.cache.geo.units * a.nsplit_total * a.gq * (sp.cache.geo.D + 2);
   return a;
+}
+
+// Whether a group of kSharedFewRows to kSharedMinRows - 1 rows is faster as a GEMM, `r` and `s` its
+// arguments in the two forms. Groups of 16 rows on the 16x16x32 path cost a pass over the packed chunks
+// each and one window workgroup per session and 64 fp32 tokens (the prefix's window included); the GEMM
+// form reads chunks and window once for all rows, costs nearly the same for 16 rows as for 96, and
+// its busiest workgroup, with `cps` chunks, sets the time of each round of workgroups (fp32 chunks are
+// not pipelined). Times in us fitted to 2538 shapes (2-64 units, 16-96 rows, 1-8 heads, 1500-40000
+// tokens, residuals of 64-2048, suffixes of 8-300, every width), 8% and 12% off in the mean. The form it
+// takes is 0.3% dearer than the faster one in the mean, 1.29 times at most. One form for all of them: the
+// GEMM up to 5.3 times (32 units x 40000 tokens, residual 2048, 2 sessions of eight heads, 4 bits: 620 us
+// against 116), the row groups up to 8.9 (32 units x 3000 tokens, residual 2048, 64 sessions of one head,
+// 8 bits: 1015 us against 114).
+bool shared_pays(const AttnArgs& r, const AttnArgs& s) {
+  if (s.nsplit_fast == 0) return false;
+  const bool wide = r.c.geo.bits == 8;
+  const double sessions = (double)r.units * r.nsess;
+  const double rows = 14.0 + sessions * r.nsplit_win * 0.0122 * (wide ? 1.23 : 1.0) * (r.gq > 4 ? 1.41 : 1.0) +
+                      (wide ? 0.0036 : 0.0031) * r.units * r.hgroups_fast * r.chunk_end;
+  const uint32_t rblocks = (s.nsess * s.gq + kShRows - 1) / kShRows;
+  const uint32_t rounds = (s.units * rblocks * s.nsplit_fast + kSharedTargetGroups - 1) / kSharedTargetGroups;
+  const uint32_t cps = (s.gemm_end + s.nsplit_fast - 1) / s.nsplit_fast;
+  const uint32_t dense = std::min(cps, s.gemm_end - s.chunk_end);
+  const double gemm = 5.0 + rounds * (16.0 + 3.7 * cps + 7.0 * dense) + 0.0155 * sessions * std::max(1u, s.nsplit_win);
+  return gemm < rows;
+}
+
+// The arguments of a launch group of `nsess` sessions in the form it takes.
+AttnArgs make_rows_args(const SessionsProblem& sp, uint32_t nsess, uint64_t max_suffix, float* ws, bool* shared) {
+  const AttnArgs r = make_session_args(sp, nsess, max_suffix, ws);
+  const uint64_t rows = (uint64_t)nsess * r.gq;
+  *shared = false;
+  if (rows < kSharedFewRows) return r;
+  const AttnArgs s = make_shared_args(sp, nsess, max_suffix, r);
+  *shared = rows >= kSharedMinRows || shared_pays(r, s);
+  return *shared ? s : r;
 }
 
 // Algorithmic bytes of one launch group: the prefix's packed and fp32 rows, the sessions'
@@ -4319,13 +4348,13 @@ AttnArgs group_args(const SessionsProblem& p, uint32_t first, uint32_t count, fl
   gp.queries = p.queries + (uint64_t)first * p.batch * p.qh * p.cache.geo.D;
   gp.out = p.out + (uint64_t)first * p.batch * p.qh * p.cache.geo.D;
   const uint64_t longest = longest_suffix(p, first, count);
-  *shared = !each && use_shared(p, count);
   if (each) {
+    *shared = false;
     AttnArgs a = make_args_as(session_problem(gp, longest), ws, SplitPlan::kUsual, count);
     set_session_strides(gp, count, a);
     return a;
   }
-  return *shared ? make_shared_args(gp, count, longest, ws) : make_session_args(gp, count, longest, ws);
+  return make_rows_args(gp, count, longest, ws, shared);
 }
 
 // Partials a batched call of single-session launches may take (256 MB); larger ones run one by one,
@@ -4353,9 +4382,14 @@ size_t sessions_reserve_floats(const SessionsProblem& p) {
   if (session_form(p) != SessionForm::kRows) return most;
   const uint64_t longest = longest_suffix(p, 0, p.n);
   for (uint32_t count = 1; count <= std::min(kMaxLaunchSessions, p.n); ++count) {
-    const AttnArgs a = use_shared(p, count) ? make_shared_args(p, count, longest, nullptr)
-                                            : make_session_args(p, count, longest, nullptr);
-    most = std::max(most, (size_t)count * a.ws_sess_stride);
+    // either form: shorter suffixes may change it, towards the row groups (where the bare prefix takes
+    // the GEMM no suffix makes those the faster form: 128 tokens cost them two window chunks per session)
+    const AttnArgs r = make_session_args(p, count, longest, nullptr);
+    const uint64_t rows = (uint64_t)count * r.gq;
+    bool gemm;
+    (void)make_rows_args(p, count, 0, nullptr, &gemm);
+    if (!gemm) most = std::max(most, (size_t)count * r.ws_sess_stride);
+    if (rows >= kSharedFewRows) most = std::max(most, (size_t)count * make_shared_args(p, count, longest, r).ws_sess_stride);
   }
   return most;
 }

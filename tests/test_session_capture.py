@@ -20,13 +20,13 @@ SCALE = np.float32(0.1)
 
 
 class Rig:
-    def __init__(self, amd, bits=4, group=32, dim=96, heads=2, gq=2, n=900):
+    def __init__(self, amd, bits=4, group=32, dim=96, heads=2, gq=2, n=900, residual=None):
         self.amd, self.heads, self.dim, self.qh = amd, heads, dim, heads * gq
         self.per = self.qh * dim
         self.rng = np.random.default_rng(7700 + dim + group)
         self.hip = C.CDLL("libamdhip64.so.7")
         self.mem = DeviceArrays()
-        self.cache = KiviCache(amd, KiviConfig(bits, group, 2 * group), 1, heads, dim)
+        self.cache = KiviCache(amd, KiviConfig(bits, group, residual or 2 * group), 1, heads, dim)
         self.cache.append(*self.rows(n), n)
         self.prefix = self.cache.share_prefix()
 
@@ -157,6 +157,26 @@ def test_fewer_sessions_than_warmed(amd, gq, most):
     stream = r.stream()
     r.batch(sessions).eager(stream)
     for count in range(most, 0, -1):
+        b = r.batch(sessions[:count])
+        exe = b.capture(stream)
+        for _ in range(3):
+            b.clear()
+            assert r.hip.hipGraphLaunch(exe, stream) == 0
+            r.wait(stream)
+            assert np.abs(b.result() - b.want).max() < 2e-4
+        assert r.hip.hipGraphExecDestroy(exe) == 0
+    assert r.hip.hipStreamDestroy(stream) == 0
+    r.mem.free()
+
+
+def test_fewer_sessions_than_warmed_behind_a_long_window(amd):
+    """A residual of 2048 tokens: 40 sessions run as a GEMM, few of them in groups of 16 rows, and the
+    captured ones have shorter suffixes than the batch that sized the workspace."""
+    r = Rig(amd, 2, 32, 128, 8, 1, 10007, 2048)
+    sessions = r.sessions(sorted((29 * i) % 150 for i in range(40)))
+    stream = r.stream()
+    r.batch(sessions).eager(stream)
+    for count in [40, 33, 31, 24, 20, 17, 16, 15, 12, 9, 6, 4, 3, 2, 1]:
         b = r.batch(sessions[:count])
         exe = b.capture(stream)
         for _ in range(3):

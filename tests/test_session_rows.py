@@ -1,8 +1,8 @@
 """Batched sessions of a shared prefix in groups of 16 rows (``-m gpu``).
 
-Below 97 rows (sessions x query heads per KV head) the prefix's packed chunks run on the matrix
-cores with the rows of all sessions as the columns of one tile, 16 at a time; from 97 on as a GEMM
-over dequantized chunks. The cases sit at the edges: one row, a group less one, a whole group, one
+Below 97 rows (sessions x query heads per KV head) and behind a short window the prefix's packed chunks
+run on the matrix cores with the rows of all sessions as the columns of one tile, 16 at a time; from
+97 on, or from 16 where that is faster, as a GEMM over dequantized chunks. The cases sit at the edges: one row, a group less one, a whole group, one
 more, the last count before the GEMM form and the first of it, head counts that do not divide 16,
 a prefix batch above 1, prefixes without a packed chunk and with waves above a whole chunk,
 sessions whose queries differ by six orders of magnitude (each row has its own operand range).
@@ -69,6 +69,31 @@ def test_sessions_of_other_shapes_against_dense(amd, case):
 def test_rows_of_sessions_against_dense(amd, case, spread):
     bits, batch, heads, gq, n, count = case
     run(amd, bits, 32, 64, 128, batch, heads, gq, n, count, spread)
+
+
+# A long prefix window, which the row groups read once per session and the GEMM form once: the form
+# is the one whose time is less, from 16 rows on.
+WINDOWS = [
+    # bits, residual, batch, kv heads, query heads per KV head, prefix tokens, sessions, GEMM form
+    (8, 1024, 2, 8, 2, 1500, 24, True),    # 48 rows
+    (4, 512, 1, 8, 1, 1200, 64, True),
+    (2, 2048, 2, 8, 8, 2100, 2, False),    # 16 rows, no packed chunk behind the window
+    (2, 1024, 4, 8, 1, 1100, 15, False),   # 15 rows
+    (2, 1024, 4, 8, 1, 1100, 16, True),    # 16 rows
+    (2, 1024, 4, 8, 1, 1050, 20, True),    # no packed chunk
+    (4, 64, 2, 8, 4, 1500, 12, False),     # a short window
+]
+
+
+@pytest.mark.parametrize("case", WINDOWS)
+def test_long_windows_run_once_for_all_rows(amd, case):
+    bits, residual, batch, heads, gq, n, count, gemm = case
+    kivi.timing_enable(amd)
+    try:
+        run(amd, bits, 32, residual, 128, batch, heads, gq, n, count, 1.0)
+        assert (kivi.timing_read(amd, "attn_shared")[0] > 0) == gemm
+    finally:
+        kivi.timing_enable(amd, False)
 
 
 def run(amd, bits, group, residual, dim, batch, heads, gq, n, count, spread):
