@@ -872,13 +872,22 @@ struct DeviceCallOrder {
   // hipStreamPerThread names another stream in every thread, so it never counts as one.
   hipStream_t only = nullptr;
   bool any = false, one = true;
-  void enter(hipStream_t s) {
+  // Whether s records no capture (false where HIP does not say).
+  static bool plain(hipStream_t s) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    const bool known = tolerated(hipStreamIsCapturing(s, &cs));
+    return tolerated(hipStreamIsCapturing(s, &cs)) && cs == hipStreamCaptureStatusNone;
+  }
+  void enter(hipStream_t s) { enter(s, plain(s)); }
+  void enter(hipStream_t s, bool is_plain) {
     std::lock_guard<std::mutex> lock(mu);
-    if ((any && s != only) || s == hipStreamPerThread || !known || cs != hipStreamCaptureStatusNone) one = false;
+    if ((any && s != only) || s == hipStreamPerThread || !is_plain) one = false;
     any = true;
     only = s;
+  }
+  // Waits for the only stream entered; true when no work of the calls is left anywhere.
+  bool finish() {
+    std::lock_guard<std::mutex> lock(mu);
+    return one && (!any || (plain(only) && tolerated(hipStreamSynchronize(only))));
   }
   void note(hipStream_t s) {
     std::lock_guard<std::mutex> lock(mu);
@@ -931,7 +940,7 @@ struct kivi_session {
   AttnSync attn;
   DevBuf keys, values;            // [units][cap][D] fp32 suffix (the reference re-splices, src/prefix.rs:196-221)
   uint64_t len = 0, cap = 0;
-  DeviceCallOrder dev;            // host-pointer calls work on the default stream
+  DeviceCallOrder dev;            // host-pointer calls enter the default stream, where they work
 };
 
 struct kivi_runtime {
@@ -1248,6 +1257,7 @@ Status session_attend(const kivi_session* se, const float* query, size_t query_l
   DeviceScope scope(core.device);
   const uint64_t stride = se->cap * core.head_dim;
   kivi_session* ms = const_cast<kivi_session*>(se);  // its workspace only
+  ms->dev.enter(device ? stream : nullptr);
   if (device)
     return attend(core, ms->attn, se->keys.as<float>(), se->values.as<float>(), se->len, stride,
                   query, num_q_heads, scale, out, stream);
@@ -1276,6 +1286,7 @@ Status session_append(kivi_session* se, const float* keys, size_t keys_len, cons
   KIVI_TRY(need_slice(values, values_len, "values"));
   DeviceScope scope(core.device);
   hipStream_t s = device ? stream : nullptr;
+  se->dev.enter(s);
   const size_t units = core.batch * core.heads, D = core.head_dim;
   const uint64_t new_len = se->len + seq_len;
   if (new_len > se->cap) {
@@ -1290,6 +1301,11 @@ Status session_append(kivi_session* se, const float* keys, size_t keys_len, cons
     HIP_TRY(hipStreamSynchronize(s), "suffix grow");
     se->keys.swap(nk);
     se->values.swap(nv);
+    if (se->cap > 0) {
+      QuietDevice quiet(se->dev.finish());
+      nk.release();
+      nv.release();
+    }
     se->cap = cap;
   }
   const size_t row = seq_len * D * 4;
@@ -1331,6 +1347,8 @@ Status batched_sessions(const kivi_session* const* sessions, size_t n, const flo
   KIVI_TRY(need_slice(out, out_len, "out"));
   DeviceScope scope(core.device);
   hipStream_t s = device ? stream : nullptr;
+  const bool plain = DeviceCallOrder::plain(s);
+  for (size_t i = 0; i < n; ++i) const_cast<kivi_session*>(sessions[i])->dev.enter(s, plain);
   const float* dq = queries;
   float* dout = out;
   Scratch sq, so;
@@ -1964,7 +1982,7 @@ void kivi_session_free(kivi_session* s) {
   kivi_prefix* p = s->prefix;
   {
     DeviceScope scope(p->state->core.device);
-    QuietDevice quiet;
+    QuietDevice quiet(s->dev.finish());
     delete s;
   }
   kivi_prefix_release(p);

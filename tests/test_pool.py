@@ -155,7 +155,7 @@ class Capture:
 
 
 @pytest.mark.parametrize("mode", [1, 2])  # thread-local, relaxed
-@pytest.mark.parametrize("what", ["cache", "growth", "session", "quantized"])
+@pytest.mark.parametrize("what", ["cache", "growth", "session", "suffix", "quantized"])
 def test_freeing_leaves_captures_of_other_threads_alone(amd, mode, what):
     cap = Capture(amd, mode)
     c = Capture.make(amd, 2)
@@ -163,6 +163,9 @@ def test_freeing_leaves_captures_of_other_threads_alone(amd, mode, what):
     dk, dv = cap.mem.upload(k.reshape(-1)), cap.mem.upload(v.reshape(-1))
     held = [None if what == "growth" else c if what == "cache" else c.share_prefix().session() if what == "session"
             else quantize_per_channel(amd, k[:, :992].copy(), 1, 2, 992, 128, 2, 32)]
+    if what == "suffix":  # device rows on the default stream
+        held[0] = c.share_prefix().session()
+        held[0].append_device(dk, k.size, dv, v.size, 1000)
     if what == "cache":
         del c
 
@@ -289,6 +292,71 @@ def test_a_buffer_waits_for_every_threads_own_stream(amd):
                 assert np.array_equal(mem.download(ptr, k.size).view(np.uint32), x.reshape(-1))
         del c
     assert hip.hipStreamDestroy(stream) == 0
+    mem.free()
+
+
+@pytest.mark.parametrize("how", ["one stream", "two streams", "graph", "growth"])
+def test_a_suffix_waits_for_its_readers(amd, how):
+    """Attention over a long suffix, then the session freed (or its suffix grown) at once and its buffers
+    taken by the next session."""
+    hip, mem = C.CDLL("libamdhip64.so.7"), DeviceArrays()
+    units, n, dim = 2, 30000, 128
+    prefix = Capture.make(amd, 4).share_prefix()
+    k, v = rows(17, units, n, dim)
+    dk, dv = mem.upload(k.reshape(-1)), mem.upload(v.reshape(-1))
+    q = np.random.default_rng(5).standard_normal(4 * dim).astype(np.float32)
+    dq = mem.upload(q)
+    outs = [mem.empty(q.size) for _ in range(2)]
+    streams = [C.c_void_p() for _ in range(3)]
+    for s in streams:
+        assert hip.hipStreamCreateWithFlags(C.byref(s), 1) == 0  # non-blocking
+
+    def filled(stream):
+        s = prefix.session()
+        s.append_device(dk, k.size, dv, v.size, n, stream.value)
+        assert hip.hipDeviceSynchronize() == 0
+        return s
+
+    def read(session, out, stream):
+        kivi.sessions_attention_device(amd, [session], dq, q.size, 4, 0.1, out, q.size, stream.value)
+
+    se = filled(streams[0])
+    read(se, outs[0], streams[0])
+    assert hip.hipDeviceSynchronize() == 0
+    want = mem.download(outs[0], q.size)
+    for _ in range(4):
+        if how == "graph":
+            graph, exe = C.c_void_p(), C.c_void_p()
+            assert hip.hipStreamBeginCapture(streams[0], 1) == 0
+            read(se, outs[0], streams[0])
+            assert hip.hipStreamEndCapture(streams[0], C.byref(graph)) == 0
+            assert hip.hipGraphInstantiate(C.byref(exe), graph, None, None, C.c_size_t(0)) == 0
+            for _ in range(16):
+                assert hip.hipGraphLaunch(exe, streams[1]) == 0
+        else:
+            for _ in range(16):
+                read(se, outs[0], streams[0])
+                if how == "two streams":
+                    read(se, outs[1], streams[1])
+        if how == "growth":
+            se.append_device(dk, units * dim, dv, units * dim, 1, streams[0].value)
+        else:
+            del se
+        se = prefix.session()
+        se.append_device(dv, k.size, dk, k.size, n, streams[2].value)  # other rows, the same size
+        assert hip.hipDeviceSynchronize() == 0
+        for out in outs[:2 if how == "two streams" else 1]:
+            assert np.array_equal(mem.download(out, q.size).view(np.uint32), want.view(np.uint32))
+        if how == "graph":
+            assert hip.hipGraphExecDestroy(exe) == 0 and hip.hipGraphDestroy(graph) == 0
+        del se
+        se = filled(streams[0])
+        if how == "graph":  # sizes the new session's workspace
+            read(se, outs[0], streams[0])
+            assert hip.hipDeviceSynchronize() == 0
+    del se
+    for s in streams:
+        assert hip.hipStreamDestroy(s) == 0
     mem.free()
 
 
