@@ -1473,6 +1473,7 @@ Status quantize(const float* data, size_t data_len, size_t batch, size_t heads, 
   q->n_params = per_channel ? units * (tokens / group_size) * head_dim * 2
                             : units * tokens * (head_dim / group_size) * 2;
   hipStream_t s = device ? stream : nullptr;
+  q->dev.enter(s);
   // the quantize launch writes every word and every (scale, zero) pair
   KIVI_TRY(q->codes.alloc(q->n_codes * 4, s, "quantized codes"));
   KIVI_TRY(q->params.alloc(q->n_params * 4, s, "quantized params"));
@@ -1507,6 +1508,7 @@ Status quantized_read(const kivi_quantized* q, void* out, size_t out_len, size_t
   KIVI_TRY(need(out, "out"));
   DeviceScope scope(q->device);
   hipStream_t s = device ? stream : nullptr;
+  q->dev.enter(s);
   const uint32_t units = static_cast<uint32_t>(q->batch * q->heads);
   if (what == 0 || what == 2) {
     const void* src = what == 0 ? q->codes.p : q->params.p;
@@ -2277,7 +2279,7 @@ kivi_status kivi_quantize_per_token_device(const float* data, size_t data_len, s
 void kivi_quantized_free(kivi_quantized* q) {
   if (q == nullptr) return;
   DeviceScope scope(q->device);
-  QuietDevice quiet;
+  QuietDevice quiet(q->dev.finish());
   delete q;
 }
 

@@ -360,6 +360,53 @@ def test_a_suffix_waits_for_its_readers(amd, how):
     mem.free()
 
 
+@pytest.mark.parametrize("how", ["one stream", "two streams", "graph"])
+def test_a_quantized_tensor_waits_for_its_readers(amd, how):
+    """Reconstructions of a tensor, which is then freed at once and its buffers taken by the next one."""
+    hip, mem = C.CDLL("libamdhip64.so.7"), DeviceArrays()
+    units, n, dim = 8, 16384, 128
+    x, y = rows(23, units, n, dim)
+    dx, dy = mem.upload(x.reshape(-1)), mem.upload(y.reshape(-1))
+    outs = [mem.alloc(x.size) for _ in range(2)]
+    streams = [C.c_void_p() for _ in range(3)]
+    for s in streams:
+        assert hip.hipStreamCreateWithFlags(C.byref(s), 1) == 0  # non-blocking
+
+    def make(data, stream):
+        return kivi.quantize_device(amd, False, data, x.size, 1, units, n, dim, 4, 32, stream.value)
+
+    t = make(dx, streams[0])
+    want = np.asarray(t.dequantize()).view(np.uint32).reshape(-1).copy()
+    for _ in range(4):
+        if how == "graph":
+            graph, exe = C.c_void_p(), C.c_void_p()
+            assert hip.hipStreamBeginCapture(streams[0], 1) == 0
+            t.dequantize_device(outs[0], x.size, streams[0].value)
+            assert hip.hipStreamEndCapture(streams[0], C.byref(graph)) == 0
+            assert hip.hipGraphInstantiate(C.byref(exe), graph, None, None, C.c_size_t(0)) == 0
+            for _ in range(16):
+                assert hip.hipGraphLaunch(exe, streams[1]) == 0
+        else:
+            for _ in range(16):
+                t.dequantize_device(outs[0], x.size, streams[0].value)
+                if how == "two streams":
+                    t.dequantize_device(outs[1], x.size, streams[1].value)
+        del t
+        t = make(dy, streams[2])  # the buffers just given back
+        assert hip.hipDeviceSynchronize() == 0
+        for out in outs[:2 if how == "two streams" else 1]:
+            assert np.array_equal(mem.download(out, x.size).view(np.uint32), want)
+        if how == "graph":
+            assert hip.hipGraphExecDestroy(exe) == 0 and hip.hipGraphDestroy(graph) == 0
+        del t
+        t = make(dx, streams[0])
+        assert hip.hipDeviceSynchronize() == 0
+    del t
+    for s in streams:
+        assert hip.hipStreamDestroy(s) == 0
+    mem.free()
+
+
 @pytest.mark.parametrize("what", ["session", "quantized", "prefix"])
 def test_a_refused_free_leaves_no_error_behind(amd, what):
     """An object freed while another thread captures in global mode (which refuses to free memory): the
