@@ -254,8 +254,9 @@ bool on_device(const void* p, int dev) {
 // frees a cache spent more on hipMalloc and hipFree (page mapping, 20-300 us each) than on its
 // kernels (16 x 8 units x 32768 tokens prefilled and exported: 1100 of 2370 us). Per device, at most
 // kPoolBytes in kPoolBlocks blocks; past that the oldest are freed at once, and all of a device's
-// are when an allocation there fails (the pool's own or a call's scratch). A block is only given back while the device is idle (see
-// QuietDevice), as hipFree would have waited for, so whoever takes it next may use it on any
+// are when an allocation there fails (the pool's own or a call's scratch). A block is only given back
+// when no work uses it any more (the device is idle, as hipFree would have waited for, or the one
+// stream its owner was used on: see QuietDevice), so whoever takes it next may use it on any
 // stream. Any thread may take and give.
 class DevicePool {
  public:
@@ -884,10 +885,16 @@ struct DeviceCallOrder {
     any = true;
     only = s;
   }
-  // Waits for the only stream entered; true when no work of the calls is left anywhere.
+  // Waits for the calls' work where all came on the default stream; true when none is left anywhere. A
+  // caller's stream may be gone by the time an object is freed, and HIP then reads its freed memory.
   bool finish() {
     std::lock_guard<std::mutex> lock(mu);
-    return one && (!any || (plain(only) && tolerated(hipStreamSynchronize(only))));
+    return one && (!any || (only == nullptr && plain(only) && tolerated(hipStreamSynchronize(only))));
+  }
+  // Whether all calls came on the stream of the one under way.
+  bool alone() {
+    std::lock_guard<std::mutex> lock(mu);
+    return one;
   }
   void note(hipStream_t s) {
     std::lock_guard<std::mutex> lock(mu);
@@ -1302,7 +1309,7 @@ Status session_append(kivi_session* se, const float* keys, size_t keys_len, cons
     se->keys.swap(nk);
     se->values.swap(nv);
     if (se->cap > 0) {
-      QuietDevice quiet(se->dev.finish());
+      QuietDevice quiet(se->dev.alone());  // s, which has no work left
       nk.release();
       nv.release();
     }

@@ -407,6 +407,45 @@ def test_a_quantized_tensor_waits_for_its_readers(amd, how):
     mem.free()
 
 
+def test_a_tensor_may_outlive_its_stream(amd):
+    """Readers queued on a stream that is destroyed (and perhaps its handle given to a new one) before the
+    tensor is freed and its buffers taken by the next one. (Sessions free themselves the same way, but
+    their prefix's batched calls need the previous call's stream.)"""
+    hip, mem = C.CDLL("libamdhip64.so.7"), DeviceArrays()
+    units, n, dim = 2, 32768, 128
+    x, y = rows(29, units, n, dim)
+    dx, dy = mem.upload(x.reshape(-1)), mem.upload(y.reshape(-1))
+    out = mem.alloc(x.size)
+
+    def stream():
+        s = C.c_void_p()
+        assert hip.hipStreamCreateWithFlags(C.byref(s), 1) == 0
+        return s
+
+    def make(data, s):
+        return kivi.quantize_device(amd, False, data, x.size, 1, units, n, dim, 4, 32, s.value)
+
+    want = None
+    for _ in range(4):
+        s = stream()
+        t = make(dx, s)
+        for _ in range(32):
+            t.dequantize_device(out, x.size, s.value)
+        if want is None:
+            assert hip.hipStreamSynchronize(s) == 0
+            want = mem.download(out, x.size)
+        assert hip.hipStreamDestroy(s) == 0
+        others = [stream() for _ in range(3)]
+        del t
+        t = make(dy, others[0])
+        assert hip.hipDeviceSynchronize() == 0
+        assert np.array_equal(mem.download(out, x.size).view(np.uint32), want.view(np.uint32))
+        del t
+        for s in others:
+            assert hip.hipStreamDestroy(s) == 0
+    mem.free()
+
+
 @pytest.mark.parametrize("what", ["session", "quantized", "prefix"])
 def test_a_refused_free_leaves_no_error_behind(amd, what):
     """An object freed while another thread captures in global mode (which refuses to free memory): the
