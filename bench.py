@@ -543,7 +543,7 @@ def measure(name, args, torch, kivi, amd, stream, with_cpu):
     elif "attn_sessions" in kernels:
         dom_fam, dom_name = "attn_sessions", "k_attn_sessions"
     else:
-        dom_fam, dom_name = "attn_tail", "k_attn_generic"
+        dom_fam, dom_name = "attn_tail", "k_attn_rows" if dim % 16 == 0 else "k_attn_generic"
     dom = kernels.get(dom_fam)
     rec = recorded_traffic(dom_name, name, dom["bytes_per_launch"]) if dom else None
     roofline = {

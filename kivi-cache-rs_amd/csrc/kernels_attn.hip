@@ -1528,8 +1528,9 @@ __global__ void __launch_bounds__(kThreads) k_attn_rows(AttnArgs a) {
 // is reconstructed as fma(code, scale, zero) before it is used). A workgroup takes up to 16
 // consecutive 64-token chunks of a unit for HP query heads.
 //
-// What bounds it is vector issue (per element: unpacking, one fma of reconstruction, HP of use) and,
-// at one head, the cache lines its loads touch. So both contractions keep a (scale, zero) set in
+// What bounds it is vector issue (per element: unpacking, one fma of reconstruction, HP of use; 77% of
+// the vector cycles at four heads, 128 units x 32768 tokens) and, at one head, waiting for its loads (45%, and
+// waves wait 43% of theirs: 96 units x 5003 tokens). So both contractions keep a (scale, zero) set in
 // registers over many elements instead of fetching pairs per element: a lane owns 16 channels of a
 // run of 16 tokens (keys; the run lies in one key group) or 16 tokens of a run of channels (values;
 // the run lies in one value group), and one to four code words hold its 16 codes. A (scale, zero)
@@ -2383,14 +2384,6 @@ constexpr int kWide16Heads = 16;
 constexpr int kWide16Cpw = 4;     // chunks per wave: four chunks of 16 heads' logits, 16.6 KB
 constexpr int kWide16Blocks = 2;  // workgroups per CU (66.6 KB of LDS each)
 
-//
-// SESS: the columns are rows (session, head) of a batched call, hg the group of 16 rows: each row
-// has its own query pointer, its own operand range (sessions' queries may differ in magnitude) and
-// its session's partials. Its codes are taken about the middle of their range (exact in f16) and
-// its zeros moved there, x = (code - mid) scale + (zero + mid scale): a group's zero is its minimum,
-// so uncentred code and zero terms largely cancel in the sums: 13 sessions of four heads over 30007
-// tokens at 4 bits are 1.9e-6 off f64 attention uncentred, 7e-7 centred (1.4e-6 in the GEMM form),
-// for 3-5% of the time.
 // The middle of the code range (a value f16 holds, whole at 8 bits).
 constexpr float code_mid(int bits) { return bits == 8 ? 128.f : bits == 4 ? 7.5f : 1.5f; }
 template <int BITS>
@@ -2404,6 +2397,13 @@ __device__ __forceinline__ void centre_pairs(float4& p, float mid) {
   p.w = fmaf(mid, p.z, p.w);
 }
 
+// SESS: the columns are rows (session, head) of a batched call, hg the group of 16 rows: each row
+// has its own query pointer, its own operand range (sessions' queries may differ in magnitude) and
+// its session's partials. Its codes are taken about the middle of their range (exact in f16) and
+// its zeros moved there, x = (code - mid) scale + (zero + mid scale): a group's zero is its minimum,
+// so uncentred code and zero terms largely cancel in the sums: 13 sessions of four heads over 30007
+// tokens at 4 bits are 1.9e-6 off f64 attention uncentred, 7e-7 centred (1.4e-6 in the GEMM form),
+// for 3-5% of the time.
 template <int BITS, bool SESS>
 __device__ __forceinline__ void wide16_split(const AttnArgs& a, uint32_t unit, uint32_t split, uint32_t hg,
                                              float* lds) {
@@ -2706,8 +2706,8 @@ __device__ __forceinline__ AttnArgs session_args(const AttnArgs& a, const Sessio
   return as;
 }
 
-// Batched sessions over one prefix, fewer than kSharedMinRows rows (session, head): the window / suffix
-// chunks of every session first (one workgroup each, the 4x4x4 MIXED path), then the prefix's packed
+// Batched sessions over one prefix, rows (session, head) for which the GEMM form is not faster (see
+// shared_pays): the window / suffix chunks of every session first (one workgroup each, the 4x4x4 MIXED path), then the prefix's packed
 // chunks for groups of 16 rows on the sixteen-head 16x16x32 path, a chunk's codes exact and its
 // scales folded into the rows, so that no chunk is dequantized. Each group of 16 reads the chunks
 // again (from L2 or the Infinity Cache) and costs the same; the GEMM form dequantizes a chunk once
@@ -2730,8 +2730,9 @@ __global__ void __launch_bounds__(kThreads, kWide16Blocks) k_attn_sessions(AttnA
 }
 
 // Batched sessions at the other shapes: the single-session launch once per session, the sessions of
-// one block index side by side, so that a prefix chunk is read from HBM once. Bound as those launches
-// are; what it saves is two launches per session. 8 units: 8 sessions x 10007 tokens at head_dim 96
+// one block index side by side, so that a prefix chunk is read from HBM once (neighbours run on
+// different XCDs: the Infinity Cache serves them). Bound as those launches are; what it saves is two
+// launches per session. 8 units: 8 sessions x 10007 tokens at head_dim 96
 // 175 -> 52 us; 20 x 20007 at head_dim 64 333 -> 65; 40 x 10007 at G = 64 535 -> 120.
 template <int BITS, int HP>
 __global__ void __launch_bounds__(kThreads, lane_min_groups(BITS, HP)) k_sessions_lanes(AttnArgs a, SessionTable t) {
@@ -3740,8 +3741,6 @@ bool lanes_eligible(const AttnProblem& p) {
 // query heads per lane-split workgroup
 uint32_t lane_heads(uint32_t gq) { return gq <= 2 ? gq : 4u; }
 
-// MFMA chunks: [0, floor(vq/64)) (keys and values packed; vq <= kq). Everything after
-// (value window, its band of packed keys, session suffix) goes to window chunks or row splits.
 // Packed splits per unit near `base` (at most four times as many, at most `most`) that leave the
 // busiest CU the fewest chunk steps: workgroups per CU, rounded up, times chunks per wave, rounded
 // up. base itself unless another count saves a fifth: below that, more workgroups measured slower as
@@ -3776,6 +3775,9 @@ enum class SplitPlan { kUsual, kFewest, kCounted };
 // problem's: their error grows with the chunks a wave adds up (22 sessions x 30616 tokens at
 // head_dim 256, 4 bits: 1.8e-6 at 4 chunks per wave, 3.4e-6 at 8, for 235 against 232 us).
 // `row_tokens`: the fewest tokens a row split takes.
+//
+// Packed chunks: [0, floor(vq/64)) (keys and values packed; vq <= kq). Everything after (value window,
+// its band of packed keys, session suffix) goes to window chunks or row splits of the same launch.
 AttnArgs make_args_as(const AttnProblem& p, float* ws, SplitPlan plan, uint32_t sessions, uint32_t row_tokens = 0) {
   AttnArgs a{};
   a.c = p.cache;
@@ -3796,8 +3798,8 @@ AttnArgs make_args_as(const AttnProblem& p, float* ws, SplitPlan plan, uint32_t 
   a.gq = p.qh / p.heads;
   a.scale2 = p.scale * kLog2e;
   // The MFMA path covers every 64-token chunk once some keys are packed: chunks
-  // [0, floor(vq/64)) (keys and values all packed) in one launch, the rest (the fp32 value
-  // window and key residual, the session suffix) in a second launch of the MIXED kernel.
+  // [0, floor(vq/64)) (keys and values all packed), and at head_dim 128 the rest (the fp32 value
+  // window and key residual, the session suffix) as MIXED window chunks of the same grid.
   // At other head_dims the MFMA launch takes only the fully packed chunks and row splits the rest,
   // as behind the lane splits of other shapes. Without packed chunks row splits cover everything.
   const bool lanes = plan != SplitPlan::kCounted && lanes_eligible(p) && std::min(p.st.kq, p.st.vq) >= 64;

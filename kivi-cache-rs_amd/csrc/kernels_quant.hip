@@ -728,7 +728,8 @@ __global__ void __launch_bounds__(kThreads)
 // channels (a float2 per row) and the workgroup's lanes run over (run of tokens, channel pair) items,
 // pairs fastest. head_dim is a multiple of G and of the ppw channels of a word, so the lanes of a
 // word and of a channel group stay together, aligned, inside a wave, and the lane exchanges of
-// the wave forms carry over. HBM-bound like them; what they replace (k_quant_keys, k_quant_values)
+// the wave forms carry over. Keys are HBM-bound like them (5.4 TB/s read and written), values bound by
+// vector issue (70% of the vector cycles, 3.2 TB/s); what they replace (k_quant_keys, k_quant_values)
 // stages rows in LDS and runs a thread per channel or per (token, group), with a byte per code:
 // 96 units x 5003 tokens x 96 channels at 4 bits, keys 136 -> 39 us, values 143 -> 68 us.
 

@@ -182,8 +182,9 @@ def test_infinite_inputs_codes_parity(amd, oracle, bits):
     """Rows with +inf and -inf entries (the reference tests hold none): a group spanning an
     infinity gets scale inf and codes 0 (the quotient is 0 or NaN, and NaN casts to 0), the
     others quantize as usual. Packed streams bit-exact through bulk and decode appends, and
-    the standalone quantize of both axes. NaN inputs are not covered: the reference's min/max
-    skip a NaN, the kernels' compare-select reductions need not."""
+    the standalone quantize of both axes. NaN inputs are not covered here (test_quant_pairs.py has
+    them for the kernels that skip one, as the reference's min/max do; the wave kernels'
+    compare-select reductions need not)."""
     batch, heads, dim, total = 1, 2, 128, 300
     rng = np.random.default_rng(500 + bits)
     keys = rng.standard_normal((batch, heads, total, dim)).astype(np.float32)
@@ -392,7 +393,7 @@ def test_session_parity(amd, oracle):
 def test_batched_sessions_kernel_parity(amd, oracle, bits, batch, qh, n_sess, doc):
     """Batched RagSession attention on the packed-chunk path (head_dim 128, G=32): one launch
     per 64 sessions over the shared prefix (70 sessions = two launch groups), in the GEMM form
-    (sessions x heads >= 16 rows) and the per-session form, suffixes of 0 to 130 tokens, every
+    (160 and 256 rows) and in groups of 16 rows (the others), suffixes of 0 to 130 tokens, every
     session against the oracle's RagSession::attention (src/prefix.rs:223-289)."""
     heads, dim = 8, 128
     rng = np.random.default_rng(bits * 1000 + n_sess)
