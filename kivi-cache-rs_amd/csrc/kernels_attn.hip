@@ -2404,6 +2404,9 @@ __device__ __forceinline__ void centre_pairs(float4& p, float mid) {
 // so uncentred code and zero terms largely cancel in the sums: 13 sessions of four heads over 30007
 // tokens at 4 bits are 1.9e-6 off f64 attention uncentred, 7e-7 centred (1.4e-6 in the GEMM form),
 // for 3-5% of the time.
+// The value range's power of two multiplies the staged scales (four multiplications per lane and chunk,
+// no time measured) and not the weights through their exponential, which would round at its size: 20
+// rows over 1571 tokens at 8 bits 5.0e-7 -> 3.1e-7 off f64 attention, at values of 1e-10 8.6e-7 -> 3.2e-7.
 template <int BITS, bool SESS>
 __device__ __forceinline__ void wide16_split(const AttnArgs& a, uint32_t unit, uint32_t split, uint32_t hg,
                                              float* lds) {
@@ -2542,11 +2545,13 @@ __device__ __forceinline__ void wide16_split(const AttnArgs& a, uint32_t unit, u
   const float mrow = mx * kout;
 
   const float vmax = vmax_all;
-  const int ev = std::min(60, std::max(-100, 15 - __builtin_amdgcn_frexp_expf(vmax)));
+  const int ev = std::min(SESS ? 126 : 60, std::max(SESS ? -117 : -100, 15 - __builtin_amdgcn_frexp_expf(vmax)));
   const float vout = ldexpf(1.f, -ev - kExp);
   const float moff = mrow == -INFINITY ? 0.f : mrow;
-  const float evoff = static_cast<float>(ev) - moff;  // weights times 2^ev from the exponential
-  const float vinv = ldexpf(1.f, -ev);
+  // 2^ev joins the weights from the exponential, or (SESS) the staged scales
+  const float evoff = SESS ? -moff : static_cast<float>(ev) - moff;
+  const float vinv = SESS ? 1.f : ldexpf(1.f, -ev);
+  const float vfac = SESS ? ldexpf(1.f, ev) : 1.f;
 
   // ---------------- phase 2: value mix
   v4f vacc[8];
@@ -2563,7 +2568,7 @@ __device__ __forceinline__ void wide16_split(const AttnArgs& a, uint32_t unit, u
     }
     auto step = [&](int k, const WideValueWords<BITS>& cur, WideValueWords<BITS>& next) {
       if constexpr (kRaise) __builtin_amdgcn_s_setprio(1);
-      // weights (times 2^ev) of head n, tokens 16g .. 16g+15, read from the slot before the
+      // weights (times 2^ev where vfac is 1) of head n, tokens 16g .. 16g+15, read from the slot before the
       // chunk's (scale, zero) pairs are staged over it
       float4 lg[4];
       {
@@ -2574,6 +2579,8 @@ __device__ __forceinline__ void wide16_split(const AttnArgs& a, uint32_t unit, u
       if constexpr (SESS) {
         centre_pairs(vp0, code_mid(BITS));
         centre_pairs(vp1, code_mid(BITS));
+        vp0.x *= vfac, vp0.z *= vfac;
+        vp1.x *= vfac, vp1.z *= vfac;
       }
       wide_stage(wl, ROW, k, lane, vp0, vp1);
       const int32_t kn = chunk_of(std::min(k + 1, nch - 1));

@@ -96,6 +96,29 @@ def test_long_windows_run_once_for_all_rows(amd, case):
         kivi.timing_enable(amd, False)
 
 
+@pytest.mark.parametrize("size", [1e-10, 1.0, 1e10])
+@pytest.mark.parametrize("bits,gq,count,residual", [(2, 8, 3, 64), (4, 4, 6, 64), (8, 1, 20, 128)])
+def test_value_magnitudes_keep_the_weights(amd, bits, gq, count, residual, size):
+    """Values far from 1 cost no precision. Bar 5e-7 in relative 2-norm: a weight whose exponential
+    takes in the values' power of two (2^33 and more) is rounded at 32 or above, 2^-19 / sqrt(3) * ln 2 =
+    7.6e-7 rms; logits below 8 alone give 1e-7."""
+    heads, dim, n = 4, 128, 1571
+    rng = np.random.default_rng(5300 + bits)
+    cache = KiviCache(amd, KiviConfig(bits, 32, residual), 1, heads, dim)
+    k, v = (rng.standard_normal((heads, n, dim)).astype(np.float32) for _ in range(2))
+    cache.append(k, v * np.float32(size), n)
+    kd, vd = (x.reshape(heads, n, dim).astype(np.float64) for x in cache.dequantize())
+    prefix = cache.share_prefix()
+    sessions = [prefix.session() for _ in range(count)]
+    q = rng.standard_normal((count, heads, gq, dim)).astype(np.float32)
+    scale = np.float32(1 / np.sqrt(dim))
+    got = kivi.sessions_attention(amd, sessions, q, heads * gq, scale).reshape(q.shape)
+    logits = q.astype(np.float64) @ kd.swapaxes(-1, -2) * float(scale)
+    w = np.exp(logits - logits.max(-1, keepdims=True))
+    want = (w / w.sum(-1, keepdims=True)) @ vd
+    assert np.linalg.norm(got - want) < 5e-7 * np.linalg.norm(want)
+
+
 def run(amd, bits, group, residual, dim, batch, heads, gq, n, count, spread):
     qh = heads * gq
     rng = np.random.default_rng(5100 + n + count)
