@@ -35,6 +35,8 @@
 //  * k_attn_generic — any other head_dim: one wavefront per token in the reference's operation
 //    order (recon = fma(code, scale, zero); logit = fma(recon, q, logit), channels ascending,
 //    src/attention.rs:143-177, 289-300).
+#include <type_traits>
+
 #include "common.hpp"
 #include "kivi.h"
 
@@ -1292,6 +1294,28 @@ __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_wave_barrier();
 }
 
+// Sum of n values `step` floats apart, in one chain or in four (n >= 4). One chain over the sixteenths of a
+// wide head (64 at head_dim 1024) was 6.6e-7 off f64 attention (rms of 33 caches) where a wavefront per token
+// with its butterfly is 4.1e-7 off; four are 3.6e-7, in the same time (117 shapes, median 1.000). From
+// kWideSum values on: below, one chain is as precise, and the four cost 10% at head_dim 16.
+constexpr uint32_t kWideSum = 16;
+template <bool WIDE>
+__device__ __forceinline__ float strided_sum(const float* p, uint32_t n, uint32_t step) {
+  if constexpr (!WIDE) {
+    float v = p[0];
+    for (uint32_t k = 1; k < n; ++k) v += p[k * step];
+    return v;
+  } else {
+    float s[4] = {p[0], p[step], p[2 * step], p[3 * step]};
+    uint32_t k = 4;
+    for (; k + 4 <= n; k += 4)
+#pragma unroll
+      for (uint32_t j = 0; j < 4; ++j) s[j] += p[(k + j) * step];
+    for (; k < n; ++k) s[0] += p[k * step];
+    return (s[0] + s[1]) + (s[2] + s[3]);
+  }
+}
+
 // ------------------------------------------------------------------ row splits
 // Tokens [t_begin, total) of any head_dim that is a multiple of 16, wherever each of them lives
 // (packed, key residual, value window, suffix): the tokens after the packed chunks at head_dims
@@ -1432,15 +1456,18 @@ __device__ __forceinline__ void row_split(const AttnArgs& a, uint32_t unit, uint
       xch[threadIdx.x * kRowHeads + h] = v[0] + v[1];
     }
     wave_lds_fence();
-    for (uint32_t o = lane; o < TP * kRowHeads; o += 64) {
-      const uint32_t r = o / kRowHeads, h = o % kRowHeads;
-      const float* src = xch + (wave * 64 + r * NB) * kRowHeads + h;
-      if (h < nh && k0 + r < ntok) {
-        float v = src[0];
-        for (uint32_t k = 1; k < NB; ++k) v += src[k * kRowHeads];
-        w_lds[h * S + k0 + r] = v * a.scale2;
+    auto gather = [&](auto wide) {
+      for (uint32_t o = lane; o < TP * kRowHeads; o += 64) {
+        const uint32_t r = o / kRowHeads, h = o % kRowHeads;
+        const float* src = xch + (wave * 64 + r * NB) * kRowHeads + h;
+        if (h < nh && k0 + r < ntok)
+          w_lds[h * S + k0 + r] = strided_sum<decltype(wide)::value>(src, NB, kRowHeads) * a.scale2;
       }
-    }
+    };
+    if (NB >= kWideSum)
+      gather(std::true_type{});
+    else
+      gather(std::false_type{});
     wave_lds_fence();
     k0 += 4 * TP;
     if (k0 < ntok) {
@@ -1505,9 +1532,7 @@ __device__ __forceinline__ void row_split(const AttnArgs& a, uint32_t unit, uint
   __syncthreads();
   for (uint32_t i = threadIdx.x; i < nh * D; i += kThreads) {
     const uint32_t h = i / D, d = i % D;
-    float v = xch[h * D + d];
-    for (uint32_t k = 1; k < rows; ++k) v += xch[(k * kRowHeads + h) * D + d];
-    part[h * (D + 2) + d] = v;
+    part[h * (D + 2) + d] = strided_sum<false>(xch + h * D + d, rows, kRowHeads * D);
   }
 }
 
@@ -1650,14 +1675,17 @@ __device__ __forceinline__ void lane_split(const AttnArgs& a, uint32_t unit, uin
               make_float4(acc[4 * k / HP][4 * k % HP], acc[(4 * k + 1) / HP][(4 * k + 1) % HP],
                           acc[(4 * k + 2) / HP][(4 * k + 2) % HP], acc[(4 * k + 3) / HP][(4 * k + 3) % HP]);
         wave_lds_fence();
-        for (uint32_t o = lane; o < TP * 4 * HP; o += 64) {
-          const uint32_t r = o / (4 * HP), ih = o % (4 * HP), run = s0 + r;
-          const float* src = xch + r * NB * REC + ih;
-          float v = src[0];
-          for (uint32_t k = 1; k < NB; ++k) v += src[k * REC];
-          v *= a.scale2;
-          if (run < nsub) w_lds[(ih % HP) * ROW + run * 16 + 4 * t4 + ih / HP] = v;
-        }
+        auto gather = [&](auto wide) {
+          for (uint32_t o = lane; o < TP * 4 * HP; o += 64) {
+            const uint32_t r = o / (4 * HP), ih = o % (4 * HP), run = s0 + r;
+            const float v = strided_sum<decltype(wide)::value>(xch + r * NB * REC + ih, NB, REC) * a.scale2;
+            if (run < nsub) w_lds[(ih % HP) * ROW + run * 16 + 4 * t4 + ih / HP] = v;
+          }
+        };
+        if (NB >= kWideSum)
+          gather(std::true_type{});
+        else
+          gather(std::false_type{});
         wave_lds_fence();
       }
     }

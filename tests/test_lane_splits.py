@@ -7,8 +7,8 @@ so the cases sit at the edges of that form: one chunk, splits of 4, 5, 8, 9, 16 
 lanes per token (head_dim / 16) that do and do not divide a wave, every code width, odd numbers of
 heads, a group of 48 tokens. Against the oracle within the parity tolerance, and against f64
 attention over the dequantized cache: the kernel reconstructs every element as the reference does
-and sums products in f32, at most 16 in a row before a tree, so its outputs lie within
-(16 + 12) 2^-24 of the products' magnitude sum, 1.7e-6 of a logit's; 2e-5 absolute bounds that at
+and sums products in f32, eight in a row, two such sums, then at most 18 partial sums in a row (15, or
+16 in each of four chains from head_dim 256 on), so its outputs lie within (16 + 12) 2^-24 of the products' magnitude sum, 1.7e-6 of a logit's; 2e-5 absolute bounds that at
 these inputs (logits below 2^4 in magnitude sum, values below 2^3)."""
 
 import numpy as np
@@ -98,3 +98,24 @@ def test_lane_splits_against_oracle_and_dense(amd, oracle, case):
             assert np.array_equal(mem.download(out, q.size), got.reshape(-1))
     finally:
         mem.free()
+
+
+@pytest.mark.parametrize("bits,group,residual", [(4, 16, 32), (8, 16, 256), (4, 8, 16)])
+def test_wide_heads_sum_in_short_chains(amd, bits, group, residual):
+    """head_dim 1024, lane splits and row splits: the 64 partial sums of a logit in four chains of 16, not
+    one of 64, which rounds twice as much in the rms. Relative 2-norm off f64 attention, rms of eight
+    caches: one chain 3.1e-7 to 3.4e-7, four 2.0e-7 (the rest of it is the softmax's and the mix's)."""
+    units, gq, n, dim = 2, 4, 300, 1024
+    errors = []
+    for seed in range(8):
+        rng = np.random.default_rng(5400 + seed)
+        k, v = (rng.standard_normal((1, units, n, dim)).astype(np.float32) for _ in range(2))
+        k[..., 0] *= 10
+        c = KiviCache(amd, KiviConfig(bits, group, residual), 1, units, dim)
+        c.append(k, v, n)
+        q = rng.standard_normal((1, units, gq, dim)).astype(np.float32)
+        scale = np.float32(1 / np.sqrt(dim))
+        want = dense_attention(c, q, units, scale)
+        got = c.attention(q, units * gq, scale).reshape(q.shape)
+        errors.append(np.linalg.norm(got - want) / np.linalg.norm(want))
+    assert np.sqrt(np.mean(np.square(errors))) < 2.6e-7
