@@ -4169,8 +4169,12 @@ void set_session_strides(const SessionsProblem& sp, uint32_t nsess, AttnArgs& a)
   a.ws_sess_stride = (uint64_t)sp.cache.geo.units * a.nsplit_total * a.gq * (sp.cache.geo.D + 2);
 }
 
-AttnArgs make_session_args(const SessionsProblem& sp, uint32_t nsess, uint64_t max_suffix, float* ws) {
-  AttnArgs a = make_args_as(session_problem(sp, max_suffix), ws, SplitPlan::kUsual, 1);
+// One session's plan, the window range sized for `max_suffix`; the forms below take theirs from it.
+AttnArgs one_session_args(const SessionsProblem& sp, uint64_t max_suffix, float* ws) {
+  return make_args_as(session_problem(sp, max_suffix), ws, SplitPlan::kUsual, 1);
+}
+
+AttnArgs make_session_args(const SessionsProblem& sp, uint32_t nsess, AttnArgs a) {
   // packed splits: 16 rows each, at most kWide16Cpw chunks per wave, at least kFastGroups workgroups
   a.hgroups_fast = (nsess * a.gq + kWide16Heads - 1) / kWide16Heads;
   const uint32_t vu = a.units * a.hgroups_fast, most = (a.chunk_end + 3) / 4;
@@ -4254,9 +4258,9 @@ bool shared_pays(const AttnArgs& r, const AttnArgs& s) {
   return gemm < rows;
 }
 
-// The arguments of a launch group of `nsess` sessions in the form it takes.
-AttnArgs make_rows_args(const SessionsProblem& sp, uint32_t nsess, uint64_t max_suffix, float* ws, bool* shared) {
-  const AttnArgs r = make_session_args(sp, nsess, max_suffix, ws);
+// The arguments of a launch group of `nsess` sessions in the form it takes; `one`: one_session_args.
+AttnArgs make_rows_args(const SessionsProblem& sp, uint32_t nsess, uint64_t max_suffix, const AttnArgs& one, bool* shared) {
+  const AttnArgs r = make_session_args(sp, nsess, one);
   const uint64_t rows = (uint64_t)nsess * r.gq;
   *shared = false;
   if (rows < kSharedFewRows) return r;
@@ -4391,7 +4395,7 @@ AttnArgs group_args(const SessionsProblem& p, uint32_t first, uint32_t count, fl
     set_session_strides(gp, count, a);
     return a;
   }
-  return make_rows_args(gp, count, longest, ws, shared);
+  return make_rows_args(gp, count, longest, one_session_args(gp, longest, ws), shared);
 }
 
 // Partials a batched call of single-session launches may take (256 MB); larger ones run one by one,
@@ -4418,15 +4422,21 @@ size_t sessions_reserve_floats(const SessionsProblem& p) {
   size_t most = sessions_workspace_floats(p);
   if (session_form(p) != SessionForm::kRows) return most;
   const uint64_t longest = longest_suffix(p, 0, p.n);
-  for (uint32_t count = 1; count <= std::min(kMaxLaunchSessions, p.n); ++count) {
-    // either form: shorter suffixes may change it, towards the row groups (where the bare prefix takes
-    // the GEMM no suffix makes those the faster form: 128 tokens cost them two window chunks per session)
-    const AttnArgs r = make_session_args(p, count, longest, nullptr);
-    const uint64_t rows = (uint64_t)count * r.gq;
-    bool gemm;
-    (void)make_rows_args(p, count, 0, nullptr, &gemm);
-    if (!gemm) most = std::max(most, (size_t)count * r.ws_sess_stride);
-    if (rows >= kSharedFewRows) most = std::max(most, (size_t)count * make_shared_args(p, count, longest, r).ws_sess_stride);
+  const AttnArgs full = one_session_args(p, longest, nullptr), bare = one_session_args(p, 0, nullptr);
+  // the counts that make up one number of 16-row groups share a plan, and the largest needs the most
+  const uint32_t counts = std::min(kMaxLaunchSessions, p.n);
+  for (uint32_t first = 1, last; first <= counts; first = last + 1) {
+    last = std::min(counts, (first * full.gq + kWide16Heads - 1) / kWide16Heads * kWide16Heads / full.gq);
+    const AttnArgs r = make_session_args(p, last, full);
+    // either form: shorter suffixes and fewer sessions may change it, towards the row groups (where the
+    // bare prefix takes the GEMM no suffix makes those faster: 128 tokens cost them two window chunks per
+    // session)
+    bool gemm_first, gemm_last;  // times are linear in the count in between
+    (void)make_rows_args(p, first, 0, bare, &gemm_first);
+    (void)make_rows_args(p, last, 0, bare, &gemm_last);
+    if (!gemm_first || !gemm_last) most = std::max(most, (size_t)last * r.ws_sess_stride);
+    if ((uint64_t)last * r.gq >= kSharedFewRows)
+      most = std::max(most, (size_t)last * make_shared_args(p, last, longest, r).ws_sess_stride);
   }
   return most;
 }
